@@ -25,7 +25,7 @@ SOURCES = ['rows_dma.hip', 'rows_dma32.hip', 'rows_f64.hip', 'rows_c128.hip', 'r
            'precond_fine.hip']
 
 FLAGS = [
-    '-std=c++17', '-O3', '-fPIC', f'--offload-arch={ARCH}',
+    '-std=c++20', '-O3', '-fPIC', f'--offload-arch={ARCH}',
     # packed FP32 instructions stay off (silent wrong results seen on this
     # hardware class); the host pass warns that it does not know the feature
     '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',

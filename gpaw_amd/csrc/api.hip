@@ -861,14 +861,20 @@ struct CoarseSolve {
     bool valid = false;
     int lc = -1;      // first level in LDS (-1: none)
     size_t lds = 0;
+    bool one = false; // k_coarse1 (else k_coarse)
     CGrid host{};
     DevBuf dev;
 };
 
 // LDS-resident coarse solve on (default) / off, and the largest first
-// level (points) it takes
+// level (points) it takes (0: the defaults below)
 static bool g_coarse_lds = true;
-static long g_coarse_max_pts = 4096;
+static long g_coarse_max_pts = 0;
+// one workgroup against a launch per sweep: the general kernel up to 16^3
+// points, nearest-neighbour levels up to 24^3 where they fit (192^3 mixed
+// solve: 5.62 ms with the FP32 24^3 level in the workgroup, 5.74 from 12^3
+// down; FP64 40^3 box, 19^3 level: 2.83 against 3.55 ms)
+constexpr long COARSE_PTS = 4096, COARSE1_PTS = 14000;
 
 struct gfd_poisson {
     int L = 0;  // number of coarsenings
@@ -1070,99 +1076,113 @@ static double sched_w(const Schedule& sc, int l)
     return sc.w[l];
 }
 
+// The grid table of an LDS-resident solve of levels [lc, coarsest], and its
+// LDS bytes.  Two iterate arrays and the right-hand side per level (the
+// first level's rhs stays in global memory when it does not fit).  False:
+// not for these operators, or too large.
+static bool coarse_layout(gfd_poisson* p, const Schedule& sc, int dtype,
+                          int lc, bool cheb, CGrid& g,
+                          size_t& bytes)
+{
+    const long es = dtype == 2 ? 4 : 8;
+    const long most = COARSE_LDS_MAX / es;  // elements
+    g = CGrid{};
+    g.nlev = sc.coarsest - lc + 1;
+    if (g.nlev > CMAXLEV) return false;
+    long total = 0;
+    for (int l = lc; l <= sc.coarsest; l++) {
+        const gfd_operator* op = p->ops[l];
+        if (!op->axis_ok || !op->real || op->ax.R > CMAXR) return false;
+        if (l < sc.coarsest &&
+            (p->rst[l]->plan.K != 2 || p->itp[l]->plan.K != 2))
+            return false;
+        total += op->ng() * (l == lc ? 2 : 3);
+    }
+    const bool r_lds = total + p->ops[lc]->ng() <= most;
+    long off = 0;
+    for (int i = 0; i < g.nlev; i++) {
+        const int l = lc + i;
+        const gfd_operator* op = p->ops[l];
+        CLevel& L = g.lev[i];
+        for (int d = 0; d < 3; d++) {
+            L.n[d] = op->n[d];
+            L.periodic[d] = op->periodic[d];
+            L.has[d] = op->ax.has[d];
+            for (int k = 0; k < CMAXR; k++) {
+                L.cp[d][k] = k < op->ax.R ? op->ax.cp[d][k] : 0.0;
+                L.cm[d][k] = k < op->ax.R ? op->ax.cm[d][k] : 0.0;
+            }
+        }
+        L.R = op->ax.R;
+        L.c0 = centre_coef(op);
+        L.w = sched_w(sc, l);
+        L.pre = sched_pre(sc, l);
+        L.post = sched_post(sc, l);
+        const long n = op->ng();
+        L.a = (int)off;
+        off += n;
+        L.b = (int)off;
+        off += n;
+        L.r = -1;
+        if (i > 0 || r_lds) {
+            L.r = (int)off;
+            off += n;
+        }
+        if (off > most) return false;
+        if (l < sc.coarsest)
+            for (int d = 0; d < 3; d++) {
+                L.roff[d] = p->rst[l]->plan.ax[d].off;
+                L.ioff[d] = p->itp[l]->plan.ax[d].off;
+                L.iskip0[d] = p->itp[l]->plan.ax[d].skip0;
+            }
+    }
+    CLevel& C = g.lev[g.nlev - 1];
+    const long nc = (long)C.n[0] * C.n[1] * C.n[2];
+    double lo, hi;
+    C.cheb = 0;
+    C.dbuf = -1;
+    if (cheb && coarse_cheb_enabled() && off + nc <= most &&
+        cheb_bounds(C, &lo, &hi)) {
+        C.cheb = 1;
+        C.dbuf = (int)off;
+        C.lam_lo = lo;
+        C.lam_hi = hi;
+        off += nc;
+    }
+    g.lds_elems = (int)off;
+    bytes = (size_t)(es * g.lds_elems);
+    return true;
+}
+
 // Plan the LDS-resident solve of levels [lc, coarsest] for a schedule: the
-// first lc >= 1 whose level arrays fit one workgroup's LDS (rhs of level lc
-// stays in global memory).  *changed reports a new plan (graphs that
-// captured the old one must be dropped).  Not callable under capture.
+// first lc >= 1 that one workgroup holds and solves faster than launches of
+// its own would.  *changed reports a new plan (graphs that captured the old
+// one must be dropped).  Not callable under capture.
 // cheb: Chebyshev iteration on the coarsest level (mixed schedules; the
 // reference schedule smooths every level with Jacobi)
 static int plan_coarse(gfd_poisson* p, const Schedule& sc, int dtype,
                        CoarseSolve& c, hipStream_t s, bool* changed,
                        bool cheb = false)
 {
-    const size_t es = dtype == 2 ? 4 : 8;
     int lc = -1;
+    bool one = false;
     size_t bytes = 0;
+    CGrid g{};
     // the LDS-resident solve smooths with Jacobi: not for the FP64
     // Gauss-Seidel schedule
     const bool lds_ok = g_coarse_lds && !(dtype == 0 && p->method == 1);
-    for (int l0 = 1; lds_ok && l0 <= sc.coarsest; l0++) {
-        if (sc.coarsest - l0 + 1 > CMAXLEV) continue;
-        if (p->ops[l0]->ng() > g_coarse_max_pts) continue;
-        size_t b = 0;
-        bool ok = true;
-        for (int l = l0; l <= sc.coarsest && ok; l++) {
-            const gfd_operator* op = p->ops[l];
-            ok = op->axis_ok && op->real && op->ax.R <= CMAXR;
-            if (l < sc.coarsest)
-                ok = ok && p->rst[l]->plan.K == 2 && p->itp[l]->plan.K == 2;
-            b += es * op->ng() * (l == l0 ? 2 : 3);
-        }
-        if (ok && b <= COARSE_LDS_MAX) {
-            lc = l0;
-            bytes = b;
-            break;
-        }
+    for (int l0 = 1; lds_ok && lc < 0 && l0 <= sc.coarsest; l0++) {
+        if (!coarse_layout(p, sc, dtype, l0, cheb, g, bytes)) continue;
+        one = coarse_plan1(&g, 1, dtype);
+        const long most = g_coarse_max_pts ? g_coarse_max_pts
+                          : one            ? COARSE1_PTS
+                                           : COARSE_PTS;
+        if (p->ops[l0]->ng() <= most) lc = l0;
     }
-    // stage the first level's rhs in LDS too when it fits
-    const bool r_lds =
-        lc >= 0 && bytes + es * p->ops[lc]->ng() <= COARSE_LDS_MAX;
-    if (r_lds) bytes += es * p->ops[lc]->ng();
-    CGrid g{};
-    if (lc >= 0) {
-        g.nlev = sc.coarsest - lc + 1;
-        int off = 0;
-        for (int i = 0; i < g.nlev; i++) {
-            const int l = lc + i;
-            const gfd_operator* op = p->ops[l];
-            CLevel& L = g.lev[i];
-            for (int d = 0; d < 3; d++) {
-                L.n[d] = op->n[d];
-                L.periodic[d] = op->periodic[d];
-                L.has[d] = op->ax.has[d];
-                for (int k = 0; k < CMAXR; k++) {
-                    L.cp[d][k] = k < op->ax.R ? op->ax.cp[d][k] : 0.0;
-                    L.cm[d][k] = k < op->ax.R ? op->ax.cm[d][k] : 0.0;
-                }
-            }
-            L.R = op->ax.R;
-            L.c0 = centre_coef(op);
-            L.w = sched_w(sc, l);
-            L.pre = sched_pre(sc, l);
-            L.post = sched_post(sc, l);
-            const int n = (int)op->ng();
-            L.a = off;
-            off += n;
-            L.b = off;
-            off += n;
-            if (i == 0 && !r_lds) {
-                L.r = -1;
-            } else {
-                L.r = off;
-                off += n;
-            }
-            if (l < sc.coarsest)
-                for (int d = 0; d < 3; d++) {
-                    L.roff[d] = p->rst[l]->plan.ax[d].off;
-                    L.ioff[d] = p->itp[l]->plan.ax[d].off;
-                    L.iskip0[d] = p->itp[l]->plan.ax[d].skip0;
-                }
-        }
-        CLevel& C = g.lev[g.nlev - 1];
-        const int nc = C.n[0] * C.n[1] * C.n[2];
-        double lo, hi;
-        C.cheb = 0;
-        C.dbuf = -1;
-        if (cheb && coarse_cheb_enabled() &&
-            bytes + es * nc <= COARSE_LDS_MAX && cheb_bounds(C, &lo, &hi)) {
-            C.cheb = 1;
-            C.dbuf = off;
-            C.lam_lo = lo;
-            C.lam_hi = hi;
-            off += nc;
-            bytes += es * nc;
-        }
-        g.lds_elems = off;
+    if (lc < 0) {
+        g = CGrid{};
+        bytes = 0;
+        one = false;
     }
     const bool same = c.valid && c.lc == lc &&
                       (lc < 0 || std::memcmp(&c.host, &g, sizeof g) == 0);
@@ -1177,6 +1197,7 @@ static int plan_coarse(gfd_poisson* p, const Schedule& sc, int dtype,
     c.host = g;
     c.lc = lc;
     c.lds = bytes;
+    c.one = one;
     c.valid = true;
     return OK;
 }
@@ -1227,7 +1248,7 @@ static int vcycle(gfd_poisson* p, Levels& lv, const Schedule& sc, int l,
         if (cs.valid && cs.lc == l + 1) {
             // levels l+1 .. coarsest in one LDS-resident workgroup
             GFD_TRY(launch_coarse((const CGrid*)cs.dev.p, 1, cs.lds, dt,
-                                  lv.rho[l + 1], c1, s));
+                                  lv.rho[l + 1], c1, cs.one, s));
         } else {
             GFD_TRY(vcycle(p, lv, sc, l + 1, &c1, &a1, lv.rho[l + 1], s,
                            true));
@@ -1843,7 +1864,7 @@ extern "C" int gfd_set_tuning(const char* key, long value)
         return OK;
     }
     if (std::strcmp(key, "coarse_max_points") == 0) {
-        g_coarse_max_pts = value > 0 ? value : 4096;
+        g_coarse_max_pts = value > 0 ? value : 0;
         return OK;
     }
     if (std::strcmp(key, "xfer_passes") == 0) {

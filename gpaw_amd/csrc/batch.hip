@@ -444,6 +444,7 @@ struct gfd_batch_poisson {
     std::vector<double> cw;
     std::vector<CGrid> cgrids;
     size_t clds = 0;
+    bool cone = false;  // coarse levels by k_coarse1
     int ckey[4] = {-1, -1, -1, -1};
     DevBuf d_cgrids;
 };
@@ -1229,7 +1230,7 @@ static int b_vcycle(gfd_batch_poisson* b, int l, void** cur, void** alt,
     }
     if (b->coarse)  // starts from e = 0 in LDS
         return launch_coarse((const CGrid*)b->d_cgrids.p, b->G, b->clds, 2,
-                             rhs, *cur, s);
+                             rhs, *cur, b->cone, s);
     return b_relax0(b, l, cur, alt, rhs, coarse, s);
 }
 
@@ -1322,6 +1323,7 @@ static int b_plan_coarse(gfd_batch_poisson* b, int pre, int post, int coarse,
                   maxb);
         return ENOTSUP_;
     }
+    b->cone = coarse_plan1(b->cgrids.data(), b->G, 2);
     GFD_TRY(b->d_cgrids.ensure(sizeof(CGrid) * b->G, s));
     GFD_CHECK_HIP(hipMemcpyAsync(b->d_cgrids.p, b->cgrids.data(),
                                  sizeof(CGrid) * b->G, hipMemcpyHostToDevice,

@@ -27,13 +27,20 @@ struct CLevel {
     int a, b, r;             // LDS element offsets: e ping-pong and rhs
                              // (first level: staged from global memory,
                              // or r < 0: read there in every pass)
+    // nearest-neighbour form (k_coarse1): x segments per column, longest
+    // segment, one wave holds the whole level
+    int parts, xl, onewave;
     // transfer to the next coarser level
     int roff[3];             // restriction: first centre per axis
     int ioff[3], iskip0[3];  // interpolation back to this level
 };
 
+// Chebyshev steps whose coefficients are tabulated with the grid
+constexpr int CCHEB = 32;
+
 struct CGrid {
     int nlev;                // levels handled (lc .. lc + nlev - 1)
+    double cheb_a[CCHEB], cheb_b[CCHEB];
     int lds_elems;           // LDS elements used
     long rhs_off, out_off;   // element offsets of the grid's rhs / result
     CLevel lev[CMAXLEV];
@@ -54,9 +61,14 @@ bool cheb_bounds(const CLevel& L, double* lo, double* hi);
 void coarse_set_cheb(bool on);
 bool coarse_cheb_enabled();
 
+// Whether k_coarse1 takes these grids; fills parts / xl / onewave of every
+// level and the Chebyshev tables.
+bool coarse_plan1(CGrid* grids, int G, int dtype);
+
+// one: k_coarse1 (coarse_plan1 took the grids), else k_coarse.
 // dtype 0: f64, 2: f32.  rhs: level-lc right-hand sides, out: level-lc
 // corrections (zero initial guess), grid g at rhs_off / out_off.
 int launch_coarse(const CGrid* d_grids, int G, size_t lds_bytes, int dtype,
-                  const void* rhs, void* out, hipStream_t s);
+                  const void* rhs, void* out, bool one, hipStream_t s);
 
 }  // namespace gfd
