@@ -41,7 +41,8 @@ void set_error(const char* fmt, ...)
 
 const char* last_error() { return g_err.c_str(); }
 
-// 0 auto, 1 general kernel, 2 tiled x-march kernel, 3 full-row kernel
+// 0 auto, 1 general kernel, 2 tiled x-march kernel, 3 full-row kernel,
+// 4 direction march
 int g_force_path = 0;
 
 static BC make_bc(const int periodic[3], const double* phases)
@@ -189,6 +190,8 @@ extern "C" int gfd_operator_new(int ncoefs, const double* coefs,
         if (op->n[c] < R) ok = false;
     ax.R = R;
     op->axis_ok = ok;
+    op->dir_ok =
+        dir_stencil(ncoefs, op->coef.data(), op->off.data(), op->dir);
     // device copies for the general kernel
     if (hipMalloc((void**)&op->d_coef, sizeof(double) * ncoefs) != hipSuccess ||
         hipMalloc((void**)&op->d_off, sizeof(int) * 3 * ncoefs) != hipSuccess) {
@@ -233,16 +236,22 @@ static bool aligned16(const void* p)
     return ((uintptr_t)p & 15) == 0;
 }
 
-// Kernel family for one pass: 3 full-row, 2 tiled x-march, 1 general.
+// Kernel family for one pass: 3 full-row, 4 direction march, 2 tiled
+// x-march, 1 general.
 static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
                    const void* out, const void* aux, int epi)
 {
-    if (!op->use_fast()) return 1;
+    const bool dir = op->dir_ok &&
+                     (g_force_path == 0 || g_force_path == 4) &&
+                     dirmarch_fits(op->dir, dtype, op->n, nin, epi);
+    if (dir && g_force_path == 4) return 4;
+    if (!op->use_fast()) return dir ? 4 : 1;
     const bool row = (g_force_path == 0 || g_force_path == 3) &&
                      aligned16(in) && aligned16(out) &&
                      (aux == nullptr || aligned16(aux)) &&
                      row_stencil_fits(op->ax, dtype, op->n, nin);
     if (row) return 3;
+    if (dir) return 4;
     // epilogues the tiled x-march kernel instantiates per data type
     const bool xm_has =
         (dtype == 0 && epi <= EPI_UPDATE) ||
@@ -265,6 +274,9 @@ static int op_pass(gfd_operator* op, int dtype, const void* in, void* out,
     if (path == 3)
         return launch_row_stencil(op->ax, dtype, op->n, bc, in, out, nin, epi,
                                   ea, s, nblocks);
+    if (path == 4)
+        return launch_dirmarch(op->dir, dtype, op->n, bc, in, out, nin, epi,
+                               ea, s, nblocks);
     if (path == 2)
         return launch_axis_stencil(op->ax, dtype, op->n, bc, in, out, nin, epi,
                                    ea, s, nblocks);
@@ -276,6 +288,8 @@ static int op_pass(gfd_operator* op, int dtype, const void* in, void* out,
 static long op_max_blocks(gfd_operator* op, int dtype, long nin)
 {
     long m = general_stencil_max_blocks(op->n, nin);
+    if (op->dir_ok)
+        m = std::max(m, dirmarch_max_blocks(op->dir, dtype, op->n, nin));
     if (op->use_fast()) {
         m = std::max(m, axis_stencil_max_blocks(op->ax, dtype, op->n, nin));
         m = std::max(m, row_stencil_max_blocks(op->ax, dtype, op->n, nin));
@@ -1835,8 +1849,8 @@ extern "C" int gfd_set_tuning(const char* key, long value)
         return OK;
     }
     if (std::strcmp(key, "force_path") == 0) {
-        if (value < 0 || value > 3) {
-            set_error("gfd_set_tuning: force_path must be 0..3");
+        if (value < 0 || value > 4) {
+            set_error("gfd_set_tuning: force_path must be 0..4");
             return EINVAL_;
         }
         g_force_path = (int)value;

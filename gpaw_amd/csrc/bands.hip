@@ -3,8 +3,8 @@
 //  * k_gram: G = A B^H for row-major complex A (M x K) and B (N x K) with a
 //    long inner dimension (K = grid points): 128 x 128 output tiles, split
 //    over K into chunks, 512 threads (8 waves, 2 x 4 MFMA tiles of 16 x 16
-//    per wave); A and B stream through LDS in 16-point stages as separate
-//    re / im planes, and every complex 16 x 16 x 4 step is four
+//    per wave); A and B stream through LDS in 16-point stages (two in turn)
+//    as separate re / im planes, and every complex 16 x 16 x 4 step is four
 //    v_mfma_f64_16x16x4f64 (re.re + im.im, im.re - re.im).  Chunk partials
 //    are reduced in a fixed order (bit-reproducible).
 //  * the Cholesky factor and its inverse come from rocSOLVER (zpotrf,
@@ -18,6 +18,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace gfd {
 
@@ -49,7 +50,6 @@ struct GramArgs {
     int nchunks;
     int ntiles;
     int tcols;           // tile columns (full matrix)
-    int lower;           // tiles (i, j <= i) in row order
     double2* partial;    // [chunk][tile][GT][GT]
 };
 
@@ -63,18 +63,43 @@ __device__ inline int2 tile_of(int t, int lower, int tcols)
     return make_int2(i, t - i * (i + 1) / 2);
 }
 
+typedef double GramStage[GK][GP];
+
+// LOWER: only the lower tiles of a Hermitian product; on a diagonal tile the
+// 16 x 16 sub-tiles above the diagonal are left out, and the waves take
+// other parts of the tile so that the two waves of every SIMD keep 8 to 10
+// of 16 sub-tiles (waves w and w + 4 share a SIMD).
+//
+// What bounds it: the FP64 matrix unit (64 cycles per MFMA, two waves per
+// SIMD at 228 VGPRs, one block per CU), so everything else has to hide
+// behind it: two LDS stages, one barrier per stage, the next stage written
+// to LDS in the middle of the current one's MFMAs, loads two stages ahead.
+// 500 bands of 96^3: all tiles 28.9 -> 27.7 ms (67 TFLOP/s executed), lower
+// tiles 18.6 -> 16.4 ms (the diagonal tiles' upper sub-tiles and a nearly
+// empty tenth round of blocks left out), the rotation 16.9 -> 16.5 ms.
+template <bool LOWER>
 __global__ void __launch_bounds__(512) k_gram(GramArgs a)
 {
-    __shared__ double sAr[GK][GP], sAi[GK][GP], sBr[GK][GP], sBi[GK][GP];
+    __shared__ GramStage sAr[2], sAi[2], sBr[2], sBi[2];
     const int tile = blockIdx.x % a.ntiles;
     const int chunk = blockIdx.x / a.ntiles;
-    const int2 tt = tile_of(tile, a.lower, a.tcols);
+    const int2 tt = tile_of(tile, LOWER, a.tcols);
     const int i0 = tt.x * GT, j0 = tt.y * GT;
     const long kb = (long)chunk * a.kchunk;
     const long ke = min(kb + a.kchunk, a.K);
     const int t = threadIdx.x;
-    const int lane = t & 63, w = t >> 6;
-    const int wr = w >> 1, wc = w & 1;  // 4 x 2 waves: 32 rows x 64 cols
+    const int lane = t & 63;
+    // wave-uniform (scalar) wave number
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const bool diag = LOWER && tt.x == tt.y;
+    int wr = w >> 1, wc = w & 1;  // 4 x 2 waves: 32 rows x 64 cols
+    if (diag) {
+        // kept sub-tiles: (2,0) 8, (3,0) 8, (1,0) 7, (3,1) 7 with
+        // (0,1) 0, (1,1) 0, (0,0) 3, (2,1) 3
+        wr = (0x20103132 >> (4 * w)) & 15;
+        wc = (0x10111000 >> (4 * w)) & 15;
+        // waves 0..3: (2,0) (3,0) (1,0) (3,1); 4..7: (0,1) (1,1) (0,0) (2,1)
+    }
     const int li = lane & 15, lk = lane >> 4;
 
     d4 accr[2][4], acci[2][4];
@@ -88,65 +113,84 @@ __global__ void __launch_bounds__(512) k_gram(GramArgs a)
 
     // stage loader: 128 rows x 16 points of A and of B, 4 rows per thread
     // (16 lanes read 16 consecutive points of a row: 256-byte segments,
-    // conflict-free LDS writes); the next stage's values are fetched into
-    // registers while the current stage is multiplied out of LDS
+    // conflict-free LDS writes).  Rows past the matrix repeat its last row
+    // (their products are never stored), points past the chunk are read at
+    // its last point and staged as zeros.
     const int lk16 = t & 15, lr = t >> 4;
+    const double2 *pa[4], *pb[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        pa[q] = a.A + (long)min(i0 + lr + 32 * q, a.M - 1) * a.lda;
+        pb[q] = a.B + (long)min(j0 + lr + 32 * q, a.N - 1) * a.ldb;
+    }
     double2 va[4], vb[4];
     auto fetch = [&](long ks) {
-        const long k = ks + lk16;
+        const long k = min(ks + lk16, ke - 1);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int row = lr + 32 * q;
-            va[q] = make_double2(0.0, 0.0);
-            vb[q] = make_double2(0.0, 0.0);
-            if (k < ke) {
-                if (i0 + row < a.M) va[q] = a.A[(long)(i0 + row) * a.lda + k];
-                if (j0 + row < a.N) vb[q] = a.B[(long)(j0 + row) * a.ldb + k];
-            }
+            va[q] = pa[q][k];
+            vb[q] = pb[q][k];
         }
     };
-    fetch(kb);
-    for (long ks = kb; ks < ke; ks += GK) {
+    auto stage = [&](long ks, int buf) {
+        const bool in = ks + lk16 < ke;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            sAr[lk16][lr + 32 * q] = va[q].x;
-            sAi[lk16][lr + 32 * q] = va[q].y;
-            sBr[lk16][lr + 32 * q] = vb[q].x;
-            sBi[lk16][lr + 32 * q] = vb[q].y;
+            sAr[buf][lk16][lr + 32 * q] = in ? va[q].x : 0.0;
+            sAi[buf][lk16][lr + 32 * q] = in ? va[q].y : 0.0;
+            sBr[buf][lk16][lr + 32 * q] = in ? vb[q].x : 0.0;
+            sBi[buf][lk16][lr + 32 * q] = in ? vb[q].y : 0.0;
         }
-        __syncthreads();
-        if (ks + GK < ke) fetch(ks + GK);
+    };
+    auto multiply = [&](auto on_diag, int buf, int kk) {
+        const int kl = kk * 4 + lk;
+        double ar[2], ai[2], br[4], bi[4], nbi[4];
 #pragma unroll
-        for (int kk = 0; kk < GK / 4; kk++) {
-            const int kl = kk * 4 + lk;
-            double ar[2], ai[2], br[4], bi[4], nbi[4];
+        for (int r = 0; r < 2; r++) {
+            ar[r] = sAr[buf][kl][wr * 32 + r * 16 + li];
+            ai[r] = sAi[buf][kl][wr * 32 + r * 16 + li];
+        }
 #pragma unroll
-            for (int r = 0; r < 2; r++) {
-                ar[r] = sAr[kl][wr * 32 + r * 16 + li];
-                ai[r] = sAi[kl][wr * 32 + r * 16 + li];
-            }
+        for (int c = 0; c < 4; c++) {
+            br[c] = sBr[buf][kl][wc * 64 + c * 16 + li];
+            bi[c] = sBi[buf][kl][wc * 64 + c * 16 + li];
+            nbi[c] = -bi[c];
+        }
+#pragma unroll
+        for (int r = 0; r < 2; r++)
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                br[c] = sBr[kl][wc * 64 + c * 16 + li];
-                bi[c] = sBi[kl][wc * 64 + c * 16 + li];
-                nbi[c] = -bi[c];
+                if (on_diag && wc * 4 + c > wr * 2 + r) continue;
+                accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    ar[r], br[c], accr[r][c], 0, 0, 0);
+                acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    ai[r], br[c], acci[r][c], 0, 0, 0);
+                accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    ai[r], bi[c], accr[r][c], 0, 0, 0);
+                acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    ar[r], nbi[c], acci[r][c], 0, 0, 0);
             }
-#pragma unroll
-            for (int r = 0; r < 2; r++)
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        ar[r], br[c], accr[r][c], 0, 0, 0);
-                    accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        ai[r], bi[c], accr[r][c], 0, 0, 0);
-                    acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        ai[r], br[c], acci[r][c], 0, 0, 0);
-                    acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        ar[r], nbi[c], acci[r][c], 0, 0, 0);
-                }
+    };
+    fetch(kb);
+    stage(kb, 0);
+    fetch(kb + GK);   // clamped to the chunk where it ends
+    __syncthreads();
+    auto loop = [&](auto on_diag) {
+        int buf = 0;
+        for (long ks = kb; ks < ke; ks += GK, buf ^= 1) {
+            multiply(on_diag, buf, 0);
+            multiply(on_diag, buf, 1);
+            if (ks + GK < ke) {
+                stage(ks + GK, buf ^ 1);
+                fetch(ks + 2 * GK);
+            }
+            multiply(on_diag, buf, 2);
+            multiply(on_diag, buf, 3);
+            __syncthreads();
         }
-        __syncthreads();
-    }
+    };
+    if (LOWER && diag) loop(std::true_type{});
+    else loop(std::false_type{});
     // D register q of lane l holds row l / 16 + 4 q, column l % 16
     double2* out = a.partial + ((long)chunk * a.ntiles + tile) * GT * GT;
 #pragma unroll
@@ -179,21 +223,23 @@ struct RotArgs {
     int lower; // C lower triangular (Cholesky), else dense (eigenvectors)
 };
 
-typedef double RotStage[GK][GP];
-
 // One 128-band x 128-point output tile (band tile bt, point tile xt) of the
 // rotation.  LOWER: K runs to the tile's last row, and an MFMA whose 16
 // rows x 4 k of C lie wholly above the diagonal (all zero) is skipped.
+// Two LDS stages with one barrier each, as k_gram.
+struct RotLds {
+    GramStage Cr[2], Ci[2], Pr[2], Pi[2];
+};
+
 template <bool LOWER>
-__device__ inline void rot_tile(const RotArgs& a, int bt, long xt,
-                                RotStage& sCr, RotStage& sCi, RotStage& sPr,
-                                RotStage& sPi)
+__device__ inline void rot_tile(const RotArgs& a, int bt, long xt, RotLds& s)
 {
     const int i0 = bt * GT;
     const long x0 = xt * GT;
     const int kend = LOWER ? min(a.n, i0 + GT) : a.n;
     const int t = threadIdx.x;
-    const int lane = t & 63, w = t >> 6;
+    const int lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = w >> 1, wc = w & 1;
     const int li = lane & 15, lk = lane >> 4;
 
@@ -208,68 +254,81 @@ __device__ inline void rot_tile(const RotArgs& a, int bt, long xt,
     // C tile: 128 rows x 16 columns, one column of 4 rows per thread; psi
     // tile: 16 rows x 128 points, one point of 4 rows per thread
     // (consecutive lanes on consecutive columns / points: conflict-free LDS
-    // writes)
+    // writes).  Rows of C and points past the end repeat the last one (never
+    // stored); columns of C past kend or above the diagonal are staged as
+    // zeros, with the psi row there read at the last valid one.
     const int ck = t & 15, cr = t >> 4;
     const int pp = t & 127, pr = t >> 7;
+    const double2* pc[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        pc[q] = a.C + (long)min(i0 + cr + 32 * q, a.n - 1) * a.n;
+    const double2* px = a.psi + min(x0 + pp, a.X - 1);
     double2 vc[4], vp[4];
     auto fetch = [&](int ks) {
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int gi = i0 + cr + 32 * q;
+            vc[q] = pc[q][min(ks + ck, kend - 1)];
+            vp[q] = px[(long)min(ks + pr + 4 * q, kend - 1) * a.ldpsi];
+        }
+    };
+    auto stage = [&](int ks, int buf) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
             const int j = ks + ck;
-            vc[q] = (gi < a.n && j < kend && (!LOWER || j <= gi))
-                        ? a.C[(long)gi * a.n + j]
-                        : make_double2(0.0, 0.0);
-            const int jp = ks + pr + 4 * q;
-            const long x = x0 + pp;
-            vp[q] = (jp < kend && x < a.X) ? a.psi[(long)jp * a.ldpsi + x]
-                                           : make_double2(0.0, 0.0);
+            const bool in = j < kend && (!LOWER || j <= i0 + cr + 32 * q);
+            const bool inp = ks + pr + 4 * q < kend;
+            s.Cr[buf][ck][cr + 32 * q] = in ? vc[q].x : 0.0;
+            s.Ci[buf][ck][cr + 32 * q] = in ? vc[q].y : 0.0;
+            s.Pr[buf][pr + 4 * q][pp] = inp ? vp[q].x : 0.0;
+            s.Pi[buf][pr + 4 * q][pp] = inp ? vp[q].y : 0.0;
+        }
+    };
+    auto multiply = [&](int ks, int buf, int kk) {
+        const int kl = kk * 4 + lk;
+        double ar[2], ai[2], nai[2], br[4], bi[4];
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            ar[r] = s.Cr[buf][kl][wr * 32 + r * 16 + li];
+            ai[r] = s.Ci[buf][kl][wr * 32 + r * 16 + li];
+            nai[r] = -ai[r];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            br[c] = s.Pr[buf][kl][wc * 64 + c * 16 + li];
+            bi[c] = s.Pi[buf][kl][wc * 64 + c * 16 + li];
+        }
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            // rows i0 + wr 32 + r 16 .. +15 against k = ks + 4 kk .. +3
+            if (LOWER && ks + 4 * kk > i0 + wr * 32 + r * 16 + 15) continue;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    ar[r], br[c], accr[r][c], 0, 0, 0);
+                acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    ar[r], bi[c], acci[r][c], 0, 0, 0);
+                accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    nai[r], bi[c], accr[r][c], 0, 0, 0);
+                acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    ai[r], br[c], acci[r][c], 0, 0, 0);
+            }
         }
     };
     fetch(0);
-    for (int ks = 0; ks < kend; ks += GK) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            sCr[ck][cr + 32 * q] = vc[q].x;
-            sCi[ck][cr + 32 * q] = vc[q].y;
-            sPr[pr + 4 * q][pp] = vp[q].x;
-            sPi[pr + 4 * q][pp] = vp[q].y;
+    stage(0, 0);
+    fetch(GK);
+    __syncthreads();
+    int buf = 0;
+    for (int ks = 0; ks < kend; ks += GK, buf ^= 1) {
+        multiply(ks, buf, 0);
+        multiply(ks, buf, 1);
+        if (ks + GK < kend) {
+            stage(ks + GK, buf ^ 1);
+            fetch(ks + 2 * GK);
         }
-        __syncthreads();
-        if (ks + GK < kend) fetch(ks + GK);
-#pragma unroll
-        for (int kk = 0; kk < GK / 4; kk++) {
-            const int kl = kk * 4 + lk;
-            double ar[2], ai[2], nai[2], br[4], bi[4];
-#pragma unroll
-            for (int r = 0; r < 2; r++) {
-                ar[r] = sCr[kl][wr * 32 + r * 16 + li];
-                ai[r] = sCi[kl][wr * 32 + r * 16 + li];
-                nai[r] = -ai[r];
-            }
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                br[c] = sPr[kl][wc * 64 + c * 16 + li];
-                bi[c] = sPi[kl][wc * 64 + c * 16 + li];
-            }
-#pragma unroll
-            for (int r = 0; r < 2; r++) {
-                // rows i0 + wr 32 + r 16 .. +15 against k = ks + 4 kk .. +3
-                if (LOWER && ks + 4 * kk > i0 + wr * 32 + r * 16 + 15)
-                    continue;
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        ar[r], br[c], accr[r][c], 0, 0, 0);
-                    accr[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        nai[r], bi[c], accr[r][c], 0, 0, 0);
-                    acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        ar[r], bi[c], acci[r][c], 0, 0, 0);
-                    acci[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        ai[r], br[c], acci[r][c], 0, 0, 0);
-                }
-            }
-        }
+        multiply(ks, buf, 2);
+        multiply(ks, buf, 3);
         __syncthreads();
     }
 #pragma unroll
@@ -293,19 +352,18 @@ __device__ inline void rot_tile(const RotArgs& a, int bt, long xt,
 template <bool LOWER>
 __global__ void __launch_bounds__(512) k_rot(RotArgs a)
 {
-    __shared__ double sCr[GK][GP], sCi[GK][GP], sPr[GK][GP], sPi[GK][GP];
+    __shared__ RotLds lds;
     const int L = xcd_remap_rot(blockIdx.x, gridDim.x);
     if (!LOWER) {
-        rot_tile<false>(a, L % a.nti, L / a.nti, sCr, sCi, sPr, sPi);
+        rot_tile<false>(a, L % a.nti, L / a.nti, lds);
         return;
     }
     const int npair = (a.nti + 1) / 2;
     const int p = L % npair;
     const long xt = L / npair;
-    rot_tile<true>(a, p, xt, sCr, sCi, sPr, sPi);
+    rot_tile<true>(a, p, xt, lds);
     if (a.nti - 1 - p != p) {
-        __syncthreads();  // the stage arrays are reused
-        rot_tile<true>(a, a.nti - 1 - p, xt, sCr, sCi, sPr, sPi);
+        rot_tile<true>(a, a.nti - 1 - p, xt, lds);
     }
 }
 
@@ -321,15 +379,21 @@ k_gram_reduce(const double2* __restrict__ partial, int nchunks, int ntiles,
     const int tile = (int)(e / per);
     const int rc = (int)(e % per);
     const int2 tt = tile_of(tile, lower, tcols);
-    const int row = tt.x * GT + rc / GT;
-    const int col = tt.y * GT + rc % GT;
+    const int tr = rc / GT, tc = rc % GT;
+    const int row = tt.x * GT + tr;
+    const int col = tt.y * GT + tc;
     if (row >= M || col >= N) return;
+    // sub-tiles above the diagonal of a Hermitian product's diagonal tile:
+    // the conjugates of those below it
+    const bool flip = lower && tt.x == tt.y && (tc >> 4) > (tr >> 4);
+    const int src = flip ? tc * GT + tr : rc;
     double sr = 0.0, si = 0.0;
     for (int c = 0; c < nchunks; c++) {
-        const double2 v = partial[((long)c * ntiles + tile) * per + rc];
+        const double2 v = partial[((long)c * ntiles + tile) * per + src];
         sr += v.x;
         si += v.y;
     }
+    if (flip) si = -si;
     out[(long)row * ldo + col] =
         make_double2(alpha * sr, conj ? -alpha * si : alpha * si);
 }
@@ -521,8 +585,21 @@ int gram(BandWork& w, const double2* A, long lda, const double2* B, long ldb,
         set_error("gram: no points");
         return EINVAL_;
     }
-    // chunks: about 9 blocks per CU (256 CUs), at least 4 stages each
-    long chunks = std::max(1L, (long)(2304 + nt - 1) / nt);
+    // chunks: 6 to 10 blocks per CU (256 CUs, one block at a time each), the
+    // count that leaves the last round fullest (500 bands, 10 lower tiles:
+    // 231 chunks started a tenth round for 6 blocks, 18.6 ms); at least 4
+    // stages each
+    long chunks = 1;
+    double best = 0.0;
+    for (long c = std::max(1L, 1536L / nt); c <= std::max(1L, 2560L / nt);
+         c++) {
+        const long b = nt * c;
+        const double full = (double)b / ((b + 255) / 256 * 256);
+        if (full >= best) {
+            best = full;
+            chunks = c;
+        }
+    }
     chunks = std::min(chunks, std::max(1L, K / (4 * GK)));
     long kchunk = (K + chunks - 1) / chunks;
     kchunk = (kchunk + GK - 1) / GK * GK;
@@ -541,10 +618,9 @@ int gram(BandWork& w, const double2* A, long lda, const double2* B, long ldb,
     g.nchunks = (int)chunks;
     g.ntiles = nt;
     g.tcols = TN;
-    g.lower = lower_only;
     g.partial = (double2*)w.partial;
-    hipLaunchKernelGGL(k_gram, dim3((unsigned)(nt * chunks)), dim3(512), 0, s,
-                       g);
+    hipLaunchKernelGGL((lower_only ? k_gram<true> : k_gram<false>),
+                       dim3((unsigned)(nt * chunks)), dim3(512), 0, s, g);
     GFD_LAUNCH_CHECK();
     const long total = (long)GT * GT * nt;
     hipLaunchKernelGGL(k_gram_reduce, dim3((unsigned)((total + 255) / 256)),

@@ -15,8 +15,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <type_traits>
-#include <utility>
 
 #include "stencil_dev.h"
 
@@ -422,17 +420,6 @@ k_coarse(const CGrid* __restrict__ grids, const T* __restrict__ rhs,
 // level (a deeper one has at most a quarter of its columns) and not with
 // the Chebyshev iteration.
 constexpr int C1_NT = 1024, C1_X = 12, C1_XFIRST = 24;
-
-// f(0) .. f(N - 1) with constant indices, so that the register arrays they
-// index stay scalars (a loop unrolled later is promoted to vector registers
-// too early, with thousands of spills)
-template <int N, typename F>
-__device__ __forceinline__ void cfor(F&& f)
-{
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-        (f(std::integral_constant<int, I>{}), ...);
-    }(std::make_integer_sequence<int, N>{});
-}
 
 template <typename T>
 struct CSeg {

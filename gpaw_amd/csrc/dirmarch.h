@@ -1,0 +1,59 @@
+// Stencils made of straight lines of points through the centre (axis
+// stencils, the Laplacians and gradients of skew cells, the Mehrstellen
+// pair), marching along x.
+#pragma once
+
+#include "stencil.h"
+
+namespace gfd {
+
+constexpr int DM_NI = 3;  // in-plane directions: (0, 1), (1, 0) and one more
+constexpr int DM_NM = 4;  // directions (1, dy, dz) off the x axis
+
+// in(x + k d) has coefficient p[k - 1], in(x - k d) m[k - 1], k = 1..R
+struct DirLine {
+    int on;      // the stencil has points on it
+    int dy, dz;
+    double p[MAXR_FAST], m[MAXR_FAST];
+};
+
+struct DirStencil {
+    int R = 0;
+    int ni = 2, nm = 0;  // in-plane / mixed directions
+    int sym = 1;         // every p[k] equals its m[k]
+    DirLine x, in[DM_NI], mix[DM_NM];
+};
+
+// The direction form of P points (offsets as triples); false when a point is
+// not a multiple of a direction with components -1, 0, 1, is given twice,
+// lies beyond MAXR_FAST steps, or more directions are needed.
+bool dir_stencil(int P, const double* coef, const int* off, DirStencil& d);
+
+// Whether k_dirmarch takes this pass.
+bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], long nin,
+                   int epi);
+long dirmarch_max_blocks(const DirStencil& d, int dtype, const int n[3],
+                         long nin);
+int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
+                    const BC& bc, const void* in, void* out, long nin,
+                    int epi, const EpiArgs& ea, hipStream_t s,
+                    int* nblocks_out);
+
+struct DirTile {
+    int tz, ty, xchunk;
+};
+
+int dirmarch_f64(const DirStencil& d, const DirTile& t, const int n[3],
+                 const BC& bc, const void* in, void* out, long nin, int epi,
+                 const EpiArgs& ea, hipStream_t s, int* nblocks_out);
+int dirmarch_c128(const DirStencil& d, const DirTile& t, const int n[3],
+                  const BC& bc, const void* in, void* out, long nin, int epi,
+                  const EpiArgs& ea, hipStream_t s, int* nblocks_out);
+int dirmarch_f32(const DirStencil& d, const DirTile& t, const int n[3],
+                 const BC& bc, const void* in, void* out, long nin, int epi,
+                 const EpiArgs& ea, hipStream_t s, int* nblocks_out);
+int dirmarch_c64(const DirStencil& d, const DirTile& t, const int n[3],
+                 const BC& bc, const void* in, void* out, long nin, int epi,
+                 const EpiArgs& ea, hipStream_t s, int* nblocks_out);
+
+}  // namespace gfd

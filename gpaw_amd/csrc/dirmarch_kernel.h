@@ -1,0 +1,443 @@
+// k_dirmarch: one pass of a direction stencil (dirmarch.h).  Included by the
+// dirmarch_*.hip units, one per data type.
+//
+// A block owns a (ty x tz) tile of one grid and marches along x.  Each input
+// plane of the tile with its R-wide halo is staged in LDS (double buffered,
+// one barrier per plane; every thread loads its share of the extended tile,
+// so halo and own points are one stream of loads) and used once for
+// everything it contributes to: a thread keeps one accumulator per output
+// plane x - R .. x + R of its column, adds the in-plane directions to the
+// middle one and every k-th point of a direction (1, dy, dz) to the one k
+// planes away, and stores the oldest.  The plane loop is unrolled by the
+// 2R + 1 accumulators, which are thereby renamed instead of moved.
+//
+// The centre value waits in a queue of R + 1 for its output plane and is
+// added last: the largest term of the sum, whose rounding every term after
+// it would inherit.
+//
+// All global traffic goes through per-plane buffer resources: zero
+// boundaries and idle lanes are out-of-range offsets, not branches.
+//
+// What bounds it: the loads and stores where the batch fills the chip; LDS
+// reads for the skew-cell stencils (18 of 16 bytes per complex point of the
+// 25-point hexagonal Laplacian).
+#pragma once
+
+#include "dirmarch.h"
+
+#include "batch.h"
+#include "rows.h"
+#include "stencil_dev.h"
+
+namespace gfd {
+
+constexpr int DM_NT = 512;  // most threads of a block
+constexpr int DM_HM = 4;    // staged elements per thread
+
+template <typename T>
+struct DmArgs {
+    const T* in;
+    void* out;
+    const void* aux;
+    int n0, n1, n2;
+    int tz, ty, tiles_z, tiles_y, chunks_x, xchunk, nblocks;
+    int hm;              // staged elements per thread, at most DM_HM
+    int epi, nt;
+    double c0, w, s;
+    int negate;
+    DirStencil st;
+    BC bc;
+    double* partial;
+    const double* shift;
+};
+
+template <typename T>
+__device__ inline void dm_store(T v, __amdgpu_buffer_rsrc_t r, unsigned off,
+                                bool nt)
+{
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    if constexpr (sizeof(T) == 4) {
+        __builtin_amdgcn_raw_buffer_store_b32(
+            __builtin_bit_cast(unsigned, v), r, (int)off, 0, 0);
+    } else if constexpr (sizeof(T) == 8) {
+        if (nt)
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v),
+                                                  r, (int)off, 0, 2);
+        else
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v),
+                                                  r, (int)off, 0, 0);
+    } else {
+        if (nt)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v),
+                                                   r, (int)off, 0, 2);
+        else
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v),
+                                                   r, (int)off, 0, 0);
+    }
+}
+
+__device__ inline float dm_narrow(double v) { return (float)v; }
+__device__ inline float2 dm_narrow(double2 v)
+{
+    return make_float2((float)v.x, (float)v.y);
+}
+
+// what an epilogue reads beside the stencil input
+enum DmAux : int { DM_NONE = 0, DM_SAME = 1, DM_POT = 2, DM_WIDE = 3 };
+
+// AUX: DmAux.  NARROW: FP64 input, result stored as FP32 (EPI_RESN).
+// SYM: equal coefficients on both sides of the centre (one copy of them:
+// the scalar registers hold all of a Laplacian's then).
+template <typename T, int R, int NI, int NM, int AUX, bool SYM, bool NARROW>
+__global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
+{
+    typedef typename ScalarOf<T>::type S;
+    typedef typename WideOf<T>::type WT;
+    typedef typename std::conditional<
+        AUX == DM_POT, double,
+        typename std::conditional<AUX == DM_WIDE, WT, T>::type>::type TA;
+    constexpr int U = 2 * R + 1;
+    constexpr bool CPLX = IsCplx<T>::value;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* lds = reinterpret_cast<T*>(smem_raw);
+
+    const int L = xcd_remap(blockIdx.x, a.nblocks);
+    int rem = L;
+    const int zt = rem % a.tiles_z;
+    rem /= a.tiles_z;
+    const int yt = rem % a.tiles_y;
+    rem /= a.tiles_y;
+    const int cx = rem % a.chunks_x;
+    const long b = rem / a.chunks_x;
+
+    const int tid = threadIdx.x, NT = blockDim.x;
+    const int n0 = a.n0, n1 = a.n1, n2 = a.n2;
+    const long plane = (long)n1 * n2, ng = plane * n0;
+    const int z0 = zt * a.tz, y0 = yt * a.ty;
+    const int xs = cx * a.xchunk, xe = min(xs + a.xchunk, n0);
+    const int LW = a.tz + 2 * R, LSZ = (a.ty + 2 * R) * LW;
+    const T* __restrict__ gin = a.in + b * ng;
+    const unsigned pbytes = (unsigned)(plane * (long)sizeof(T));
+    const BC& bc = a.bc;
+
+    // staged elements tid + m NT of the extended tile: offset in the plane
+    // (BXM_OOB: zero or unused) and Bloch factor of the y and z wraps
+    unsigned hoff[DM_HM];
+    bool hph[DM_HM];
+    double2 hf[DM_HM];
+#pragma unroll
+    for (int m = 0; m < DM_HM; m++) {
+        const int e = tid + m * NT;
+        hoff[m] = BXM_OOB;
+        hph[m] = false;
+        hf[m] = make_double2(1.0, 0.0);
+        if (e < LSZ) {
+            const int row = e / LW;
+            int y = y0 + row - R, z = z0 + (e - row * LW) - R;
+            // beyond the halo of the last row or column: never read
+            if (y < n1 + R && z < n2 + R &&
+                wrap_full(z, n2, bc.periodic[2], bc.phase[2][0],
+                          bc.phase[2][1], hf[m], hph[m]) &&
+                wrap_full(y, n1, bc.periodic[1], bc.phase[1][0],
+                          bc.phase[1][1], hf[m], hph[m]))
+                hoff[m] = (unsigned)(y * n2 + z) * (unsigned)sizeof(T);
+        }
+    }
+    // own point
+    const int tr = tid / a.tz, tc = tid - tr * a.tz;
+    const bool on = tr < a.ty && y0 + tr < n1 && z0 + tc < n2;
+    const int lown = (min(tr, a.ty - 1) + R) * LW + tc + R;
+    const unsigned oidx = on ? (unsigned)((y0 + tr) * n2 + z0 + tc) : BXM_OOB;
+    auto bytes_at = [&](unsigned es) { return on ? oidx * es : BXM_OOB; };
+
+    // input plane of step x (wrapped; empty beyond a zero boundary)
+    auto in_plane = [&](int x, double2& f, bool& ph) {
+        ph = false;
+        f = make_double2(1.0, 0.0);
+        const bool ok = wrap_full(x, n0, bc.periodic[0], bc.phase[0][0],
+                                  bc.phase[0][1], f, ph);
+        return brsrc(gin + (long)(ok ? x : 0) * plane, ok ? pbytes : 0u);
+    };
+    T hv[DM_HM];
+    double2 fx;
+    bool phx;
+    auto ld_plane = [&](int x) {
+        const __amdgpu_buffer_rsrc_t r = in_plane(x, fx, phx);
+#pragma unroll
+        for (int m = 0; m < DM_HM; m++)
+            if (m < a.hm) hv[m] = bload<T>(r, hoff[m]);
+    };
+    TA av{};
+    // auxiliary operand of output plane x
+    auto ld_aux = [&](int x) {
+        if constexpr (AUX != DM_NONE) {
+            const bool ok = x >= xs && x < xe;
+            const TA* p = (const TA*)a.aux + (AUX == DM_POT ? 0 : b * ng) +
+                          (long)(ok ? x : xs) * plane;
+            av = bload<TA>(brsrc(p, (unsigned)(plane * (long)sizeof(TA))),
+                           bytes_at(sizeof(TA)));
+        }
+    };
+    auto cm = [](const DirLine& l, int k) {
+        return (S)(SYM ? l.p[k - 1] : l.m[k - 1]);
+    };
+    S shift = (S)0;
+    if constexpr (AUX == DM_POT)
+        if (a.shift) shift = -(S)a.shift[b];
+
+    T acc[U];
+#pragma unroll
+    for (int j = 0; j < U; j++) acc[j] = zero_of<T>();
+    T vq[R + 1];  // centre values of planes x - R .. x
+#pragma unroll
+    for (int j = 0; j <= R; j++) vq[j] = zero_of<T>();
+    double nrm = 0.0;
+
+    ld_plane(xs - R);
+    int par = 0;
+    for (int xb = xs - R; xb < xe + R; xb += U) {
+        cfor<U>([&](auto uc) {
+            constexpr int u = uc;
+            const int x = xb + u;
+            if (x >= xe + R) return;
+            T* buf = lds + par * LSZ;
+            par ^= 1;
+#pragma unroll
+            for (int m = 0; m < DM_HM; m++)
+                if (m < a.hm) {
+                    T v = hv[m];
+                    if constexpr (CPLX) {
+                        if (hph[m]) v = scale_by<T>(v, hf[m], true);
+                        if (phx) v = scale_by<T>(v, fx, true);
+                    }
+                    const int e = tid + m * NT;
+                    if (e < LSZ) buf[e] = v;
+                }
+            const TA a0 = av;
+            ld_plane(min(x + 1, xe + R - 1));
+            ld_aux(x + 1 - R);
+            __syncthreads();
+
+            // accumulator of output plane x + j: (u + R + j) mod U
+            auto at = [&](auto j) -> T& {
+                constexpr int i = (u + R + decltype(j)::value + U) % U;
+                return acc[i];
+            };
+            constexpr std::integral_constant<int, 0> here;
+            constexpr std::integral_constant<int, -R> oldest;
+            const T* p = buf + lown;
+            const T v = p[0];
+            cfor<R>([&](auto j) { vq[j] = vq[j + 1]; });
+            vq[R] = v;
+            T mid = at(here);
+            // (a direction without points is skipped, not multiplied by
+            // zeros: its neighbours may hold infinities)
+            if (a.st.in[0].on) {
+#pragma unroll
+                for (int k = 1; k <= R; k++) {
+                    mid = fmac(mid, (S)a.st.in[0].p[k - 1], p[k]);
+                    mid = fmac(mid, cm(a.st.in[0], k), p[-k]);
+                }
+            }
+#pragma unroll
+            for (int i = 1; i < NI; i++) {
+                if (!a.st.in[i].on) continue;
+                const int o = i == 1 ? LW
+                                     : a.st.in[i].dy * LW + a.st.in[i].dz;
+#pragma unroll
+                for (int k = 1; k <= R; k++) {
+                    mid = fmac(mid, (S)a.st.in[i].p[k - 1], p[k * o]);
+                    mid = fmac(mid, cm(a.st.in[i], k), p[-k * o]);
+                }
+            }
+            at(here) = mid;
+            // the point k steps ahead of output x - k, behind output x + k
+            if (a.st.x.on)
+                cfor<R>([&](auto k0) {
+                    constexpr int k = k0 + 1;
+                    std::integral_constant<int, -k> ahead;
+                    std::integral_constant<int, k> behind;
+                    at(ahead) = fmac(at(ahead), (S)a.st.x.p[k - 1], v);
+                    at(behind) = fmac(at(behind), cm(a.st.x, k), v);
+                });
+#pragma unroll
+            for (int i = 0; i < NM; i++) {
+                if (!a.st.mix[i].on) continue;
+                const int o = a.st.mix[i].dy * LW + a.st.mix[i].dz;
+                cfor<R>([&](auto k0) {
+                    constexpr int k = k0 + 1;
+                    std::integral_constant<int, -k> ahead;
+                    std::integral_constant<int, k> behind;
+                    at(ahead) = fmac(at(ahead), (S)a.st.mix[i].p[k - 1],
+                                     p[k * o]);
+                    at(behind) = fmac(at(behind), cm(a.st.mix[i], k),
+                                      p[-k * o]);
+                });
+            }
+            // output plane x - R is complete
+            const int xo = x - R;
+            if (xo >= xs) {
+                T r = at(oldest);
+                const T vo = vq[0];
+                if constexpr (AUX == DM_POT) {
+                    r = fmac(fmac(r, (S)a.c0, vo), (S)a0, vo);
+                    if (a.shift) r = fmac(r, shift, vo);
+                } else if constexpr (AUX == DM_NONE) {
+                    r = fmac(r, (S)a.c0, vo);
+                } else {
+                    T ax;
+                    if constexpr (AUX == DM_WIDE) ax = dm_narrow(a0);
+                    else ax = a0;
+                    if (a.epi == EPI_RELAX)
+                        r = epi_apply<T, EPI_RELAX>(r, vo, ax, a.c0, a.w, a.s,
+                                                    a.negate, nrm);
+                    else if (a.epi == EPI_RESID) {
+                        r = fmac(r, (S)a.c0, vo) - ax;
+                        if (on) nrm += sq(r);
+                    } else
+                        r = epi_apply<T, EPI_UPDATE>(r, vo, ax, a.c0, a.w,
+                                                     a.s, a.negate, nrm);
+                }
+                if constexpr (NARROW) {
+                    const __amdgpu_buffer_rsrc_t ro =
+                        brsrc((float*)a.out + b * ng + (long)xo * plane,
+                              (unsigned)(plane * 4));
+                    dm_store((float)r, ro, bytes_at(4), false);
+                } else if constexpr (AUX == DM_WIDE) {
+                    const __amdgpu_buffer_rsrc_t ro = brsrc(
+                        (WT*)a.out + b * ng + (long)xo * plane,
+                        (unsigned)(plane * (long)sizeof(WT)));
+                    dm_store(to_wide(r), ro, bytes_at(sizeof(WT)),
+                             a.nt != 0);
+                } else {
+                    const __amdgpu_buffer_rsrc_t ro =
+                        brsrc((T*)a.out + b * ng + (long)xo * plane, pbytes);
+                    dm_store(r, ro, bytes_at(sizeof(T)), a.nt != 0);
+                }
+            }
+            at(oldest) = zero_of<T>();
+        });
+    }
+    if (a.partial) block_sum_store(nrm, a.partial, L);
+}
+
+template <typename T, int R, int NI, int NM, int AUX, bool SYM = true,
+          bool NARROW = false>
+static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
+                       const BC& bc, const void* in, void* out, long nin,
+                       int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
+{
+    DmArgs<T> a;
+    a.in = (const T*)in;
+    a.out = out;
+    a.aux = AUX == DM_POT ? (const void*)ea.pot : ea.aux;
+    a.n0 = n[0];
+    a.n1 = n[1];
+    a.n2 = n[2];
+    a.tz = t.tz;
+    a.ty = t.ty;
+    a.tiles_z = ceil_div(n[2], t.tz);
+    a.tiles_y = ceil_div(n[1], t.ty);
+    a.xchunk = t.xchunk;
+    a.chunks_x = ceil_div(n[0], t.xchunk);
+    const long nb = (long)a.tiles_z * a.tiles_y * a.chunks_x * nin;
+    const int threads = (t.tz * t.ty + 63) / 64 * 64;
+    const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
+    if (nb <= 0) return OK;
+    if (nb > 0x7fffffffL || threads > DM_NT ||
+        lsz > (long)DM_HM * threads) {
+        set_error("direction march: %ld blocks of %d x %d do not fit", nb,
+                  t.ty, t.tz);
+        return ENOTSUP_;
+    }
+    a.nblocks = (int)nb;
+    a.hm = ceil_div(lsz, threads);
+    a.nt = xr_nt_flags((long)n[0] * n[1] * n[2] * nin * (long)sizeof(T)) & 1;
+    a.epi = epi == EPI_RESN ? (int)EPI_RESID : epi;
+    a.c0 = ea.c0;
+    a.w = ea.w;
+    a.s = ea.s;
+    a.negate = ea.negate;
+    a.st = d;
+    a.bc = bc;
+    a.partial = epi == EPI_RESID || epi == EPI_RESN ? ea.partial : nullptr;
+    a.shift = ea.shift;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL((k_dirmarch<T, R, NI, NM, AUX, SYM, NARROW>),
+                       dim3((unsigned)nb), dim3(threads),
+                       2 * lsz * sizeof(T), s, a);
+    GFD_LAUNCH_CHECK();
+    if (nbo) *nbo = (int)nb;
+    return OK;
+}
+
+template <typename T, int R, int NI, int NM>
+static int dm_launch_e(const DirStencil& d, const DirTile& t, const int n[3],
+                       const BC& bc, const void* in, void* out, long nin,
+                       int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
+{
+#define GFD_DM(...)                                                         \
+    return dm_launch_t<T, R, NI, NM, __VA_ARGS__>(d, t, n, bc, in, out,     \
+                                                  nin, epi, ea, s, nbo)
+    switch (epi) {
+    case EPI_PLAIN:
+        if (!d.sym) GFD_DM(DM_NONE, false);
+        GFD_DM(DM_NONE);
+    case EPI_RELAX:
+    case EPI_RESID:
+    case EPI_UPDATE: GFD_DM(DM_SAME);
+    case EPI_POT:
+        if constexpr (sizeof(typename ScalarOf<T>::type) == 8)
+            GFD_DM(DM_POT);
+        break;
+    case EPI_UPDW:
+        if constexpr (sizeof(typename ScalarOf<T>::type) == 4)
+            GFD_DM(DM_WIDE);
+        break;
+    case EPI_RESN:
+        if constexpr (std::is_same<T, double>::value) GFD_DM(DM_SAME, true, true);
+        break;
+    }
+#undef GFD_DM
+    set_error("direction march: epilogue %d not built", epi);
+    return ENOTSUP_;
+}
+
+template <typename T, int R>
+static int dm_launch_r(const DirStencil& d, const DirTile& t, const int n[3],
+                       const BC& bc, const void* in, void* out, long nin,
+                       int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
+{
+#define GFD_DM(NI, NM)                                                      \
+    if (d.ni <= NI && d.nm <= NM)                                           \
+        return dm_launch_e<T, R, NI, NM>(d, t, n, bc, in, out, nin, epi,    \
+                                         ea, s, nbo)
+    GFD_DM(2, 0);
+    if constexpr (R <= 3) {
+        GFD_DM(2, 1);
+        GFD_DM(3, 0);
+        GFD_DM(3, 2);
+        GFD_DM(3, 4);
+    }
+#undef GFD_DM
+    set_error("direction march: too many directions");
+    return ENOTSUP_;
+}
+
+template <typename T>
+static int dm_launch(const DirStencil& d, const DirTile& t, const int n[3],
+                     const BC& bc, const void* in, void* out, long nin,
+                     int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
+{
+    switch (d.R) {
+    case 1: return dm_launch_r<T, 1>(d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+    case 2: return dm_launch_r<T, 2>(d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+    case 3: return dm_launch_r<T, 3>(d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+    case 4: return dm_launch_r<T, 4>(d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+    }
+    set_error("direction march: radius %d", d.R);
+    return ENOTSUP_;
+}
+
+}  // namespace gfd

@@ -5,6 +5,7 @@
 
 #include <vector>
 
+#include "dirmarch.h"
 #include "gfd_common.h"
 #include "stencil.h"
 #include "transfer.h"
@@ -83,6 +84,8 @@ struct gfd_operator {
         g.off = d_off;
         return g;
     }
+    gfd::DirStencil dir;   // direction form (dir_ok)
+    bool dir_ok = false;
     bool use_fast() const { return axis_ok && g_force_path != 1; }
 };
 

@@ -2,9 +2,23 @@
 // reductions, XCD-aware block order).
 #pragma once
 
+#include <type_traits>
+#include <utility>
+
 #include "stencil.h"
 
 namespace gfd {
+
+// f(0) .. f(N - 1) with constant indices, so that the register arrays they
+// index stay scalars (a loop unrolled later is promoted to vector registers
+// too early, with thousands of spills)
+template <int N, typename F>
+__device__ __forceinline__ void cfor(F&& f)
+{
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (f(std::integral_constant<int, I>{}), ...);
+    }(std::make_integer_sequence<int, N>{});
+}
 
 template <typename T> struct IsCplx { static constexpr bool value = false; };
 template <> struct IsCplx<double2> { static constexpr bool value = true; };

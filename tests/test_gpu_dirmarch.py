@@ -1,0 +1,160 @@
+"""The direction march: stencils whose points lie on straight lines through
+the centre, against the oracle, over cells, boundaries, data types, odd
+sides, tile remainders and every epilogue."""
+import contextlib
+
+import numpy as np
+import pytest
+
+import oracle
+from gpaw_amd import _lib, bands
+from gpaw_amd.fd_operators import (FDOperator, Gradient, Laplace, LaplaceA,
+                                   LaplaceB)
+from gpaw_amd.grid_descriptor import GridDescriptor
+from gpu_util import dev, host, say
+from helpers import bloch_phases, rand, relerr, spec
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-13
+
+HEX = np.array([[1, 0, 0], [-0.5, 0.75**0.5, 0], [0, 0, 1.1]])
+FCC = np.array([[0, 1, 1], [1, 0, 1], [1, 1, 0]]) * 0.5**0.5
+BCC = np.array([[-1, 1, 1], [1, -1, 1], [1, 1, -1]]) * 0.5
+SKEW = np.array([[1, 0.13, 0.04], [0.2, 1.05, -0.11], [-0.1, 0.15, 0.95]])
+CELLS = {'box': np.eye(3), 'hex': HEX, 'fcc': FCC, 'bcc': BCC, 'skew': SKEW}
+
+
+@contextlib.contextmanager
+def path(p):
+    lib = _lib.load()
+    _lib.check(lib.gfd_set_tuning(b'force_path', p), 'force_path')
+    try:
+        yield
+    finally:
+        lib.gfd_set_tuning(b'force_path', 0)
+
+
+def grid(N, cell, pbc):
+    return GridDescriptor(N, CELLS[cell] * 0.3 * np.array(N)[:, None], pbc)
+
+
+@pytest.mark.parametrize('cell', list(CELLS))
+@pytest.mark.parametrize('nn', [1, 2, 3])
+@pytest.mark.parametrize('N,pbc', [((8, 7, 9), True),
+                                   ((13, 22, 71), (True, True, False)),
+                                   ((24, 19, 130), False)])
+@pytest.mark.parametrize('dtype', [float, complex])
+def test_laplace(cell, nn, N, pbc, dtype):
+    rng = np.random.default_rng(nn)
+    gd = grid(N, cell, pbc)
+    op = Laplace(gd, -0.7, nn, dtype)
+    a = rand(rng, (3,) + tuple(gd.n_c), dtype)
+    ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
+    out = dev(np.zeros_like(a))
+    say('dirmarch laplace', cell, nn, N, pbc, dtype)
+    with path(4):
+        op.apply(dev(a), out, ph)
+    ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a,
+                          ph)
+    assert relerr(host(out), ref) < TOL
+
+
+@pytest.mark.parametrize('make', [
+    lambda gd: Gradient(gd, 1, 1.0, 3), lambda gd: LaplaceA(gd, 0.3),
+    lambda gd: LaplaceB(gd),
+    lambda gd: FDOperator([1.0, 0.5], [(0, 0, 0), (0, 2, 2)], gd)])
+def test_other_stencils(make):
+    """One axis only, the Mehrstellen pair (edges of the cube), points on
+    one side of the centre."""
+    rng = np.random.default_rng(3)
+    gd = grid((9, 20, 33), 'box', (True, False, True))
+    op = make(gd)
+    a = rand(rng, (2,) + tuple(gd.n_c))
+    out = dev(np.zeros_like(a))
+    say('dirmarch stencil', op.description)
+    with path(4):
+        op.apply(dev(a), out)
+    ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a)
+    assert relerr(host(out), ref) < TOL
+
+
+def test_infinities_stay_on_their_lines():
+    """A direction without points does not multiply its neighbours."""
+    gd = grid((8, 9, 12), 'box', True)
+    op = Gradient(gd, 2, 1.0, 2)
+    a = np.ones((1, 8, 9, 12))
+    a[0, 4, 4, :] = np.inf
+    out = dev(np.zeros_like(a))
+    with path(4):
+        op.apply(dev(a), out)
+    bad = ~np.isfinite(host(out)[0])
+    assert bad[4, 4].all() and bad.sum() == 12
+
+
+@pytest.mark.parametrize('cell,N,pbc', [('box', (14, 23, 47), False),
+                                        ('hex', (12, 12, 21), True)])
+def test_epilogues(cell, N, pbc):
+    """Jacobi sweeps, residual with its norm, H psi - eps psi, on the shapes
+    the full-row kernel does not take."""
+    rng = np.random.default_rng(11)
+    gd = grid(N, cell, pbc)
+    n = tuple(gd.n_c)
+    op = Laplace(gd, -0.5, 3)
+    sp = spec(op)
+    f, src = rand(rng, n), rand(rng, n)
+    say('dirmarch epilogues', cell, N)
+    with path(4):
+        for w in (2.0 / 3.0, 1.0):
+            g = dev(f.copy())
+            op.relax(2, g, dev(src), 3, w)
+            ref = oracle.fd_relax(2, op.coef_p, op.offset_pc, gd.n_c,
+                                  gd.neighbor_cd, f.copy(), src, 3, w)
+            assert relerr(host(g), ref) < TOL
+        lib = _lib.load()
+        r = dev(np.zeros_like(f))
+        df, ds = dev(f), dev(src)
+        norm = _lib.ctypes.c_double()
+        _lib.check(lib.gfd_operator_residual(
+            op._handle(), df.data_ptr(), ds.data_ptr(), r.data_ptr(), 1,
+            None, _lib.ctypes.byref(norm), None), 'residual')
+        want = oracle.fd_apply(sp.coef_p, sp.offset_pc, gd.n_c,
+                               gd.neighbor_cd, f) - src
+        assert relerr(host(r), want) < TOL
+        assert abs(norm.value / (want**2).sum() - 1) < 1e-12
+        for dtype in (float, complex):
+            kin = Laplace(gd, -0.5, 3, dtype)
+            psi = rand(rng, (3,) + n, dtype)
+            vt, eps = rng.uniform(-2, 0, n), rng.uniform(-1, 1, 3)
+            ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
+            out = dev(np.zeros_like(psi))
+            bands.apply_hamiltonian(kin, dev(vt), dev(psi), out, ph,
+                                    eps=dev(eps))
+            want = oracle.fd_apply(kin.coef_p, kin.offset_pc, gd.n_c,
+                                   gd.neighbor_cd, psi, ph) + \
+                (vt - eps[:, None, None, None]) * psi
+            assert relerr(host(out), want) < TOL
+
+
+@pytest.mark.parametrize('cell,N,pbc', [('box', (20, 28, 36), False),
+                                        ('hex', (16, 16, 24), True)])
+@pytest.mark.parametrize('dtype', [float, complex])
+@pytest.mark.parametrize('fp32', [False, True])
+def test_preconditioner(cell, N, pbc, dtype, fp32):
+    """The UPDATE epilogues, FP32 data with FP64 residual and result among
+    them, against the general kernel (2e-6: the FP32 chain's bar)."""
+    from types import SimpleNamespace
+
+    from gpaw_amd.preconditioner import Preconditioner
+    rng = np.random.default_rng(5)
+    gd = grid(N, cell, pbc)
+    kin = Laplace(gd, -0.5, 3, dtype)
+    pc = Preconditioner(gd, kin, dtype, block=3, fp32=fp32)
+    res = dev(rand(rng, (3,) + tuple(gd.n_c), dtype))
+    ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
+    kpt = SimpleNamespace(phase_cd=ph)
+    outs = []
+    say('dirmarch preconditioner', cell, N, dtype, fp32)
+    for p in (4, 1):
+        with path(p):
+            outs.append(host(pc(res, kpt)))
+    assert relerr(outs[0], outs[1]) < (2e-6 if fp32 else TOL)
