@@ -41,8 +41,7 @@ void set_error(const char* fmt, ...)
 
 const char* last_error() { return g_err.c_str(); }
 
-// 0 auto, 1 general kernel, 2 tiled x-march kernel, 3 full-row kernel,
-// 4 direction march
+// 0 auto, 1 general kernel, 2 direction march, 3 full-row kernel
 int g_force_path = 0;
 
 static BC make_bc(const int periodic[3], const double* phases)
@@ -236,32 +235,27 @@ static bool aligned16(const void* p)
     return ((uintptr_t)p & 15) == 0;
 }
 
-// Kernel family for one pass: 3 full-row, 4 direction march, 2 tiled
-// x-march, 1 general.
+// Kernel family for one pass: 3 full-row, 2 direction march, 1 general.
 static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
                    const void* out, const void* aux, int epi)
 {
-    const bool dir = op->dir_ok &&
-                     (g_force_path == 0 || g_force_path == 4) &&
-                     dirmarch_fits(op->dir, dtype, op->n, nin, epi);
-    if (dir && g_force_path == 4) return 4;
-    if (!op->use_fast()) return dir ? 4 : 1;
-    const bool row = (g_force_path == 0 || g_force_path == 3) &&
-                     aligned16(in) && aligned16(out) &&
-                     (aux == nullptr || aligned16(aux)) &&
-                     row_stencil_fits(op->ax, dtype, op->n, nin);
-    if (row) return 3;
-    if (dir) return 4;
-    // epilogues the tiled x-march kernel instantiates per data type
-    const bool xm_has =
-        (dtype == 0 && epi <= EPI_UPDATE) ||
-        (dtype == 1 && (epi == EPI_PLAIN || epi == EPI_RESID ||
-                        epi == EPI_UPDATE)) ||
-        (dtype == 2 && epi <= EPI_RESID);
-    if (xm_has && (g_force_path == 0 || g_force_path == 2) &&
-        axis_stencil_fits(op->ax, dtype, op->n, nin))
-        return 2;
-    return 1;
+    if (g_force_path == 1) return 1;
+    const bool dir = op->dir_ok && g_force_path != 3 &&
+                     dirmarch_fits(op->dir, dtype, op->n, epi);
+    if (dir && g_force_path == 2) return 2;
+    // Complex FP64: the direction march from radius 3 on and for H psi at
+    // any radius.  k_xrow holds 2R + 2 planes of 16-byte points in registers
+    // (2 waves per SIMD at R = 3); measured over 1, 4 and 32 grids of 48^3,
+    // 96^3, 128^3 and 64x100x180, its time over the march's: H psi 1.11-1.84
+    // at R = 3, 1.26-4.1 at R = 4, 1.11-1.57 at R = 2, 0.99-1.72 at R = 1;
+    // plain passes 1.03-1.70 at R = 3, 1.06-4.1 at R = 4, but 0.92-1.20
+    // below.  Real data: 0.70-1.10 (plain), so the full rows stay first.
+    if (dir && dtype == 1 && (op->dir.R >= 3 || epi == EPI_POT)) return 2;
+    if (op->axis_ok && g_force_path != 2 && aligned16(in) &&
+        aligned16(out) && (aux == nullptr || aligned16(aux)) &&
+        row_stencil_fits(op->ax, dtype, op->n, nin))
+        return 3;
+    return dir ? 2 : 1;
 }
 
 // One stencil pass with an epilogue (the building block of every driver).
@@ -274,12 +268,9 @@ static int op_pass(gfd_operator* op, int dtype, const void* in, void* out,
     if (path == 3)
         return launch_row_stencil(op->ax, dtype, op->n, bc, in, out, nin, epi,
                                   ea, s, nblocks);
-    if (path == 4)
+    if (path == 2)
         return launch_dirmarch(op->dir, dtype, op->n, bc, in, out, nin, epi,
                                ea, s, nblocks);
-    if (path == 2)
-        return launch_axis_stencil(op->ax, dtype, op->n, bc, in, out, nin, epi,
-                                   ea, s, nblocks);
     return launch_general_stencil(op->gen(ea.c0), dtype, op->n, bc, in, out,
                                   nin, epi, ea, s, nblocks);
 }
@@ -291,7 +282,6 @@ static long op_max_blocks(gfd_operator* op, int dtype, long nin)
     if (op->dir_ok)
         m = std::max(m, dirmarch_max_blocks(op->dir, dtype, op->n, nin));
     if (op->use_fast()) {
-        m = std::max(m, axis_stencil_max_blocks(op->ax, dtype, op->n, nin));
         m = std::max(m, row_stencil_max_blocks(op->ax, dtype, op->n, nin));
     }
     return m;
@@ -1849,8 +1839,8 @@ extern "C" int gfd_set_tuning(const char* key, long value)
         return OK;
     }
     if (std::strcmp(key, "force_path") == 0) {
-        if (value < 0 || value > 4) {
-            set_error("gfd_set_tuning: force_path must be 0..4");
+        if (value < 0 || value > 3) {
+            set_error("gfd_set_tuning: force_path must be 0..3");
             return EINVAL_;
         }
         g_force_path = (int)value;
@@ -1984,7 +1974,7 @@ extern "C" int gfd_set_tuning(const char* key, long value)
     }
     if (std::strcmp(key, "xm_tile") == 0) {
         if (value == 0) {
-            xm_set_override(nullptr);
+            dirmarch_set_tile(nullptr);
             return OK;
         }
         XmTile t;
@@ -1996,7 +1986,7 @@ extern "C" int gfd_set_tuning(const char* key, long value)
             set_error("gfd_set_tuning: bad xm_tile");
             return EINVAL_;
         }
-        xm_set_override(&t);
+        dirmarch_set_tile(&t);
         return OK;
     }
     set_error("gfd_set_tuning: unknown key '%s'", key);

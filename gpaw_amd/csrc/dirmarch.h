@@ -9,6 +9,9 @@ namespace gfd {
 
 constexpr int DM_NI = 3;  // in-plane directions: (0, 1), (1, 0) and one more
 constexpr int DM_NM = 4;  // directions (1, dy, dz) off the x axis
+// largest radius of the skew forms (the 9 accumulators of radius 4 and the
+// directions do not fit the registers)
+constexpr int DM_RSKEW = 3;
 
 // in(x + k d) has coefficient p[k - 1], in(x - k d) m[k - 1], k = 1..R
 struct DirLine {
@@ -20,7 +23,7 @@ struct DirLine {
 struct DirStencil {
     int R = 0;
     int ni = 2, nm = 0;  // in-plane / mixed directions
-    int sym = 1;         // every p[k] equals its m[k]
+    int full = 0;  // x and the ni, nm directions all there, p[k] = m[k]
     DirLine x, in[DM_NI], mix[DM_NM];
 };
 
@@ -30,14 +33,18 @@ struct DirStencil {
 bool dir_stencil(int P, const double* coef, const int* off, DirStencil& d);
 
 // Whether k_dirmarch takes this pass.
-bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], long nin,
-                   int epi);
+bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi);
 long dirmarch_max_blocks(const DirStencil& d, int dtype, const int n[3],
                          long nin);
 int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
                     const BC& bc, const void* in, void* out, long nin,
                     int epi, const EpiArgs& ea, hipStream_t s,
                     int* nblocks_out);
+
+// Tile in place of the estimated one (tuning key "xm_tile"; rows nseg x py),
+// where it fits and the pass sums no norm (its buffer is sized for the
+// estimated tile); nullptr clears.
+void dirmarch_set_tile(const XmTile* t);
 
 struct DirTile {
     int tz, ty, xchunk;

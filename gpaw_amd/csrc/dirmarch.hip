@@ -2,9 +2,8 @@
 #include "dirmarch.h"
 
 #include <algorithm>
-#include <cstdio>
 #include <cstdlib>
-#include <cstring>
+#include <mutex>
 
 namespace gfd {
 
@@ -64,91 +63,83 @@ bool dir_stencil(int P, const double* coef, const int* off, DirStencil& d)
         (sg > 0 ? line->p : line->m)[k - 1] = coef[q];
         d.R = std::max(d.R, k);
     }
-    auto same = [](const DirLine& l) {
-        return std::equal(l.p, l.p + MAXR_FAST, l.m);
+    auto full = [](const DirLine& l) {
+        return l.on && std::equal(l.p, l.p + MAXR_FAST, l.m);
     };
-    d.sym = same(d.x);
-    for (const DirLine& l : d.in) d.sym = d.sym && same(l);
-    for (const DirLine& l : d.mix) d.sym = d.sym && same(l);
+    d.full = full(d.x) && std::all_of(d.in, d.in + d.ni, full) &&
+             std::all_of(d.mix, d.mix + d.nm, full);
     return d.R > 0;
 }
 
-// largest radius of the skew forms (9 accumulators and their directions do
-// not fit the registers)
-constexpr int DM_RSKEW = 3;
 constexpr int DM_THREADS = 512;
-constexpr int DM_STAGED = 4;  // staged elements per thread
 
-static bool tile_fits(const DirTile& t, int R)
+static std::mutex g_dm_mu;
+static bool g_dm_override = false;
+static DirTile g_dm_tile;
+
+void dirmarch_set_tile(const XmTile* t)
 {
-    const int threads = (t.tz * t.ty + 63) / 64 * 64;
-    return t.tz >= 1 && t.ty >= 1 && t.xchunk >= 1 && threads <= DM_THREADS &&
-           (long)(t.tz + 2 * R) * (t.ty + 2 * R) <= (long)DM_STAGED * threads;
+    std::lock_guard<std::mutex> lk(g_dm_mu);
+    g_dm_override = t != nullptr;
+    if (t) g_dm_tile = DirTile{t->tz, t->nseg * t->py, t->xchunk};
 }
 
-// Tile: equal parts of a row by as many rows as a block holds, the pair with
-// the least work for the whole plane, counting a staged element (a load
-// from L2 and an LDS write) like half a computed lane.  x chunks: whole x
-// unless that leaves the chip idle; every chunk stages 2R planes more, and
-// about two blocks of 512 threads are resident per CU.
-static bool dm_tile(const DirStencil& d, const int n[3], long nin, DirTile& t)
+// Tile (equal parts of a row by as many rows as 512 or 256 threads hold,
+// the rows split evenly) and x chunk with the least estimated time:
+//   planes per block (every chunk stages 2R planes more)
+//   x waves of all blocks of one CU x (1 + 0.12 per staged element)
+//   x (1 + 4 / resident waves per CU): too few do not hide the latency.
+// The weights fit measured sweeps (48 c128 grids of 128^3: 64 x 8 threads
+// 703 us, 128 x 4 with 4 staged elements 795, 32 x 8 802; 40 f64 grids of
+// 87x103x95: 48 x 10 in two chunks 174 us, whole x 184, 95 x 5 209; 24 c128
+// grids of 60x60x84, hexagonal: 28 x 9 in two chunks 55 us, whole x 58, in
+// four 64).
+static DirTile dm_tile(const DirStencil& d, int dtype, const int n[3],
+                       long nin)
 {
     const int R = d.R;
-#ifdef DM_PROBE
-    if (const char* e = getenv("DM_TILE")) {
-        if (sscanf(e, "%d,%d,%d", &t.tz, &t.ty, &t.xchunk) == 3) {
-            t.xchunk = std::min(t.xchunk, n[0]);
-            if (tile_fits(t, R)) return true;
-        }
-    }
-#endif
-    double best = 1e300;
-    bool found = false;
+    // waves a CU holds: complex FP64 takes about 128 registers at R = 3
+    const int hold = dtype == 1 && R > 1 ? 16 : 32;
+    DirTile best{std::min(n[2], 64), std::min(n[1], 8), n[0]};
+    double least = 1e300;
     for (int parts = 1; parts <= n[2]; parts++) {
-        DirTile c;
-        c.tz = (n[2] + parts - 1) / parts;
-        c.xchunk = n[0];
-        if (c.tz > DM_THREADS) continue;
-        if (c.tz < 12 && parts > 1) break;
-        for (int ry = 1; ry <= n[1]; ry++) {
-            c.ty = (n[1] + ry - 1) / ry;
-            if (!tile_fits(c, R)) continue;
-            const int threads = (c.tz * c.ty + 63) / 64 * 64;
-            const double cost =
-                (double)((n[2] + c.tz - 1) / c.tz) *
-                ((n[1] + c.ty - 1) / c.ty) *
-                (threads + 0.5 * (c.tz + 2 * R) * (c.ty + 2 * R));
-            if (cost < best) {
-                best = cost;
-                t = c;
-                found = true;
+        DirTile t;
+        t.tz = (n[2] + parts - 1) / parts;
+        if (t.tz > DM_THREADS) continue;
+        if (t.tz < 16 && parts > 1) break;
+        for (int nt = DM_THREADS; nt >= DM_THREADS / 2; nt /= 2) {
+            if (t.tz > nt) break;
+            const int rows = std::min(nt / t.tz, n[1]);
+            const int nr = (n[1] + rows - 1) / rows;
+            t.ty = (n[1] + nr - 1) / nr;
+            const int threads = (t.tz * t.ty + 63) / 64 * 64;
+            const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
+            if (lsz > 4L * threads) continue;
+            const int hm = lsz <= 2L * threads ? 2 : 4;
+            const int waves = threads / 64;
+            const long tiles = (long)parts * nr * nin;
+            for (int chunks = 1; chunks <= std::max(1, n[0] / 4);
+                 chunks++) {
+                t.xchunk = (n[0] + chunks - 1) / chunks;
+                const long per =
+                    (tiles * ((n[0] + t.xchunk - 1) / t.xchunk) + 255) / 256;
+                const double resident =
+                    std::min<long>(per, std::max(1, hold / waves)) * waves;
+                const double cost = (double)(t.xchunk + 2 * R) * per * waves *
+                                    (1.0 + 0.12 * hm) *
+                                    (1.0 + 4.0 / resident);
+                if (cost < least) {
+                    least = cost;
+                    best = t;
+                }
+                if (per * waves > 4 * hold) break;
             }
         }
     }
-    if (!found) return false;
-    const int threads = (t.tz * t.ty + 63) / 64 * 64;
-    const long tiles = (long)((n[2] + t.tz - 1) / t.tz) *
-                       ((n[1] + t.ty - 1) / t.ty) * nin;
-    const long resident = 256L * std::max(1, 1024 / threads);
-    double least = 1e300;
-    for (int chunks = 1; chunks <= std::max(1, n[0] / 4); chunks++) {
-        const int xc = (n[0] + chunks - 1) / chunks;
-        const long blocks = tiles * ((n[0] + xc - 1) / xc);
-        const double rounds = blocks <= 8 * resident
-                                  ? (double)((blocks + resident - 1) / resident)
-                                  : (double)blocks / resident;
-        const double cost = rounds * (xc + 2 * R);
-        if (cost < least * 0.98) {
-            least = cost;
-            t.xchunk = xc;
-        }
-        if (blocks > 8 * resident) break;
-    }
-    return true;
+    return best;
 }
 
-bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], long nin,
-                   int epi)
+bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi)
 {
     if (d.R < 1 || d.R > MAXR_FAST ||
         (d.R > DM_RSKEW && (d.ni > 2 || d.nm > 0)))
@@ -158,21 +149,18 @@ bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], long nin,
     if (dtype == 3 ? (long)n[1] * n[2] * 16 >= (1L << 31)
                    : (long)n[1] * n[2] * es >= (1L << 31))
         return false;
-    if (!d.sym && epi != EPI_PLAIN) return false;
     if (epi == EPI_RELAX && (dtype == 1 || dtype == 3)) return false;
     if (epi == EPI_POT && dtype > 1) return false;
     if (epi == EPI_UPDW && dtype < 2) return false;
     if (epi == EPI_RESN && dtype != 0) return false;
-    DirTile t;
-    return dm_tile(d, n, nin, t);
+    return true;
 }
 
 long dirmarch_max_blocks(const DirStencil& d, int dtype, const int n[3],
                          long nin)
 {
-    (void)dtype;
-    DirTile t;
-    if (d.R < 1 || !dm_tile(d, n, nin, t)) return 0;
+    if (d.R < 1) return 0;
+    const DirTile t = dm_tile(d, dtype, n, nin);
     return (long)ceil_div(n[2], t.tz) * ceil_div(n[1], t.ty) *
            ceil_div(n[0], t.xchunk) * nin;
 }
@@ -182,10 +170,14 @@ int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
                     int epi, const EpiArgs& ea, hipStream_t s,
                     int* nblocks_out)
 {
-    DirTile t;
-    if (!dm_tile(d, n, nin, t)) {
-        set_error("direction march: no tile fits this grid");
-        return ENOTSUP_;
+    DirTile t = dm_tile(d, dtype, n, nin);
+    if (!ea.partial) {
+        std::lock_guard<std::mutex> lk(g_dm_mu);
+        const DirTile& o = g_dm_tile;
+        const int threads = (o.tz * o.ty + 63) / 64 * 64;
+        if (g_dm_override && threads <= DM_THREADS &&
+            (o.tz + 2 * d.R) * (o.ty + 2 * d.R) <= 4 * threads)
+            t = o;
     }
     switch (dtype) {
     case 0: return dirmarch_f64(d, t, n, bc, in, out, nin, epi, ea, s, nblocks_out);

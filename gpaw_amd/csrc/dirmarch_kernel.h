@@ -18,9 +18,13 @@
 // All global traffic goes through per-plane buffer resources: zero
 // boundaries and idle lanes are out-of-range offsets, not branches.
 //
-// What bounds it: the loads and stores where the batch fills the chip; LDS
-// reads for the skew-cell stencils (18 of 16 bytes per complex point of the
-// 25-point hexagonal Laplacian).
+// What bounds it: loads and stores for complex data (48 c128 grids of 128^3,
+// H psi - eps psi: 702 us, 4.6 TB/s; k_xrow 1006 us at 2 waves per SIMD);
+// for real data the instruction stream of one point per thread and plane
+// (40 f64 grids of 87x103x95: H psi 175 us, 3.1 TB/s; one point per thread
+// with every index wrapped took 790 us); for the skew stencils the LDS
+// reads (18 of 16 bytes per complex point of the 25-point hexagonal
+// Laplacian: 24 grids of 60x60x84 65 us; wrapped point by point 247 us).
 #pragma once
 
 #include "dirmarch.h"
@@ -32,7 +36,6 @@
 namespace gfd {
 
 constexpr int DM_NT = 512;  // most threads of a block
-constexpr int DM_HM = 4;    // staged elements per thread
 
 template <typename T>
 struct DmArgs {
@@ -41,8 +44,7 @@ struct DmArgs {
     const void* aux;
     int n0, n1, n2;
     int tz, ty, tiles_z, tiles_y, chunks_x, xchunk, nblocks;
-    int hm;              // staged elements per thread, at most DM_HM
-    int epi, nt;
+    int epi;
     double c0, w, s;
     int negate;
     DirStencil st;
@@ -52,29 +54,14 @@ struct DmArgs {
 };
 
 template <typename T>
-__device__ inline void dm_store(T v, __amdgpu_buffer_rsrc_t r, unsigned off,
-                                bool nt)
+__device__ inline void dm_store(T v, __amdgpu_buffer_rsrc_t r, unsigned off)
 {
-    typedef unsigned u2 __attribute__((ext_vector_type(2)));
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    if constexpr (sizeof(T) == 4) {
-        __builtin_amdgcn_raw_buffer_store_b32(
-            __builtin_bit_cast(unsigned, v), r, (int)off, 0, 0);
-    } else if constexpr (sizeof(T) == 8) {
-        if (nt)
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v),
-                                                  r, (int)off, 0, 2);
-        else
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v),
-                                                  r, (int)off, 0, 0);
-    } else {
-        if (nt)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v),
-                                                   r, (int)off, 0, 2);
-        else
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v),
-                                                   r, (int)off, 0, 0);
-    }
+    if constexpr (sizeof(T) <= 8)
+        bstore(v, r, off);
+    else
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r,
+                                               (int)off, 0, 0);
 }
 
 __device__ inline float dm_narrow(double v) { return (float)v; }
@@ -86,10 +73,16 @@ __device__ inline float2 dm_narrow(double2 v)
 // what an epilogue reads beside the stencil input
 enum DmAux : int { DM_NONE = 0, DM_SAME = 1, DM_POT = 2, DM_WIDE = 3 };
 
-// AUX: DmAux.  NARROW: FP64 input, result stored as FP32 (EPI_RESN).
-// SYM: equal coefficients on both sides of the centre (one copy of them:
-// the scalar registers hold all of a Laplacian's then).
-template <typename T, int R, int NI, int NM, int AUX, bool SYM, bool NARROW>
+// AUX: DmAux.  HM: staged elements per thread.  NARROW: FP64 input, result
+// stored as FP32 (EPI_RESN).
+// FULL: every direction of the form is there with equal coefficients on
+// both sides of the centre (a Laplacian).  Then nothing is tested in the
+// plane loop, whose many scalar tests and branches were what bound the
+// first version (142 scalar instructions, 20 of them branches, beside 38
+// vector ones per plane), and one copy of the coefficients stays in scalar
+// registers.
+template <typename T, int R, int NI, int NM, int AUX, int HM, bool FULL,
+          bool NARROW>
 __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
 {
     typedef typename ScalarOf<T>::type S;
@@ -97,6 +90,9 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     typedef typename std::conditional<
         AUX == DM_POT, double,
         typename std::conditional<AUX == DM_WIDE, WT, T>::type>::type TA;
+    typedef typename std::conditional<
+        NARROW, float,
+        typename std::conditional<AUX == DM_WIDE, WT, T>::type>::type TO;
     constexpr int U = 2 * R + 1;
     constexpr bool CPLX = IsCplx<T>::value;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -113,21 +109,21 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
 
     const int tid = threadIdx.x, NT = blockDim.x;
     const int n0 = a.n0, n1 = a.n1, n2 = a.n2;
-    const long plane = (long)n1 * n2, ng = plane * n0;
+    const long ng = (long)n1 * n2 * n0;
+    const unsigned plane = (unsigned)n1 * (unsigned)n2;
     const int z0 = zt * a.tz, y0 = yt * a.ty;
     const int xs = cx * a.xchunk, xe = min(xs + a.xchunk, n0);
     const int LW = a.tz + 2 * R, LSZ = (a.ty + 2 * R) * LW;
-    const T* __restrict__ gin = a.in + b * ng;
-    const unsigned pbytes = (unsigned)(plane * (long)sizeof(T));
+    const int buf1 = HM * NT;  // elements of one buffer (LSZ at most)
     const BC& bc = a.bc;
 
     // staged elements tid + m NT of the extended tile: offset in the plane
     // (BXM_OOB: zero or unused) and Bloch factor of the y and z wraps
-    unsigned hoff[DM_HM];
-    bool hph[DM_HM];
-    double2 hf[DM_HM];
+    unsigned hoff[HM];
+    bool hph[HM];
+    double2 hf[HM];
 #pragma unroll
-    for (int m = 0; m < DM_HM; m++) {
+    for (int m = 0; m < HM; m++) {
         const int e = tid + m * NT;
         hoff[m] = BXM_OOB;
         hph[m] = false;
@@ -148,39 +144,47 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     const int tr = tid / a.tz, tc = tid - tr * a.tz;
     const bool on = tr < a.ty && y0 + tr < n1 && z0 + tc < n2;
     const int lown = (min(tr, a.ty - 1) + R) * LW + tc + R;
-    const unsigned oidx = on ? (unsigned)((y0 + tr) * n2 + z0 + tc) : BXM_OOB;
-    auto bytes_at = [&](unsigned es) { return on ? oidx * es : BXM_OOB; };
+    const unsigned oidx = (unsigned)((y0 + tr) * n2 + z0 + tc);
+    const unsigned ooff = on ? oidx * (unsigned)sizeof(TO) : BXM_OOB;
+    const unsigned aoff = on ? oidx * (unsigned)sizeof(TA) : BXM_OOB;
 
-    // input plane of step x (wrapped; empty beyond a zero boundary)
-    auto in_plane = [&](int x, double2& f, bool& ph) {
-        ph = false;
-        f = make_double2(1.0, 0.0);
-        const bool ok = wrap_full(x, n0, bc.periodic[0], bc.phase[0][0],
-                                  bc.phase[0][1], f, ph);
-        return brsrc(gin + (long)(ok ? x : 0) * plane, ok ? pbytes : 0u);
+    // resource of plane x of an array of E (empty unless ok)
+    auto plane_at = [&](const void* base, int x, unsigned es, bool ok) {
+        const unsigned pb = plane * es;
+        return brsrc((const char*)base + (unsigned long)pb * (unsigned)x,
+                     ok ? pb : 0u);
     };
-    T hv[DM_HM];
-    double2 fx;
-    bool phx;
+    const void* gin = a.in + b * ng;
+    const void* gaux = (const TA*)a.aux + (AUX == DM_POT ? 0 : b * ng);
+    void* gout = (TO*)a.out + b * ng;
+    T hv[HM];
+    double2 fx = make_double2(1.0, 0.0);
+    bool phx = false;
+    // input plane x in [-R, n0 + R): wrapped at most once (n0 >= R), empty
+    // beyond a zero boundary
     auto ld_plane = [&](int x) {
-        const __amdgpu_buffer_rsrc_t r = in_plane(x, fx, phx);
+        const bool lo = x < 0, hi = x >= n0;
+        const int xw = lo ? x + n0 : hi ? x - n0 : x;
+        const __amdgpu_buffer_rsrc_t r =
+            plane_at(gin, xw, sizeof(T), !(lo || hi) || bc.periodic[0]);
+        if constexpr (CPLX) {
+            phx = lo || hi;
+            fx = lo ? bc.phase[0][1] : bc.phase[0][0];
+        }
 #pragma unroll
-        for (int m = 0; m < DM_HM; m++)
-            if (m < a.hm) hv[m] = bload<T>(r, hoff[m]);
+        for (int m = 0; m < HM; m++) hv[m] = bload<T>(r, hoff[m]);
     };
     TA av{};
-    // auxiliary operand of output plane x
+    // auxiliary operand of output plane x (the chunk's nearest plane before
+    // and after it: the array has no others)
     auto ld_aux = [&](int x) {
-        if constexpr (AUX != DM_NONE) {
-            const bool ok = x >= xs && x < xe;
-            const TA* p = (const TA*)a.aux + (AUX == DM_POT ? 0 : b * ng) +
-                          (long)(ok ? x : xs) * plane;
-            av = bload<TA>(brsrc(p, (unsigned)(plane * (long)sizeof(TA))),
-                           bytes_at(sizeof(TA)));
-        }
+        if constexpr (AUX != DM_NONE)
+            av = bload<TA>(plane_at(gaux, min(max(x, xs), xe - 1),
+                                    sizeof(TA), true),
+                           aoff);
     };
     auto cm = [](const DirLine& l, int k) {
-        return (S)(SYM ? l.p[k - 1] : l.m[k - 1]);
+        return (S)(FULL ? l.p[k - 1] : l.m[k - 1]);
     };
     S shift = (S)0;
     if constexpr (AUX == DM_POT)
@@ -195,28 +199,25 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     double nrm = 0.0;
 
     ld_plane(xs - R);
-    int par = 0;
+    ld_aux(xs);
+    int cur = 0;
     for (int xb = xs - R; xb < xe + R; xb += U) {
         cfor<U>([&](auto uc) {
             constexpr int u = uc;
             const int x = xb + u;
             if (x >= xe + R) return;
-            T* buf = lds + par * LSZ;
-            par ^= 1;
+            T* buf = lds + cur;
+            cur = buf1 - cur;
 #pragma unroll
-            for (int m = 0; m < DM_HM; m++)
-                if (m < a.hm) {
-                    T v = hv[m];
-                    if constexpr (CPLX) {
-                        if (hph[m]) v = scale_by<T>(v, hf[m], true);
-                        if (phx) v = scale_by<T>(v, fx, true);
-                    }
-                    const int e = tid + m * NT;
-                    if (e < LSZ) buf[e] = v;
+            for (int m = 0; m < HM; m++) {
+                T v = hv[m];
+                if constexpr (CPLX) {
+                    if (hph[m]) v = scale_by<T>(v, hf[m], true);
+                    if (phx) v = scale_by<T>(v, fx, true);
                 }
-            const TA a0 = av;
+                buf[tid + m * NT] = v;
+            }
             ld_plane(min(x + 1, xe + R - 1));
-            ld_aux(x + 1 - R);
             __syncthreads();
 
             // accumulator of output plane x + j: (u + R + j) mod U
@@ -233,7 +234,7 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
             T mid = at(here);
             // (a direction without points is skipped, not multiplied by
             // zeros: its neighbours may hold infinities)
-            if (a.st.in[0].on) {
+            if (FULL || a.st.in[0].on) {
 #pragma unroll
                 for (int k = 1; k <= R; k++) {
                     mid = fmac(mid, (S)a.st.in[0].p[k - 1], p[k]);
@@ -242,7 +243,7 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
             }
 #pragma unroll
             for (int i = 1; i < NI; i++) {
-                if (!a.st.in[i].on) continue;
+                if (!FULL && !a.st.in[i].on) continue;
                 const int o = i == 1 ? LW
                                      : a.st.in[i].dy * LW + a.st.in[i].dz;
 #pragma unroll
@@ -253,7 +254,7 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
             }
             at(here) = mid;
             // the point k steps ahead of output x - k, behind output x + k
-            if (a.st.x.on)
+            if (FULL || a.st.x.on)
                 cfor<R>([&](auto k0) {
                     constexpr int k = k0 + 1;
                     std::integral_constant<int, -k> ahead;
@@ -263,7 +264,7 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
                 });
 #pragma unroll
             for (int i = 0; i < NM; i++) {
-                if (!a.st.mix[i].on) continue;
+                if (!FULL && !a.st.mix[i].on) continue;
                 const int o = a.st.mix[i].dy * LW + a.st.mix[i].dz;
                 cfor<R>([&](auto k0) {
                     constexpr int k = k0 + 1;
@@ -275,55 +276,45 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
                                       p[-k * o]);
                 });
             }
-            // output plane x - R is complete
+            // output plane x - R is complete (before the chunk: not stored)
             const int xo = x - R;
-            if (xo >= xs) {
-                T r = at(oldest);
-                const T vo = vq[0];
-                if constexpr (AUX == DM_POT) {
-                    r = fmac(fmac(r, (S)a.c0, vo), (S)a0, vo);
-                    if (a.shift) r = fmac(r, shift, vo);
-                } else if constexpr (AUX == DM_NONE) {
-                    r = fmac(r, (S)a.c0, vo);
-                } else {
-                    T ax;
-                    if constexpr (AUX == DM_WIDE) ax = dm_narrow(a0);
-                    else ax = a0;
-                    if (a.epi == EPI_RELAX)
-                        r = epi_apply<T, EPI_RELAX>(r, vo, ax, a.c0, a.w, a.s,
-                                                    a.negate, nrm);
-                    else if (a.epi == EPI_RESID) {
-                        r = fmac(r, (S)a.c0, vo) - ax;
-                        if (on) nrm += sq(r);
-                    } else
-                        r = epi_apply<T, EPI_UPDATE>(r, vo, ax, a.c0, a.w,
-                                                     a.s, a.negate, nrm);
-                }
-                if constexpr (NARROW) {
-                    const __amdgpu_buffer_rsrc_t ro =
-                        brsrc((float*)a.out + b * ng + (long)xo * plane,
-                              (unsigned)(plane * 4));
-                    dm_store((float)r, ro, bytes_at(4), false);
-                } else if constexpr (AUX == DM_WIDE) {
-                    const __amdgpu_buffer_rsrc_t ro = brsrc(
-                        (WT*)a.out + b * ng + (long)xo * plane,
-                        (unsigned)(plane * (long)sizeof(WT)));
-                    dm_store(to_wide(r), ro, bytes_at(sizeof(WT)),
-                             a.nt != 0);
-                } else {
-                    const __amdgpu_buffer_rsrc_t ro =
-                        brsrc((T*)a.out + b * ng + (long)xo * plane, pbytes);
-                    dm_store(r, ro, bytes_at(sizeof(T)), a.nt != 0);
-                }
+            T r = at(oldest);
+            const T vo = vq[0];
+            if constexpr (AUX == DM_POT) {
+                r = fmac(fmac(r, (S)a.c0, vo), (S)av, vo);
+                if (a.shift) r = fmac(r, shift, vo);
+            } else if constexpr (AUX == DM_NONE) {
+                r = fmac(r, (S)a.c0, vo);
+            } else {
+                T ax;
+                if constexpr (AUX == DM_WIDE) ax = dm_narrow(av);
+                else ax = av;
+                if (a.epi == EPI_RELAX)
+                    r = epi_apply<T, EPI_RELAX>(r, vo, ax, a.c0, a.w, a.s,
+                                                a.negate, nrm);
+                else if (a.epi == EPI_RESID) {
+                    r = fmac(r, (S)a.c0, vo) - ax;
+                    if (on && xo >= xs) nrm += sq(r);
+                } else
+                    r = epi_apply<T, EPI_UPDATE>(r, vo, ax, a.c0, a.w, a.s,
+                                                 a.negate, nrm);
             }
+            TO ro;
+            if constexpr (NARROW) ro = (float)r;
+            else if constexpr (AUX == DM_WIDE) ro = to_wide(r);
+            else ro = r;
+            dm_store(ro, plane_at(gout, xo, sizeof(TO), xo >= xs), ooff);
             at(oldest) = zero_of<T>();
+            // reloaded once used: a copy of a value in flight would wait
+            ld_aux(xo + 1);
         });
     }
-    if (a.partial) block_sum_store(nrm, a.partial, L);
+    if constexpr (AUX == DM_SAME)
+        if (a.partial) block_sum_store(nrm, a.partial, L);
 }
 
-template <typename T, int R, int NI, int NM, int AUX, bool SYM = true,
-          bool NARROW = false>
+template <typename T, int R, int NI, int NM, int AUX, int HM, bool FULL,
+          bool NARROW>
 static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
                        int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
@@ -345,15 +336,12 @@ static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
     const int threads = (t.tz * t.ty + 63) / 64 * 64;
     const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
     if (nb <= 0) return OK;
-    if (nb > 0x7fffffffL || threads > DM_NT ||
-        lsz > (long)DM_HM * threads) {
+    if (nb > 0x7fffffffL || threads > DM_NT || lsz > (long)HM * threads) {
         set_error("direction march: %ld blocks of %d x %d do not fit", nb,
                   t.ty, t.tz);
         return ENOTSUP_;
     }
     a.nblocks = (int)nb;
-    a.hm = ceil_div(lsz, threads);
-    a.nt = xr_nt_flags((long)n[0] * n[1] * n[2] * nin * (long)sizeof(T)) & 1;
     a.epi = epi == EPI_RESN ? (int)EPI_RESID : epi;
     a.c0 = ea.c0;
     a.w = ea.w;
@@ -364,39 +352,51 @@ static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
     a.partial = epi == EPI_RESID || epi == EPI_RESN ? ea.partial : nullptr;
     a.shift = ea.shift;
     (void)hipGetLastError();
-    hipLaunchKernelGGL((k_dirmarch<T, R, NI, NM, AUX, SYM, NARROW>),
+    hipLaunchKernelGGL((k_dirmarch<T, R, NI, NM, AUX, HM, FULL, NARROW>),
                        dim3((unsigned)nb), dim3(threads),
-                       2 * lsz * sizeof(T), s, a);
+                       2 * (size_t)HM * threads * sizeof(T), s, a);
     GFD_LAUNCH_CHECK();
     if (nbo) *nbo = (int)nb;
     return OK;
 }
 
-template <typename T, int R, int NI, int NM>
+template <typename T, int R, int NI, int NM, int AUX, bool FULL, bool NARROW>
+static int dm_launch_h(const DirStencil& d, const DirTile& t, const int n[3],
+                       const BC& bc, const void* in, void* out, long nin,
+                       int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
+{
+    const int threads = (t.tz * t.ty + 63) / 64 * 64;
+    const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
+    if (FULL && lsz <= 2L * threads)
+        return dm_launch_t<T, R, NI, NM, AUX, 2, FULL, NARROW>(
+            d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+    return dm_launch_t<T, R, NI, NM, AUX, 4, FULL, NARROW>(
+        d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+}
+
+template <typename T, int R, int NI, int NM, bool FULL>
 static int dm_launch_e(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
                        int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
 {
-#define GFD_DM(...)                                                         \
-    return dm_launch_t<T, R, NI, NM, __VA_ARGS__>(d, t, n, bc, in, out,     \
-                                                  nin, epi, ea, s, nbo)
+#define GFD_DM(AUX, NARROW)                                                 \
+    return dm_launch_h<T, R, NI, NM, AUX, FULL, NARROW>(                    \
+        d, t, n, bc, in, out, nin, epi, ea, s, nbo)
     switch (epi) {
-    case EPI_PLAIN:
-        if (!d.sym) GFD_DM(DM_NONE, false);
-        GFD_DM(DM_NONE);
+    case EPI_PLAIN: GFD_DM(DM_NONE, false);
     case EPI_RELAX:
     case EPI_RESID:
-    case EPI_UPDATE: GFD_DM(DM_SAME);
+    case EPI_UPDATE: GFD_DM(DM_SAME, false);
     case EPI_POT:
         if constexpr (sizeof(typename ScalarOf<T>::type) == 8)
-            GFD_DM(DM_POT);
+            GFD_DM(DM_POT, false);
         break;
     case EPI_UPDW:
         if constexpr (sizeof(typename ScalarOf<T>::type) == 4)
-            GFD_DM(DM_WIDE);
+            GFD_DM(DM_WIDE, false);
         break;
     case EPI_RESN:
-        if constexpr (std::is_same<T, double>::value) GFD_DM(DM_SAME, true, true);
+        if constexpr (std::is_same<T, double>::value) GFD_DM(DM_SAME, true);
         break;
     }
 #undef GFD_DM
@@ -409,20 +409,21 @@ static int dm_launch_r(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
                        int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
 {
-#define GFD_DM(NI, NM)                                                      \
-    if (d.ni <= NI && d.nm <= NM)                                           \
-        return dm_launch_e<T, R, NI, NM>(d, t, n, bc, in, out, nin, epi,    \
-                                         ea, s, nbo)
-    GFD_DM(2, 0);
-    if constexpr (R <= 3) {
-        GFD_DM(2, 1);
-        GFD_DM(3, 0);
-        GFD_DM(3, 2);
-        GFD_DM(3, 4);
+#define GFD_DM(NI, NM, FULL)                                                \
+    return dm_launch_e<T, R, NI, NM, FULL>(d, t, n, bc, in, out, nin, epi,  \
+                                           ea, s, nbo)
+    if (d.full) {
+        if (d.ni == 2 && d.nm == 0) GFD_DM(2, 0, true);
+        if constexpr (R <= DM_RSKEW) {
+            if (d.ni == 2 && d.nm == 1) GFD_DM(2, 1, true);
+            if (d.ni == 3 && d.nm == 0) GFD_DM(3, 0, true);
+            if (d.ni == 3 && d.nm == 2) GFD_DM(3, 2, true);
+        }
     }
+    // anything else: the general form of the directions
+    if constexpr (R <= DM_RSKEW) GFD_DM(3, 4, false);
+    else GFD_DM(2, 0, false);
 #undef GFD_DM
-    set_error("direction march: too many directions");
-    return ENOTSUP_;
 }
 
 template <typename T>

@@ -8,7 +8,7 @@
 
 namespace gfd {
 
-constexpr int MAXR_FAST = 4;   // largest radius of the x-marching kernel
+constexpr int MAXR_FAST = 4;   // largest radius of the x-marching kernels
 constexpr int MAXP = 256;      // largest number of stencil points
 
 // What the kernel does with acc = sum_{p != centre} c_p in(x + o_p) and the
@@ -54,7 +54,7 @@ struct GeneralStencil {
     const int* off;           // [P][3]
 };
 
-// Tile choice of the x-marching kernel (exposed for the autotuner).
+// Tile choice of the x-marching kernels (exposed for the autotuner).
 struct XmTile {
     int tz;      // tile width along z (threads per row)
     int nseg;    // row segments (threads along y)
@@ -66,12 +66,7 @@ struct XmTile {
     int wide = 0;   // k_xrow on 16-byte data: 2 = two points per thread
 };
 // Launch one stencil pass over `nin` grids of shape n[3].
-// dtype: 0 = f64, 1 = c128, 2 = f32, 3 = c64 (row kernel and general
-// kernel; the tiled x-march kernel takes 0-2).
-int launch_axis_stencil(const AxisStencil& st, int dtype, const int n[3],
-                        const BC& bc, const void* in, void* out, long nin,
-                        int epi, const EpiArgs& ea, hipStream_t stream,
-                        int* nblocks_out);
+// dtype: 0 = f64, 1 = c128, 2 = f32, 3 = c64.
 int launch_general_stencil(const GeneralStencil& st, int dtype,
                            const int n[3], const BC& bc, const void* in,
                            void* out, long nin, int epi, const EpiArgs& ea,
@@ -105,20 +100,11 @@ void xr_set_dma(bool on);
 void xr_set_nt(int flags);
 void xr_set_override(const XmTile* t);
 
-// Whether the x-marching kernel takes this stencil / grid (else general).
-bool axis_stencil_fits(const AxisStencil& st, int dtype, const int n[3],
-                       long nin);
-
 // Block-count upper bounds for the residual-norm partial buffer.
-long axis_stencil_max_blocks(const AxisStencil& st, int dtype, const int n[3],
-                             long nin);
 long general_stencil_max_blocks(const int n[3], long nin);
 
 // Deterministic final reduction of `np` partial sums into *result (device).
 int launch_sum_partials(const double* partial, long np, double* result,
                         hipStream_t stream);
-
-XmTile xm_default_tile(int R, int dtype, const int n[3], long nin);
-void xm_set_override(const XmTile* t);  // nullptr clears
 
 }  // namespace gfd

@@ -52,7 +52,7 @@ def test_laplace(cell, nn, N, pbc, dtype):
     ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
     out = dev(np.zeros_like(a))
     say('dirmarch laplace', cell, nn, N, pbc, dtype)
-    with path(4):
+    with path(2):
         op.apply(dev(a), out, ph)
     ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a,
                           ph)
@@ -72,7 +72,7 @@ def test_other_stencils(make):
     a = rand(rng, (2,) + tuple(gd.n_c))
     out = dev(np.zeros_like(a))
     say('dirmarch stencil', op.description)
-    with path(4):
+    with path(2):
         op.apply(dev(a), out)
     ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a)
     assert relerr(host(out), ref) < TOL
@@ -85,7 +85,7 @@ def test_infinities_stay_on_their_lines():
     a = np.ones((1, 8, 9, 12))
     a[0, 4, 4, :] = np.inf
     out = dev(np.zeros_like(a))
-    with path(4):
+    with path(2):
         op.apply(dev(a), out)
     bad = ~np.isfinite(host(out)[0])
     assert bad[4, 4].all() and bad.sum() == 12
@@ -103,7 +103,7 @@ def test_epilogues(cell, N, pbc):
     sp = spec(op)
     f, src = rand(rng, n), rand(rng, n)
     say('dirmarch epilogues', cell, N)
-    with path(4):
+    with path(2):
         for w in (2.0 / 3.0, 1.0):
             g = dev(f.copy())
             op.relax(2, g, dev(src), 3, w)
@@ -154,7 +154,7 @@ def test_preconditioner(cell, N, pbc, dtype, fp32):
     kpt = SimpleNamespace(phase_cd=ph)
     outs = []
     say('dirmarch preconditioner', cell, N, dtype, fp32)
-    for p in (4, 1):
+    for p in (2, 1):
         with path(p):
             outs.append(host(pc(res, kpt)))
     assert relerr(outs[0], outs[1]) < (2e-6 if fp32 else TOL)
