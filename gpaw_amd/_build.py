@@ -22,7 +22,7 @@ SOURCES = ['dirmarch_c128.hip', 'dirmarch_f64.hip', 'dirmarch_c64.hip',
            'stencil.hip', 'batch.hip', 'transfer.hip', 'api.hip',
            'stencil_rows.hip', 'vector.hip', 'bands.hip', 'coarse.hip',
            'fftpoisson.hip', 'wstencil.hip', 'gs.hip',
-           'xfer_march.hip', 'wxmarch.hip', 'bxmarch.hip', 'bxfer_march.hip',
+           'xfer_march.hip', 'wxmarch.hip', 'wdielectric.hip', 'bxmarch.hip', 'bxfer_march.hip',
            'precond_fine.hip']
 
 FLAGS = [

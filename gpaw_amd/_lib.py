@@ -95,6 +95,10 @@ SIGNATURES = {
     'gfd_h_residual': (_i, [_vp, _vp, _vp, _vp, _vp, _l, _dp, _vp]),
     'gfd_band_dots': (_i, [_i, _vp, _vp, _i, _l, _l, _d, _vp, _vp]),
     'gfd_rmm_lambda': (_i, [_i, _vp, _vp, _i, _l, _l, _vp, _vp]),
+    'gfd_band_dots_work': (_i, [_i, _vp, _vp, _i, _l, _l, _d, _vp, _vp, _l,
+                                _vp]),
+    'gfd_rmm_lambda_work': (_i, [_i, _vp, _vp, _i, _l, _l, _vp, _vp, _l,
+                                 _vp]),
     'gfd_band_update': (_i, [_i, _i, _vp, _d, _vp, _vp, _vp, _vp, _i, _l, _l,
                              _vp]),
     'gfd_h_apply': (_i, [_vp, _vp, _vp, _vp, _l, _dp, _vp]),

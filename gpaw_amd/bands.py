@@ -109,10 +109,19 @@ def band_dots(a, b, dv, out=None):
         _bands_vector(out, nb)
     if out is None:
         out = torch.empty(nb, dtype=torch.float64, device=a.device)
-    _lib.check(_lib.load().gfd_band_dots(
+    work = split_work(nb, a.device)
+    _lib.check(_lib.load().gfd_band_dots_work(
         int(a.dtype == torch.complex128), ptr(a), ptr(b), nb, npts, npts,
-        float(dv), ptr(out), stream_handle()), 'band_dots')
+        float(dv), ptr(out), ptr(work), work.numel(), stream_handle()),
+        'band_dots')
     return out
+
+
+def split_work(nb, device):
+    """Work space of the band sums (gfd_band_dots_work): from the caching
+    allocator on the current stream, so calls on several streams have one
+    each."""
+    return torch.empty(2 * (2048 + nb), dtype=torch.float64, device=device)
 
 
 def overlap(psi, dv, lower_only=True, out=None):

@@ -1676,7 +1676,35 @@ extern "C" int gfd_band_dots(int is_complex, const void* a, const void* b,
         return EINVAL_;
     }
     return band_dots(is_complex ? 1 : 0, a, b, nbands, npts, ld, dv, out,
-                     (hipStream_t)stream);
+                     nullptr, 0, (hipStream_t)stream);
+}
+
+extern "C" int gfd_band_dots_work(int is_complex, const void* a,
+                                  const void* b, int nbands, long npts,
+                                  long ld, double dv, double* out,
+                                  double* work, long nwork, void* stream)
+{
+    if (!a || !b || !out || nbands < 0 || npts < 0 || ld < npts ||
+        nwork < 0 || (nwork > 0 && !work)) {
+        set_error("gfd_band_dots_work: bad arguments");
+        return EINVAL_;
+    }
+    return band_dots(is_complex ? 1 : 0, a, b, nbands, npts, ld, dv, out,
+                     work, nwork, (hipStream_t)stream);
+}
+
+extern "C" int gfd_rmm_lambda_work(int is_complex, const void* dR,
+                                   const void* R, int nbands, long npts,
+                                   long ld, double* lam, double* work,
+                                   long nwork, void* stream)
+{
+    if (!dR || !R || !lam || nbands < 0 || npts < 0 || ld < npts ||
+        nwork < 0 || (nwork > 0 && !work)) {
+        set_error("gfd_rmm_lambda_work: bad arguments");
+        return EINVAL_;
+    }
+    return rmm_lambda(is_complex ? 1 : 0, dR, R, nbands, npts, ld, lam, work,
+                      nwork, (hipStream_t)stream);
 }
 
 extern "C" int gfd_rmm_lambda(int is_complex, const void* dR, const void* R,
@@ -1688,7 +1716,7 @@ extern "C" int gfd_rmm_lambda(int is_complex, const void* dR, const void* R,
         return EINVAL_;
     }
     return rmm_lambda(is_complex ? 1 : 0, dR, R, nbands, npts, ld, lam,
-                      (hipStream_t)stream);
+                      nullptr, 0, (hipStream_t)stream);
 }
 
 extern "C" int gfd_band_update(int is_complex, int mode, const double* alpha,

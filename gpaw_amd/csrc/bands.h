@@ -24,13 +24,17 @@ int gram(BandWork& w, const double2* A, long lda, const double2* B, long ldb,
          double2* out, long ldo, hipStream_t s);
 
 // out[n] = dv Re sum_x conj(A_n(x)) B_n(x), dtype 0 f64 / 1 c128, rows of
-// npts points at stride ld; out a device array of nbands doubles.
+// npts points at stride ld; out a device array of nbands doubles.  work:
+// nwork doubles of device memory (or null): with 2 (2048 + nbands) a band is
+// split over several blocks.
 int band_dots(int dtype, const void* A, const void* B, int nbands, long npts,
-              long ld, double dv, double* out, hipStream_t s);
+              long ld, double dv, double* out, double* work, long nwork,
+              hipStream_t s);
 
-// lam[n] = -Re<dR_n|R_n> / <dR_n|dR_n> (0 where dR_n = 0)
+// lam[n] = -Re<dR_n|R_n> / <dR_n|dR_n> (0 where dR_n = 0); work as above
 int rmm_lambda(int dtype, const void* dR, const void* R, int nbands,
-               long npts, long ld, double* lam, hipStream_t s);
+               long npts, long ld, double* lam, double* work, long nwork,
+               hipStream_t s);
 
 // c_n = scale alpha[n]; mode 0: y_n += c_n x_n; mode 1 also
 // w_n <- v_n + c_n w_n in the same pass.

@@ -428,22 +428,6 @@ k_band_dot(const T* __restrict__ A, const T* __restrict__ B, long npts,
     if (threadIdx.x == 0) out[blockIdx.x] = dv * red[0];
 }
 
-int band_dots(int dtype, const void* A, const void* B, int nbands, long npts,
-              long ld, double dv, double* out, hipStream_t s)
-{
-    if (nbands <= 0) return OK;
-    if (dtype == 1)
-        hipLaunchKernelGGL(k_band_dot<double2>, dim3(nbands), dim3(1024), 0,
-                           s, (const double2*)A, (const double2*)B, npts, ld,
-                           dv, out);
-    else
-        hipLaunchKernelGGL(k_band_dot<double>, dim3(nbands), dim3(1024), 0,
-                           s, (const double*)A, (const double*)B, npts, ld,
-                           dv, out);
-    GFD_LAUNCH_CHECK();
-    return OK;
-}
-
 // Two real parts of band inner products at once: s0 = Re sum conj(a) b,
 // s1 = Re sum conj(a) a.
 template <typename T>
@@ -488,10 +472,101 @@ k_rmm_lambda(const T* __restrict__ dR, const T* __restrict__ R, long npts,
         lam[blockIdx.x] = r1[0] > 0.0 ? -r0[0] / r1[0] : 0.0;
 }
 
+// Band sums with a few bands: a band split over `chunks` blocks, whose
+// partial sums (two per block, in `work`) a second launch adds in a fixed
+// order.  One block per band leaves most CUs idle below a few hundred bands
+// (40 f64 bands of 87x103x95: lambda 440 us with one block each, SPLIT_US
+// split).  LAMBDA: both sums of the step length, else Re <a|b> only.
+constexpr int SPLIT_NT = 256;
+
+template <typename T, bool LAMBDA>
+__global__ void __launch_bounds__(SPLIT_NT)
+k_band_split(const T* __restrict__ A, const T* __restrict__ B, long npts,
+             long ld, long per, double* __restrict__ work)
+{
+    const T* a = A + (long)blockIdx.y * ld;
+    const T* b = B + (long)blockIdx.y * ld;
+    const long x1 = min((long)(blockIdx.x + 1) * per, npts);
+    double s0 = 0.0, s1 = 0.0;
+    for (long x = (long)blockIdx.x * per + threadIdx.x; x < x1;
+         x += SPLIT_NT)
+        dot2(a, b, x, s0, s1);
+    for (int o = 32; o > 0; o >>= 1) {
+        s0 += __shfl_down(s0, o, 64);
+        s1 += __shfl_down(s1, o, 64);
+    }
+    __shared__ double r[2][SPLIT_NT / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0) {
+        r[0][w] = s0;
+        r[1][w] = s1;
+    }
+    __syncthreads();
+    if (threadIdx.x < (LAMBDA ? 2 : 1)) {
+        double s = 0.0;
+        for (int i = 0; i < SPLIT_NT / 64; i++) s += r[threadIdx.x][i];
+        work[2 * ((long)blockIdx.y * gridDim.x + blockIdx.x) + threadIdx.x] =
+            s;
+    }
+}
+
+template <bool LAMBDA>
+__global__ void __launch_bounds__(64)
+k_band_join(const double* __restrict__ work, int chunks, double dv,
+            double* __restrict__ out)
+{
+    const double* p = work + 2 * (long)blockIdx.x * chunks;
+    double s0 = 0.0, s1 = 0.0;
+    for (int c = threadIdx.x; c < chunks; c += 64) {
+        s0 += p[2 * c];
+        if (LAMBDA) s1 += p[2 * c + 1];
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        s0 += __shfl_down(s0, o, 64);
+        if (LAMBDA) s1 += __shfl_down(s1, o, 64);
+    }
+    if (threadIdx.x == 0)
+        out[blockIdx.x] = LAMBDA ? (s1 > 0.0 ? -s0 / s1 : 0.0) : dv * s0;
+}
+
+// Blocks per band: about 2048 in all, at least 4096 points each (1: not
+// split, and no work space needed).
+static int band_chunks(int nbands, long npts, long nwork)
+{
+    long c = std::min((2048L + nbands - 1) / nbands, npts / 4096);
+    c = std::min(c, nwork / (2L * nbands));
+    return nbands > 65535 || c < 2 ? 1 : (int)c;
+}
+
+template <typename T, bool LAMBDA>
+static int band_split(const void* A, const void* B, int nbands, long npts,
+                      long ld, double dv, double* work, int chunks,
+                      double* out, hipStream_t s)
+{
+    const long per = (npts + chunks - 1) / chunks;
+    hipLaunchKernelGGL((k_band_split<T, LAMBDA>),
+                       dim3((unsigned)chunks, (unsigned)nbands),
+                       dim3(SPLIT_NT), 0, s, (const T*)A, (const T*)B, npts,
+                       ld, per, work);
+    GFD_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_band_join<LAMBDA>, dim3((unsigned)nbands), dim3(64),
+                       0, s, work, chunks, dv, out);
+    GFD_LAUNCH_CHECK();
+    return OK;
+}
+
 int rmm_lambda(int dtype, const void* dR, const void* R, int nbands,
-               long npts, long ld, double* lam, hipStream_t s)
+               long npts, long ld, double* lam, double* work, long nwork,
+               hipStream_t s)
 {
     if (nbands <= 0) return OK;
+    const int chunks = band_chunks(nbands, npts, work ? nwork : 0);
+    if (chunks > 1)
+        return dtype == 1
+                   ? band_split<double2, true>(dR, R, nbands, npts, ld, 0.0,
+                                               work, chunks, lam, s)
+                   : band_split<double, true>(dR, R, nbands, npts, ld, 0.0,
+                                              work, chunks, lam, s);
     if (dtype == 1)
         hipLaunchKernelGGL(k_rmm_lambda<double2>, dim3(nbands), dim3(1024),
                            0, s, (const double2*)dR, (const double2*)R, npts,
@@ -500,6 +575,30 @@ int rmm_lambda(int dtype, const void* dR, const void* R, int nbands,
         hipLaunchKernelGGL(k_rmm_lambda<double>, dim3(nbands), dim3(1024),
                            0, s, (const double*)dR, (const double*)R, npts,
                            ld, lam);
+    GFD_LAUNCH_CHECK();
+    return OK;
+}
+
+int band_dots(int dtype, const void* A, const void* B, int nbands, long npts,
+              long ld, double dv, double* out, double* work, long nwork,
+              hipStream_t s)
+{
+    if (nbands <= 0) return OK;
+    const int chunks = band_chunks(nbands, npts, work ? nwork : 0);
+    if (chunks > 1)
+        return dtype == 1
+                   ? band_split<double2, false>(A, B, nbands, npts, ld, dv,
+                                                work, chunks, out, s)
+                   : band_split<double, false>(A, B, nbands, npts, ld, dv,
+                                               work, chunks, out, s);
+    if (dtype == 1)
+        hipLaunchKernelGGL(k_band_dot<double2>, dim3(nbands), dim3(1024), 0,
+                           s, (const double2*)A, (const double2*)B, npts, ld,
+                           dv, out);
+    else
+        hipLaunchKernelGGL(k_band_dot<double>, dim3(nbands), dim3(1024), 0,
+                           s, (const double*)A, (const double*)B, npts, ld,
+                           dv, out);
     GFD_LAUNCH_CHECK();
     return OK;
 }

@@ -27,7 +27,13 @@ struct WAxis {
 int launch_wxmarch(const WAxis& st, int real, const int n[3], const BC& bc,
                    const void* in, void* out, const double* src, long nin,
                    double w, bool relax, hipStream_t s);
-// Route weighted operators through the fast kernel (default on).
+// The same for the dielectric operator (a Laplacian-like symmetric stencil,
+// then an antisymmetric one per axis); ENOTSUP_ for any other.
+int launch_wdielectric(const WAxis& st, int real, const int n[3],
+                       const BC& bc, const void* in, void* out,
+                       const double* src, long nin, double w, bool relax,
+                       hipStream_t s);
+// Route weighted operators through the fast kernels (default on).
 void wx_set_enabled(bool on);
 // Tile overrides of the weighted x-march kernel (0: automatic): rows per
 // thread (1, 2, 4) and x planes per block.

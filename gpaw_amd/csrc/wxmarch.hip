@@ -424,6 +424,11 @@ int launch_wxmarch(const WAxis& st, int real, const int n[3], const BC& bc,
         set_error("weighted x-march: not for this operator");
         return ENOTSUP_;
     }
+    if (g_wx_py == 0 && g_wx_xchunk == 0) {
+        const int e = launch_wdielectric(st, real, n, bc, in, out, src, nin,
+                                         w, relax, s);
+        if (e != ENOTSUP_) return e;
+    }
     XmTile tl;
     if (!wx_tile(st.R, real ? 8 : 16, n, nin, tl)) {
         set_error("weighted x-march: no tile fits this grid");

@@ -20,7 +20,7 @@ import numpy as np
 
 from . import _lib
 from .arrays import ptr, stream_handle, torch
-from .bands import apply_hamiltonian
+from .bands import apply_hamiltonian, split_work
 
 
 def _check(psi, *others):
@@ -40,9 +40,10 @@ def rmm_lambda(dR, R, out=None):
     npts = int(np.prod(dR.shape[1:]))
     if out is None:
         out = torch.empty(nb, dtype=torch.float64, device=dR.device)
-    _lib.check(_lib.load().gfd_rmm_lambda(
+    work = split_work(nb, dR.device)
+    _lib.check(_lib.load().gfd_rmm_lambda_work(
         int(dR.is_complex()), ptr(dR), ptr(R), nb, npts, npts, ptr(out),
-        stream_handle()), 'rmm_lambda')
+        ptr(work), work.numel(), stream_handle()), 'rmm_lambda')
     return out
 
 

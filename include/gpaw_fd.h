@@ -334,6 +334,18 @@ int gfd_band_dots(int is_complex, const void* a, const void* b, int nbands,
 int gfd_rmm_lambda(int is_complex, const void* dR, const void* R, int nbands,
                    long npts, long ld, double* lam, void* stream);
 
+/* gfd_band_dots and gfd_rmm_lambda with nwork doubles of device memory as
+ * work space (not shared by calls that overlap in time): from
+ * 2 (2048 + nbands) on, a band's sum is split over several blocks when
+ * there are too few bands to fill the GPU.  The order of the sum is fixed
+ * by nbands, npts and nwork. */
+int gfd_band_dots_work(int is_complex, const void* a, const void* b,
+                       int nbands, long npts, long ld, double dv, double* out,
+                       double* work, long nwork, void* stream);
+int gfd_rmm_lambda_work(int is_complex, const void* dR, const void* R,
+                        int nbands, long npts, long ld, double* lam,
+                        double* work, long nwork, void* stream);
+
 /* Per-band updates with c_n = scale * alpha[n] (alpha: device array):
  * mode 0: y_n += c_n x_n (rmmdiis.py:252-257, the final preconditioned
  * step); mode 1: y_n += c_n x_n and w_n <- v_n + c_n w_n in one pass
