@@ -20,6 +20,7 @@
 #include "bands.h"
 #include "handles.h"
 #include "coarse.h"
+#include "tsmooth.h"
 #include "gs.h"
 #include "wstencil.h"
 #include "precond_fine.h"
@@ -868,16 +869,23 @@ struct CoarseSolve {
     bool one = false; // k_coarse1 (else k_coarse)
     CGrid host{};
     DevBuf dev;
+    // levels between the finest and lc whose half cycles are one launch each
+    // (tsmooth.hip): table on host and device, tiles per level (0: not)
+    std::vector<TsGrid> ts;
+    std::vector<int> tstiles;
+    DevBuf tsdev;
 };
 
 // LDS-resident coarse solve on (default) / off, and the largest first
 // level (points) it takes (0: the defaults below)
 static bool g_coarse_lds = true;
 static long g_coarse_max_pts = 0;
-// one workgroup against a launch per sweep: the general kernel up to 16^3
-// points, nearest-neighbour levels up to 24^3 where they fit (192^3 mixed
-// solve: 5.62 ms with the FP32 24^3 level in the workgroup, 5.74 from 12^3
-// down; FP64 40^3 box, 19^3 level: 2.83 against 3.55 ms)
+// One workgroup against launches per level: from 16^3 points down where the
+// level above can run in blocked half cycles (192^3 mixed solve: 4.52 ms,
+// with the FP32 24^3 level in the workgroup 4.86, from 6^3 down 4.60; 40^3
+// FP64 box, 19^3 level: 1.23 against 1.43 ms).  Without those (more than
+// TS_MAXS sweeps) the nearest-neighbour form beats a launch per sweep up to
+// 24^3 where it fits, the general kernel up to 16^3.
 constexpr long COARSE_PTS = 4096, COARSE1_PTS = 14000;
 
 struct gfd_poisson {
@@ -1025,6 +1033,10 @@ extern "C" void gfd_poisson_free(gfd_poisson* p)
     p->lv.pool.release();
     p->lv32.pool.release();
     p->lv64r.pool.release();
+    for (CoarseSolve* c : {&p->cs64, &p->cs32, &p->cs64r}) {
+        c->dev.release();
+        c->tsdev.release();
+    }
     p->scalar.release();
     p->partial.release();
     p->xscratch.release();
@@ -1158,6 +1170,42 @@ static bool coarse_layout(gfd_poisson* p, const Schedule& sc, int dtype,
     return true;
 }
 
+// Level l's entry of the blocked-smoothing table (tsmooth.hip) and its tiles;
+// 0 for a level that keeps its separate launches.
+static int ts_level(gfd_poisson* p, const Schedule& sc, int dtype, int l,
+                    TsGrid& g)
+{
+    g = TsGrid{};
+    if (l < 1 || l >= sc.coarsest || !ts_enabled() ||
+        (dtype == 0 && p->method == 1))
+        return 0;
+    const gfd_operator* op = p->ops[l];
+    const AxisStencil& ax = op->ax;
+    const XferPlan& r = p->rst[l]->plan;
+    const XferPlan& i = p->itp[l]->plan;
+    const int pre = sched_pre(sc, l), post = sched_post(sc, l);
+    if (!op->axis_ok || !op->real || ax.R != 1 || !ax.has[0] || !ax.has[1] ||
+        !ax.has[2] || r.K != 2 || i.K != 2 || pre < 1 || pre > TS_MAXS ||
+        post < 1 || post > TS_MAXS || op->ng() > TS_PTS)
+        return 0;
+    TsGrid t{};
+    for (int d = 0; d < 3; d++) {
+        t.n[d] = op->n[d];
+        t.nc[d] = p->ops[l + 1]->n[d];
+        t.periodic[d] = op->periodic[d];
+        t.roff[d] = r.ax[d].off;
+        t.ioff[d] = i.ax[d].off;
+        t.iskip0[d] = i.ax[d].skip0;
+        t.cp[d] = ax.cp[d][0];
+        t.cm[d] = ax.cm[d][0];
+        if (t.roff[d] != 0 && t.roff[d] != 1) return 0;
+    }
+    t.c0 = centre_coef(op);
+    t.w = sched_w(sc, l);
+    g = t;
+    return ts_tiles(g);
+}
+
 // Plan the LDS-resident solve of levels [lc, coarsest] for a schedule: the
 // first lc >= 1 that one workgroup holds and solves faster than launches of
 // its own would.  *changed reports a new plan (graphs that captured the old
@@ -1178,9 +1226,11 @@ static int plan_coarse(gfd_poisson* p, const Schedule& sc, int dtype,
     for (int l0 = 1; lds_ok && lc < 0 && l0 <= sc.coarsest; l0++) {
         if (!coarse_layout(p, sc, dtype, l0, cheb, g, bytes)) continue;
         one = coarse_plan1(&g, 1, dtype);
+        TsGrid t;
         const long most = g_coarse_max_pts ? g_coarse_max_pts
-                          : one            ? COARSE1_PTS
-                                           : COARSE_PTS;
+                          : one && !ts_level(p, sc, dtype, l0, t)
+                              ? COARSE1_PTS
+                              : COARSE_PTS;
         if (p->ops[l0]->ng() <= most) lc = l0;
     }
     if (lc < 0) {
@@ -1188,10 +1238,24 @@ static int plan_coarse(gfd_poisson* p, const Schedule& sc, int dtype,
         bytes = 0;
         one = false;
     }
-    const bool same = c.valid && c.lc == lc &&
+    // one entry per level whatever lc is: the device table keeps its place
+    std::vector<TsGrid> ts(p->L + 1);
+    std::vector<int> tiles(p->L + 1, 0);
+    for (int l = 1; l < (lc >= 0 ? lc : sc.coarsest); l++)
+        tiles[l] = ts_level(p, sc, dtype, l, ts[l]);
+    const size_t tsb = sizeof(TsGrid) * ts.size();
+    const bool same = c.valid && c.lc == lc && c.tstiles == tiles &&
+                      std::memcmp(c.ts.data(), ts.data(), tsb) == 0 &&
                       (lc < 0 || std::memcmp(&c.host, &g, sizeof g) == 0);
     if (changed) *changed = !same;
     if (same) return OK;
+    c.valid = false;  // until the tables are uploaded
+    GFD_TRY(c.tsdev.ensure(tsb, s));
+    GFD_CHECK_HIP(hipMemcpyAsync(c.tsdev.p, ts.data(), tsb,
+                                 hipMemcpyHostToDevice, s));
+    GFD_CHECK_HIP(hipStreamSynchronize(s));
+    c.ts = ts;
+    c.tstiles = tiles;
     if (lc >= 0) {
         GFD_TRY(c.dev.ensure(sizeof(CGrid), s));
         GFD_CHECK_HIP(hipMemcpyAsync(c.dev.p, &g, sizeof(CGrid),
@@ -1232,6 +1296,25 @@ static int vcycle(gfd_poisson* p, Levels& lv, const Schedule& sc, int l,
         }
         return vec_zero_bytes(*cur, es * op->ng(), s);
     };
+    const CoarseSolve& cs =
+        &lv == &p->lv64r ? p->cs64r : (dt == 2 ? p->cs32 : p->cs64);
+    if (zero && cs.valid && l < (int)cs.tstiles.size() && cs.tstiles[l]) {
+        const TsGrid* g = (const TsGrid*)cs.tsdev.p + l;
+        GFD_TRY(launch_ts_down(g, 1, cs.tstiles[l], dt, sched_pre(sc, l),
+                               rho, *cur, lv.rho[l + 1], s));
+        void* c1 = lv.phi[l + 1];
+        void* a1 = lv.tmp[l + 1];
+        if (cs.lc == l + 1)
+            GFD_TRY(launch_coarse((const CGrid*)cs.dev.p, 1, cs.lds, dt,
+                                  lv.rho[l + 1], c1, cs.one, s));
+        else
+            GFD_TRY(vcycle(p, lv, sc, l + 1, &c1, &a1, lv.rho[l + 1], s,
+                           true));
+        GFD_TRY(launch_ts_up(g, 1, cs.tstiles[l], dt, sched_post(sc, l), rho,
+                             *cur, c1, *alt, s));
+        std::swap(*cur, *alt);
+        return OK;
+    }
     if (l < sc.coarsest) {
         int done = 0;
         GFD_TRY(relax_from(sched_pre(sc, l), done));
@@ -1247,8 +1330,6 @@ static int vcycle(gfd_poisson* p, Levels& lv, const Schedule& sc, int l,
                         xe, s, p->xscratch.p));
         void* c1 = lv.phi[l + 1];
         void* a1 = lv.tmp[l + 1];
-        const CoarseSolve& cs =
-            &lv == &p->lv64r ? p->cs64r : (dt == 2 ? p->cs32 : p->cs64);
         if (cs.valid && cs.lc == l + 1) {
             // levels l+1 .. coarsest in one LDS-resident workgroup
             GFD_TRY(launch_coarse((const CGrid*)cs.dev.p, 1, cs.lds, dt,
@@ -1370,10 +1451,22 @@ static int read_scalar(gfd_poisson* p, hipStream_t s, double* h)
     return OK;
 }
 
+// The FP64 schedule's plan; a captured cycle of an older plan is dropped.
+static int plan_reference(gfd_poisson* p, hipStream_t s)
+{
+    bool changed = false;
+    GFD_TRY(plan_coarse(p, ref_schedule(p), 0, p->cs64, s, &changed));
+    if (changed && p->g64) {
+        (void)hipGraphExecDestroy(p->g64);
+        p->g64 = nullptr;
+    }
+    return OK;
+}
+
 static int poisson_iterate(gfd_poisson* p, double* phi, const double* rho,
                            double* error, hipStream_t s)
 {
-    GFD_TRY(plan_coarse(p, ref_schedule(p), 0, p->cs64, s, nullptr));
+    GFD_TRY(plan_reference(p, s));
     GFD_TRY(p->scalar.ensure(4 * sizeof(double), s));
     GFD_TRY(vcycle64_norm(p, phi, rho, (double*)p->scalar.p, s));
     double h = 0.0;
@@ -1441,14 +1534,7 @@ extern "C" int gfd_poisson_solve(gfd_poisson* p, double* phi,
     double* dn = (double*)p->scalar.p;
     int it = 1;
     double err = 0.0;
-    {
-        bool changed = false;
-        GFD_TRY(plan_coarse(p, ref_schedule(p), 0, p->cs64, s, &changed));
-        if (changed && p->g64) {
-            (void)hipGraphExecDestroy(p->g64);
-            p->g64 = nullptr;
-        }
-    }
+    GFD_TRY(plan_reference(p, s));
     if (p->use_graph) {
         GFD_TRY(enter_owned(p, phi, rho, s));
         double* phi0 = (double*)p->lv.phi[0];
@@ -1889,6 +1975,10 @@ extern "C" int gfd_set_tuning(const char* key, long value)
     }
     if (std::strcmp(key, "coarse_lds") == 0) {
         g_coarse_lds = value != 0;
+        return OK;
+    }
+    if (std::strcmp(key, "tsmooth") == 0) {
+        ts_set_enabled(value != 0);
         return OK;
     }
     if (std::strcmp(key, "coarse_cheb") == 0) {

@@ -684,22 +684,25 @@ int gram(BandWork& w, const double2* A, long lda, const double2* B, long ldb,
         set_error("gram: no points");
         return EINVAL_;
     }
-    // chunks: 6 to 10 blocks per CU (256 CUs, one block at a time each), the
-    // count that leaves the last round fullest (500 bands, 10 lower tiles:
-    // 231 chunks started a tenth round for 6 blocks, 18.6 ms); at least 4
-    // stages each
+    // chunks: the count with the least estimated time on 256 CUs that run
+    // one block at a time each, rounds x (points of a chunk + 61): a block's
+    // 262 KB of partial sums cost as much to write and read back as some 61
+    // points of its tile take to multiply.  (500 bands, 10 lower tiles: 231
+    // chunks started a tenth round for 6 blocks, 18.6 ms.)  At most 10
+    // rounds, at least 4 stages per chunk; a few per cent in favour of more
+    // rounds, which even out blocks of unequal speed.
     long chunks = 1;
-    double best = 0.0;
-    for (long c = std::max(1L, 1536L / nt); c <= std::max(1L, 2560L / nt);
-         c++) {
-        const long b = nt * c;
-        const double full = (double)b / ((b + 255) / 256 * 256);
-        if (full >= best) {
-            best = full;
+    double least = 1e300;
+    const long top = std::max(1L, std::min(2560L / nt, K / (4 * GK)));
+    for (long c = 1; c <= top; c++) {
+        const double rounds = (double)((nt * c + 255) / 256);
+        const double cost =
+            rounds * ((double)K / c + 61.0) * (1.0 + 0.06 / rounds);
+        if (cost < least) {
+            least = cost;
             chunks = c;
         }
     }
-    chunks = std::min(chunks, std::max(1L, K / (4 * GK)));
     long kchunk = (K + chunks - 1) / chunks;
     kchunk = (kchunk + GK - 1) / GK * GK;
     chunks = (K + kchunk - 1) / kchunk;

@@ -23,6 +23,7 @@
 
 #include "batch.h"
 #include "coarse.h"
+#include "tsmooth.h"
 #include "gfd_common.h"
 #include "handles.h"
 #include "stencil_dev.h"
@@ -424,6 +425,10 @@ struct gfd_batch_poisson {
     std::vector<BLevel> lev;
     std::vector<BPair> pair;
     BLevel l0_64;                   // level 0 for the FP64 residual
+    // blocked half cycles of levels 1 .. L - 2 (tiles 0: separate launches)
+    std::vector<std::vector<TsGrid>> ts;
+    std::vector<long> tstiles;
+    std::vector<DevBuf> d_ts;
     bool tuned = false;
     // FP64 level-0 arrays, FP32 arrays per level
     DevBuf phi, rho;
@@ -913,6 +918,39 @@ extern "C" int gfd_batch_poisson_new(int G, int L, gfd_operator** ops,
         pr.nr = p0r;
         pr.ni = p0i;
     }
+    b->ts.resize(L);
+    b->tstiles.assign(L, 0);
+    b->d_ts.resize(L);
+    for (int l = 1; l + 1 < L; l++) {
+        long t = 0;
+        bool ok = b->lev[l].total <= TS_PTS;
+        for (int g = 0; g < G && ok; g++) {
+            const AxisStencil& ax = ops[g * L + l]->ax;
+            const XferPlan& r = rst[g * (L - 1) + l]->plan;
+            const XferPlan& i = itp[g * (L - 1) + l]->plan;
+            TsGrid x{};
+            ok = ax.R == 1 && ax.has[0] && ax.has[1] && ax.has[2];
+            for (int d = 0; d < 3; d++) {
+                x.n[d] = b->lev[l].st[g].n[d];
+                x.nc[d] = b->lev[l + 1].st[g].n[d];
+                x.periodic[d] = b->lev[l].st[g].periodic[d];
+                x.roff[d] = r.ax[d].off;
+                x.ioff[d] = i.ax[d].off;
+                x.iskip0[d] = i.ax[d].skip0;
+                x.cp[d] = ax.cp[d][0];
+                x.cm[d] = ax.cm[d][0];
+                ok = ok && (x.roff[d] == 0 || x.roff[d] == 1);
+            }
+            x.off = b->lev[l].st[g].off;
+            x.offc = b->lev[l + 1].st[g].off;
+            x.c0 = b->lev[l].st[g].c0;
+            x.w = b->lev[l].st[g].w;
+            x.tile0 = (int)t;
+            t += ts_tiles(x);
+            b->ts[l].push_back(x);
+        }
+        b->tstiles[l] = ok ? t : 0;
+    }
     int dev = 0;
     if (hipGetDevice(&dev) == hipSuccess) {
         hipDeviceProp_t pr;
@@ -934,6 +972,7 @@ extern "C" void gfd_batch_poisson_free(gfd_batch_poisson* b)
     if (b->gs) (void)hipStreamSynchronize(b->gs);
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
     for (auto& lv : b->lev) lv.d_st.release();
+    for (auto& d : b->d_ts) d.release();
     b->l0_64.d_st.release();
     for (auto& pr : b->pair) {
         pr.d_rst.release();
@@ -1197,6 +1236,33 @@ static int b_relax0(gfd_batch_poisson* b, int l, void** cur, void** alt,
     return b_relax(b, l, cur, alt, rhs, n - 1, s);
 }
 
+// Whether level l's half cycles run blocked (their table is uploaded).
+static bool b_blocked(const gfd_batch_poisson* b, int l, int pre, int post)
+{
+    return ts_enabled() && b->tstiles[l] > 0 && pre >= 1 && pre <= TS_MAXS &&
+           post >= 1 && post <= TS_MAXS;
+}
+
+// Upload the tables of the blocked levels (once; not under capture).
+static int b_plan_blocked(gfd_batch_poisson* b, int pre, int post,
+                          hipStream_t s)
+{
+    for (int l = 1; l + 1 < b->L; l++) {
+        if (!b_blocked(b, l, pre, post) || b->d_ts[l].p) continue;
+        const size_t bytes = sizeof(TsGrid) * b->ts[l].size();
+        GFD_TRY(b->d_ts[l].ensure(bytes, s));
+        if (hipMemcpyAsync(b->d_ts[l].p, b->ts[l].data(), bytes,
+                           hipMemcpyHostToDevice, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess) {
+            (void)hipGetLastError();
+            b->d_ts[l].release();  // never run on a table not filled
+            set_error("batched Poisson: upload of a level's table failed");
+            return EHIP;
+        }
+    }
+    return OK;
+}
+
 // FP32 V-cycle on e_l for right-hand side r_l, from e_l = 0 (*cur is not
 // read).  phi (level 0 only, may be null): when the level's stencil runs
 // on x-march tiles, the last post-smoothing sweep subtracts its result
@@ -1207,6 +1273,19 @@ static int b_vcycle(gfd_batch_poisson* b, int l, void** cur, void** alt,
                     hipStream_t s, double* phi = nullptr,
                     bool* sub = nullptr)
 {
+    if (l >= 1 && l + 1 < b->L && b_blocked(b, l, pre, post)) {
+        const TsGrid* g = (const TsGrid*)b->d_ts[l].p;
+        GFD_TRY(launch_ts_down(g, b->G, b->tstiles[l], 2, pre, rhs, *cur,
+                               b->r32[l + 1].p, s));
+        void* c1 = b->e32[l + 1].p;
+        void* a1 = b->t32[l + 1].p;
+        GFD_TRY(b_vcycle(b, l + 1, &c1, &a1, b->r32[l + 1].p, pre, post,
+                         coarse, s));
+        GFD_TRY(launch_ts_up(g, b->G, b->tstiles[l], 2, post, rhs, *cur, c1,
+                             *alt, s));
+        std::swap(*cur, *alt);
+        return OK;
+    }
     if (l + 1 < b->L) {
         GFD_TRY(b_relax0(b, l, cur, alt, rhs, pre, s));
         GFD_TRY(bst(b->lev[l], 2, EPI_RESID, *cur, b->s32[l].p, rhs, nullptr,
@@ -1512,6 +1591,7 @@ extern "C" int gfd_batch_poisson_solve_mixed(
     };
     bool cchanged = false;
     GFD_TRY(b_plan_coarse(b, pre, post, coarse_sweeps, s, &cchanged));
+    GFD_TRY(b_plan_blocked(b, pre, post, s));
     const int key[4] = {pre, post, coarse_sweeps, b->coarse ? 1 : 0};
     if (b->graph && (cchanged || !std::equal(key, key + 4, b->gkey))) {
         (void)hipGraphExecDestroy(b->graph);

@@ -453,8 +453,11 @@ int gfd_woperator_get_diagonal_element(gfd_woperator* op, double* out,
  * bit 0 non-temporal stores, bit 1 non-temporal loads);
  * "coarse_lds" (0/1, default 1) runs the coarse levels of the Poisson
  * V-cycles that fit in one workgroup's LDS as a single launch;
- * "coarse_max_points" (default and 0: 14000 with radius-1 stencils, else
- * 4096) caps the points of its first level; "coarse_cheb" (0/1, default 1) makes the coarsest level of
+ * "coarse_max_points" (default and 0: 4096, or 14000 with radius-1 stencils
+ * and more than 4 sweeps) caps the points of its first level; "tsmooth"
+ * (0/1, default 1) runs each half cycle of the levels between it and the
+ * finest as one launch; "coarse_cheb" (0/1, default 1) makes the coarsest
+ * level of
  * that solve in the mixed-precision schedules (single grid and batched)
  * run Chebyshev iteration on D^-1 A (eigenvalue bounds from the radius-1
  * stencil's Fourier / sine modes) instead of Jacobi sweeps; the reference
