@@ -20,7 +20,7 @@ ARCH = 'gfx950'
 SOURCES = ['dirmarch_c128.hip', 'dirmarch_f64.hip', 'dirmarch_c64.hip',
            'dirmarch_f32.hip', 'dirmarch.hip', 'rows_dma.hip', 'rows_dma32.hip', 'rows_f64.hip', 'rows_c128.hip', 'rows_f32.hip', 'rows_c64.hip',
            'stencil.hip', 'batch.hip', 'transfer.hip', 'api.hip',
-           'stencil_rows.hip', 'vector.hip', 'bands.hip', 'coarse.hip', 'tsmooth.hip',
+           'stencil_rows.hip', 'point.hip', 'vector.hip', 'bands.hip', 'coarse.hip', 'tsmooth.hip',
            'fftpoisson.hip', 'wstencil.hip', 'gs.hip',
            'xfer_march.hip', 'wxmarch.hip', 'wdielectric.hip', 'bxmarch.hip', 'bxfer_march.hip',
            'precond_fine.hip']

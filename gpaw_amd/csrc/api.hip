@@ -20,6 +20,7 @@
 #include "bands.h"
 #include "handles.h"
 #include "coarse.h"
+#include "point.h"
 #include "tsmooth.h"
 #include "gs.h"
 #include "wstencil.h"
@@ -236,7 +237,8 @@ static bool aligned16(const void* p)
     return ((uintptr_t)p & 15) == 0;
 }
 
-// Kernel family for one pass: 3 full-row, 2 direction march, 1 general.
+// Kernel family for one pass: 4 one point per thread, 3 full-row, 2 direction
+// march, 1 general.
 static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
                    const void* out, const void* aux, int epi)
 {
@@ -244,6 +246,9 @@ static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
     const bool dir = op->dir_ok && g_force_path != 3 &&
                      dirmarch_fits(op->dir, dtype, op->n, epi);
     if (dir && g_force_path == 2) return 2;
+    if (g_force_path == 0 && op->axis_ok &&
+        point_fits(op->ax, dtype, op->n, nin, epi))
+        return 4;
     // Complex FP64: the direction march from radius 3 on and for H psi at
     // any radius.  k_xrow holds 2R + 2 planes of 16-byte points in registers
     // (2 waves per SIMD at R = 3); measured over 1, 4 and 32 grids of 48^3,
@@ -269,6 +274,9 @@ static int op_pass(gfd_operator* op, int dtype, const void* in, void* out,
     if (path == 3)
         return launch_row_stencil(op->ax, dtype, op->n, bc, in, out, nin, epi,
                                   ea, s, nblocks);
+    if (path == 4)
+        return launch_point(op->ax, dtype, op->n, bc, in, out, nin, epi, ea,
+                            s, nblocks);
     if (path == 2)
         return launch_dirmarch(op->dir, dtype, op->n, bc, in, out, nin, epi,
                                ea, s, nblocks);
