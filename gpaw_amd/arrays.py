@@ -24,11 +24,14 @@ def torch_dtype(dtype):
     return _NP2T[np.dtype(dtype)]
 
 
+_T2NP = {t: d for d, t in _NP2T.items()}
+
+
 def np_dtype(t):
-    for k, v in _NP2T.items():
-        if v == t:
-            return k
-    raise TypeError(f'unsupported dtype {t}')
+    try:
+        return _T2NP[t]
+    except KeyError:
+        raise TypeError(f'unsupported dtype {t}') from None
 
 
 def is_device(a) -> bool:
@@ -47,8 +50,10 @@ def device():
 
 
 def stream_handle():
-    """hipStream_t of torch's current stream (ordering with torch ops)."""
-    return torch.cuda.current_stream().cuda_stream
+    """hipStream_t of torch's current stream (ordering with torch ops).
+    The raw handle of the current device's stream: building the Stream
+    object around it took 3 us of an 11 us call."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def ptr(t) -> int:
@@ -93,10 +98,9 @@ class Staging:
     """Run device code on host arrays: upload inputs, download outputs."""
 
     def __init__(self, *arrays):
-        self.host = [a for a in arrays]
-        self.any_host = any(a is not None and not is_device(a)
-                            for a in arrays)
-        self.dev = [None if a is None else to_device(a) for a in arrays]
+        self.host = arrays
+        self.dev = [a if a is None or is_device(a) else to_device(a)
+                    for a in arrays]
 
     def download(self, *idx):
         for i in idx:

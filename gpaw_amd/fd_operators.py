@@ -21,7 +21,7 @@ built here from the defining equations, written down next to each builder:
 from __future__ import annotations
 
 import itertools
-from math import pi
+from math import pi, prod
 
 import numpy as np
 
@@ -54,7 +54,7 @@ _HALF_STEPS = np.array([m for m in itertools.product((-1, 0, 1), repeat=3)
 
 
 def _nin(shape):
-    return int(np.prod(shape[:-3], dtype=np.int64))
+    return prod(shape[:-3])
 
 
 def _line(step_c, weights, sign):
@@ -143,11 +143,11 @@ class FDOperator:
     #    (gpaw/fd_operators.py:150-174), always on here: the kernels trust
     #    shapes and dtypes
     def _check(self, in_xg, out_xg, phase_cd):
-        if tuple(in_xg.shape) != tuple(out_xg.shape):
+        shape = tuple(in_xg.shape)
+        if shape != tuple(out_xg.shape):
             raise ValueError('input and output shapes differ')
-        if tuple(in_xg.shape[-3:]) != self.shape:
-            raise ValueError(f'grid shape {tuple(in_xg.shape[-3:])} != '
-                             f'{self.shape}')
+        if shape[-3:] != self.shape:
+            raise ValueError(f'grid shape {shape[-3:]} != {self.shape}')
         want = np.dtype(self.dtype)
         if dtype_of(in_xg) != want or dtype_of(out_xg) != want:
             raise TypeError(f'arrays must be {want}')

@@ -8,6 +8,8 @@ into the interior-index offsets of its wrap-based kernels.
 """
 from __future__ import annotations
 
+from math import prod
+
 import numpy as np
 
 from . import _lib
@@ -119,7 +121,7 @@ class _Transformer:
         if self.dtype != float:
             keep, ph = _lib.phases_arg(np.ones((3, 2), complex)
                                        if phases is None else phases)
-        nin = int(np.prod(input.shape[:-3], dtype=np.int64))
+        nin = prod(input.shape[:-3])
         h = self._handle()
         _lib.check(self._lib.gfd_transformer_apply(
             h, ptr(st.dev[0]), ptr(st.dev[1]), nin, ph, stream_handle()),
