@@ -249,6 +249,9 @@ static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
     if (g_force_path == 0 && op->axis_ok &&
         point_fits(op->ax, dtype, op->n, nin, epi))
         return 4;
+    // Real FP64 just beyond those: 8 x 48^3, nn=3: 8.6 us, full rows 9.5;
+    // 96^3 8.8 / 9.5; but 4 x 64^3 9.1 / 8.8, 2 x 96^3 11.4 / 11.5.
+    if (dir && dtype == 0 && (double)op->ng() * nin <= 900e3) return 2;
     // Complex FP64: the direction march from radius 3 on and for H psi at
     // any radius.  k_xrow holds 2R + 2 planes of 16-byte points in registers
     // (2 waves per SIMD at R = 3); measured over 1, 4 and 32 grids of 48^3,

@@ -88,7 +88,9 @@ void dirmarch_set_tile(const XmTile* t)
 // the rows split evenly) and x chunk with the least estimated time:
 //   planes per block (every chunk stages 2R planes more)
 //   x waves of all blocks of one CU x (1 + 0.12 per staged element)
-//   x (1 + 4 / resident waves per CU): too few do not hide the latency.
+//   x (1 + 4 / resident waves per CU): too few do not hide the latency
+//   x (1 + 0.2 x cache lines loaded per line of results): short rows and
+//     small tiles load partial lines and more halo.
 // The weights fit measured sweeps (48 c128 grids of 128^3: 64 x 8 threads
 // 703 us, 128 x 4 with 4 staged elements 795, 32 x 8 802; 40 f64 grids of
 // 87x103x95: 48 x 10 in two chunks 174 us, whole x 184, 95 x 5 209; 24 c128
@@ -117,6 +119,10 @@ static DirTile dm_tile(const DirStencil& d, int dtype, const int n[3],
             if (lsz > 4L * threads) continue;
             const int hm = lsz <= 2L * threads ? 2 : 4;
             const int waves = threads / 64;
+            const int es = dtype == 1 ? 16 : dtype == 2 ? 4 : 8;
+            const double lines = (t.ty + 2 * R) *
+                                 ((t.tz + 2 * R) * es / 128.0 + 1.0) /
+                                 (t.tz * t.ty * es / 128.0);
             const long tiles = (long)parts * nr * nin;
             for (int chunks = 1; chunks <= std::max(1, n[0] / 4);
                  chunks++) {
@@ -127,7 +133,8 @@ static DirTile dm_tile(const DirStencil& d, int dtype, const int n[3],
                     std::min<long>(per, std::max(1, hold / waves)) * waves;
                 const double cost = (double)(t.xchunk + 2 * R) * per * waves *
                                     (1.0 + 0.12 * hm) *
-                                    (1.0 + 4.0 / resident);
+                                    (1.0 + 4.0 / resident) *
+                                    (1.0 + 0.2 * lines);
                 if (cost < least) {
                     least = cost;
                     best = t;

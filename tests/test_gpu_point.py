@@ -58,10 +58,10 @@ def test_passes(nn, N, pbc):
     assert relerr(host(out), want) < TOL
 
 
-@pytest.mark.parametrize('count', [9, 10])
+@pytest.mark.parametrize('count', [9, 10, 14, 15])
 def test_either_side_of_the_limit(count):
-    """600 000 points are 9.4 grids of 40^3: one point per thread, then a
-    marching kernel."""
+    """600 000 points are 9.4 grids of 40^3, 900 000 are 14.1: one point per
+    thread, the direction march, full rows."""
     rng = np.random.default_rng(2)
     gd = grid((40, 40, 40), True)
     op = Laplace(gd, 1.0, 3)
