@@ -1988,6 +1988,10 @@ extern "C" int gfd_set_tuning(const char* key, long value)
         g_coarse_lds = value != 0;
         return OK;
     }
+    if (std::strcmp(key, "xfer_tile") == 0) {
+        xfer_set_tile(value != 0);
+        return OK;
+    }
     if (std::strcmp(key, "tsmooth") == 0) {
         ts_set_enabled(value != 0);
         return OK;

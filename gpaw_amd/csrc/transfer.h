@@ -52,12 +52,16 @@ bool xfer_passes_forced();
 // (default 1: about four).
 void xfer_set_march_scale(int s);
 
+// K = 2 restrictions on the tiled kernel wherever it fits (default: where it
+// was timed to be the fastest).
+void xfer_set_tile(bool on);
+
 // Timed choice between the x-marching kernel and the other kernels per
 // transfer shape (on by default; off also forgets the choices).
 void xfer_set_autotune(bool on);
 // Whether this shape has no choice yet (and the tuner is on).
 bool xfer_needs_tuning(const XferPlan& p, int dtype, long nin, int in_wide);
-// Time both kernel families with PLAIN passes of `in` into tune_out
+// Time the kernel families with PLAIN passes of `in` into tune_out
 // (output-sized scratch) and record the faster.  Not under graph capture.
 int xfer_tune(const XferPlan& p, int dtype, const BC& bc, const void* in,
               void* tune_out, long nin, void* scratch, int in_wide,

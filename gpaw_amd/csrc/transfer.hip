@@ -18,7 +18,11 @@
 // The weights are exact dyadic rationals.
 #include "transfer.h"
 
+#include "batch.h"
+#include "stencil_dev.h"
+
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <mutex>
 
@@ -263,6 +267,147 @@ __global__ void __launch_bounds__(256) k_restrict2(F3Args<T, TI> a)
     f3store<T, EPI, TI>(a, gid, v);
 }
 
+// ------------------------------------------------- tiled K = 2 restriction
+//
+// A block stages the (2 CX + 1) x (2 CY + 1) x (2 cz + 1) fine points under
+// its CX x CY x cz coarse ones in LDS, every load of the tile in flight at
+// once (a wave per fine row, addresses uniform but for the lane), then forms
+// each output from its 27 values.  One load latency and one barrier, where
+// the marching kernel has one of each per fine plane and the
+// one-point-per-thread kernel reads every fine point 3.4 times through L1
+// with a stride of two.  A tile fits LDS three or four times per CU, and its
+// rows are loaded in two rounds.  Measured, before (the faster of the two
+// others) and with the tiles: 192^3 FP32 in the V-cycle 21.6 -> 16.0 us (read
+// once 5); 8 complex grids of 128^3 84 -> 64 (50); 32 of 108x120x132 narrowed
+// to FP32 283 -> 231 (160; 250 with five rounds of loads).  16 real grids of
+// 96^3 stay with marching, 36 against 39: the kernel is timed per shape.
+// Arrays of at least 2 GiB per grid (buffer offsets) stay with those.
+template <typename T> struct RtTile {
+    static constexpr int CX = sizeof(T) == 4 ? 4 : 2;
+    static constexpr int CY = sizeof(T) == 16 ? 4 : 8;
+};
+constexpr int RT_CZ = 32;          // most coarse z points of a tile
+constexpr int RT_P = 2 * RT_CZ + 1;
+
+template <typename T, int EPI, typename TI>
+__global__ void __launch_bounds__(256)
+k_restrict_tile(F3Args<T, TI> a, int cz, int tiles_z, int tiles_y,
+                int tiles_x, int nblocks)
+{
+    typedef typename ScalarOf<T>::type S;
+    constexpr int CX = RtTile<T>::CX, CY = RtTile<T>::CY;
+    constexpr int RX = 2 * CX + 1, RY = 2 * CY + 1, ROWS = RX * RY;
+    constexpr bool CPLX = XIsCplx<TI>::value;
+    __shared__ T E[ROWS * RT_P];
+    int rem = xcd_remap(blockIdx.x, nblocks);
+    const int zt = rem % tiles_z;
+    rem /= tiles_z;
+    const int yt = rem % tiles_y;
+    rem /= tiles_y;
+    const int xt = rem % tiles_x;
+    const long b = rem / tiles_x;
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int W = 2 * cz + 1;
+    // first fine point of the tile (halo included)
+    const int fx = 2 * xt * CX + a.off[0] - 1, fy = 2 * yt * CY + a.off[1] - 1,
+              fz = 2 * zt * cz + a.off[2] - 1;
+    const __amdgpu_buffer_rsrc_t src =
+        brsrc(a.in + b * a.in_grid, (unsigned)(a.in_grid * sizeof(TI)));
+    // wrapped index along an axis (-1: zero) and its Bloch factor, applied
+    // after those of the axes before
+    auto wrap = [&](int i, int c, double2& f, bool& ph) {
+        if (i >= 0 && i < a.ni[c]) return i;
+        if (!a.periodic[c]) return -1;
+        while (i < 0) {
+            i += a.ni[c];
+            f = ph ? cmul(a.ph[c][1], f) : a.ph[c][1];
+            ph = true;
+        }
+        while (i >= a.ni[c]) {
+            i -= a.ni[c];
+            f = ph ? cmul(a.ph[c][0], f) : a.ph[c][0];
+            ph = true;
+        }
+        return i;
+    };
+    // byte offset of a fine row, BXM_OOB if it is zero
+    auto row_at = [&](int r, double2& f, bool& ph) -> unsigned {
+        f = make_double2(1.0, 0.0);
+        ph = false;
+        const int x = wrap(fx + r / RY, 0, f, ph);
+        const int y = wrap(fy + r % RY, 1, f, ph);
+        return x < 0 || y < 0
+                   ? BXM_OOB
+                   : ((unsigned)x * a.ni[1] + (unsigned)y) * a.ni[2] *
+                         (unsigned)sizeof(TI);
+    };
+    // the z factor comes last: f_z (f_y f_x)
+    auto put = [&](int r, int z, TI v, double2 f, bool ph, double2 g,
+                   bool gph) {
+        if constexpr (CPLX)
+            if (ph || gph)
+                v = apply_phase(v, ph ? (gph ? cmul(g, f) : f) : g);
+        E[r * RT_P + z] = narrow<T, TI>(v);
+    };
+    double2 zf = make_double2(1.0, 0.0);
+    bool zph = false;
+    const int zw = lane < W ? wrap(fz + lane, 2, zf, zph) : -1;
+    const unsigned zo = zw < 0 ? BXM_OOB : (unsigned)zw * sizeof(TI);
+    // two rounds of loads per wave
+    constexpr int J = (ROWS + 3) / 4, JU = (J + 1) / 2;
+    for (int j0 = 0; j0 < J; j0 += JU) {
+        TI v[JU];
+        double2 rf[JU];
+        bool rph[JU];
+        cfor<JU>([&](auto j) {
+            const int r = min(w + 4 * (j0 + j), ROWS - 1);
+            const unsigned ro = row_at(r, rf[j], rph[j]);
+            v[j] = bload<TI>(src, ro == BXM_OOB || zo == BXM_OOB
+                                      ? BXM_OOB : ro + zo);
+        });
+        cfor<JU>([&](auto j) {
+            const int r = min(w + 4 * (j0 + j), ROWS - 1);
+            if (lane < W) put(r, lane, v[j], rf[j], rph[j], zf, zph);
+        });
+    }
+    if (W > 64 && t < ROWS) {  // the last point of each full row
+        double2 f, g = make_double2(1.0, 0.0);
+        bool ph, gph = false;
+        const int z = wrap(fz + 64, 2, g, gph);
+        const unsigned ro = row_at(t, f, ph);
+        put(t, 64,
+            bload<TI>(src, ro == BXM_OOB || z < 0
+                               ? BXM_OOB : ro + (unsigned)z * sizeof(TI)),
+            f, ph, g, gph);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < CX * CY * RT_CZ / 256; k++) {
+        const int id = t + 256 * k;
+        const int z = id % RT_CZ, y = id / RT_CZ % CY, x = id / (RT_CZ * CY);
+        const int oz = zt * cz + z, oy = yt * CY + y, ox = xt * CX + x;
+        if (z >= cz || oz >= a.no[2] || oy >= a.no[1] || ox >= a.no[0])
+            continue;
+        const T* p = E + (2 * x * RY + 2 * y) * RT_P + 2 * z;
+        T px[3];
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) {
+            T py[3];
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                const T* q = p + (dx * RY + dy) * RT_P;
+                const T zp = q[2] + q[0];
+                py[dy] = (S)0.5 * fmac(q[1], (S)0.5, zp);
+            }
+            px[dx] = (S)0.5 * fmac(py[1], (S)0.5, py[2] + py[0]);
+        }
+        const T v = (S)0.5 * fmac(px[1], (S)0.5, px[2] + px[0]);
+        f3store<T, EPI, TI>(
+            a, b * a.out_grid + ((long)ox * a.no[1] + oy) * a.no[2] + oz, v);
+    }
+}
+
 template <typename T, int EPI, typename TI>
 __global__ void __launch_bounds__(256) k_interp2(F3Args<T, TI> a)
 {
@@ -344,10 +489,9 @@ __global__ void __launch_bounds__(256) k_interp2p(F3Args<T, TI> a)
     f3store<T, EPI, TI>(a, gid + 1, v1);
 }
 
-template <typename T, int EPI, typename TI>
-static int launch_fused2_t(const XferPlan& p, const BC& bc, const void* in,
-                           void* out, long nin, const XEpiArgs& ea,
-                           hipStream_t s)
+template <typename T, typename TI>
+static F3Args<T, TI> f3args(const XferPlan& p, const BC& bc, const void* in,
+                            void* out, long nin, const XEpiArgs& ea)
 {
     F3Args<T, TI> a;
     a.in = (const TI*)in;
@@ -368,6 +512,72 @@ static int launch_fused2_t(const XferPlan& p, const BC& bc, const void* in,
     a.total = a.out_grid * nin;
     a.negate = ea.negate;
     a.alpha = ea.alpha;
+    return a;
+}
+
+template <typename T, int EPI, typename TI>
+static int launch_rtile_t(const XferPlan& p, const BC& bc, const void* in,
+                          void* out, long nin, const XEpiArgs& ea,
+                          hipStream_t s)
+{
+    const F3Args<T, TI> a = f3args<T, TI>(p, bc, in, out, nin, ea);
+    if (p.interpolate || p.K != 2 ||
+        a.in_grid * (long)sizeof(TI) >= (1L << 31)) {
+        set_error("tiled restriction: not for this transfer");
+        return ENOTSUP_;
+    }
+    const int tz = ceil_div(a.no[2], RT_CZ), cz = ceil_div(a.no[2], tz);
+    const int ty = ceil_div(a.no[1], RtTile<T>::CY);
+    const int tx = ceil_div(a.no[0], RtTile<T>::CX);
+    const long nb = (long)tz * ty * tx * nin;
+    if (nb <= 0) return OK;
+    if (nb > 0x7fffffffL) {
+        set_error("transfer: too many blocks");
+        return ENOTSUP_;
+    }
+    hipLaunchKernelGGL((k_restrict_tile<T, EPI, TI>), dim3((unsigned)nb),
+                       dim3(256), 0, s, a, cz, tz, ty, tx, (int)nb);
+    GFD_LAUNCH_CHECK();
+    return OK;
+}
+
+template <typename T, typename TI = T>
+static int launch_rtile(const XferPlan& p, const BC& bc, const void* in,
+                        void* out, long nin, const XEpiArgs& ea,
+                        hipStream_t s)
+{
+    switch (ea.epi) {
+    case XEPI_PLAIN: return launch_rtile_t<T, XEPI_PLAIN, TI>(p, bc, in, out, nin, ea, s);
+    case XEPI_NEG: return launch_rtile_t<T, XEPI_NEG, TI>(p, bc, in, out, nin, ea, s);
+    case XEPI_SCALE2: return launch_rtile_t<T, XEPI_SCALE2, TI>(p, bc, in, out, nin, ea, s);
+    case XEPI_SUBFROM: return launch_rtile_t<T, XEPI_SUBFROM, TI>(p, bc, in, out, nin, ea, s);
+    }
+    set_error("transfer: bad epilogue %d", ea.epi);
+    return EINVAL_;
+}
+
+static int launch_restrict_tile(const XferPlan& p, int dtype, const BC& bc,
+                                const void* in, void* out, long nin,
+                                const XEpiArgs& ea, hipStream_t s)
+{
+    switch (dtype) {
+    case 0: return launch_rtile<double>(p, bc, in, out, nin, ea, s);
+    case 1: return launch_rtile<double2>(p, bc, in, out, nin, ea, s);
+    case 2: return ea.in_wide ? launch_rtile<float, double>(p, bc, in, out, nin, ea, s)
+                              : launch_rtile<float>(p, bc, in, out, nin, ea, s);
+    case 3: return ea.in_wide ? launch_rtile<float2, double2>(p, bc, in, out, nin, ea, s)
+                              : launch_rtile<float2>(p, bc, in, out, nin, ea, s);
+    }
+    set_error("transfer: bad dtype %d", dtype);
+    return EINVAL_;
+}
+
+template <typename T, int EPI, typename TI>
+static int launch_fused2_t(const XferPlan& p, const BC& bc, const void* in,
+                           void* out, long nin, const XEpiArgs& ea,
+                           hipStream_t s)
+{
+    const F3Args<T, TI> a = f3args<T, TI>(p, bc, in, out, nin, ea);
     const long nb = (a.total + 255) / 256;
     if (nb <= 0) return OK;
     if (nb > 0x7fffffffL) {
@@ -530,7 +740,12 @@ struct XKey {
 };
 
 static std::mutex g_xc_mu;
-static std::map<XKey, int> g_xchoice;  // 0 marching, 1 other kernels
+// 0 marching, 1 other kernels, 2 tiled K = 2 restriction
+static std::map<XKey, int> g_xchoice;
+static std::atomic<bool> g_xfer_tile{false};  // tiled wherever it fits
+
+void xfer_set_tile(bool on) { g_xfer_tile = on; }
+
 static bool g_xtune = true;
 
 void xfer_set_autotune(bool on)
@@ -582,12 +797,14 @@ int xfer_tune(const XferPlan& p, int dtype, const BC& bc, const void* in,
     }
     float best = 1e30f;
     int choice = 0;
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < (p.K == 2 && !p.interpolate ? 3 : 2); c++) {
         auto run = [&]() {
             return c == 0 ? launch_transfer_march(p, dtype, bc, in, tune_out,
                                                   nin, ea, s)
-                          : launch_other(p, dtype, bc, in, tune_out, nin,
-                                         scratch, ea, s);
+                 : c == 1 ? launch_other(p, dtype, bc, in, tune_out, nin,
+                                         scratch, ea, s)
+                          : launch_restrict_tile(p, dtype, bc, in, tune_out,
+                                                 nin, ea, s);
         };
         if (run() != OK) {  // this kernel cannot take the shape
             set_error("");
@@ -625,10 +842,20 @@ int launch_transfer(const XferPlan& p, int dtype, const BC& bc,
         return EINVAL_;
     }
     bool march = g_xfer_march && !g_xfer_force_passes;
-    if (march) {
+    bool tile = g_xfer_tile && p.K == 2 && !p.interpolate;
+    if (march && !tile) {
         std::lock_guard<std::mutex> lk(g_xc_mu);
         auto it = g_xchoice.find(xkey(p, dtype, nin, ea.in_wide));
-        if (it != g_xchoice.end() && it->second == 1) march = false;
+        if (it != g_xchoice.end()) {
+            march = it->second == 0;
+            tile = it->second == 2;
+        }
+    }
+    if (tile) {
+        const int st =
+            launch_restrict_tile(p, dtype, bc, in, out, nin, ea, stream);
+        if (st != ENOTSUP_) return st;
+        set_error("");
     }
     if (march) {
         // the x-marching fused kernel (xfer_march.hip), any K

@@ -454,8 +454,9 @@ int gfd_woperator_get_diagonal_element(gfd_woperator* op, double* out,
  * "coarse_lds" (0/1, default 1) runs the coarse levels of the Poisson
  * V-cycles that fit in one workgroup's LDS as a single launch;
  * "coarse_max_points" (default and 0: 4096, or 14000 with radius-1 stencils
- * and more than 4 sweeps) caps the points of its first level; "tsmooth"
- * (0/1, default 1) runs each half cycle of the levels between it and the
+ * and more than 4 sweeps) caps the points of its first level; "xfer_tile"
+ * (0/1, default 0) runs every K = 2 restriction on the tiled kernel, which
+ * is otherwise one of the timed choices; "tsmooth" (0/1, default 1) runs each half cycle of the levels between it and the
  * finest as one launch; "coarse_cheb" (0/1, default 1) makes the coarsest
  * level of
  * that solve in the mixed-precision schedules (single grid and batched)
