@@ -43,7 +43,8 @@ struct XferPlan {
 // K = 2 transfers run as one fused kernel unless forced to the 3 passes.
 void xfer_force_passes(bool on);
 // Use the x-marching fused kernels (every K; default on).  Off: K = 2 by
-// the one-point-per-thread fused kernels, K > 2 by three 1-D passes.
+// the one-point-per-thread fused kernels, K > 2 by separable passes (z and y in one
+// launch, then x).
 void xfer_set_march(bool on);
 // Whether K = 2 transfers are forced onto the separable passes (they then
 // need the passes' work space).

@@ -104,8 +104,9 @@ __device__ inline T xload(const XArgs<T>& a, const T* __restrict__ g,
     return v;
 }
 
-template <typename T, int AX, int K, bool INTERP, int EPI>
-__global__ void __launch_bounds__(256) k_xfer1d(XArgs<T> a)
+// x pass
+template <typename T, int K, bool INTERP, int EPI>
+__global__ void __launch_bounds__(256) k_xfer_x(XArgs<T> a)
 {
     typedef typename ScalarOf<T>::type S;
     const long gid = (long)blockIdx.x * 256 + threadIdx.x;
@@ -113,19 +114,8 @@ __global__ void __launch_bounds__(256) k_xfer1d(XArgs<T> a)
     long b;
     int o0, o1, o2;
     flat_split(gid, a.total, a.out_grid, a.d[1], a.d[2], b, o0, o1, o2);
-    // input position with the pass axis at 0
-    long pos;
-    int i;
-    if (AX == 2) {
-        pos = ((long)o0 * a.d[1] + o1) * a.ilen;
-        i = o2;
-    } else if (AX == 1) {
-        pos = (long)o0 * a.ilen * a.d[2] + o2;
-        i = o1;
-    } else {
-        pos = (long)o1 * a.d[2] + o2;
-        i = o0;
-    }
+    const long pos = (long)o1 * a.d[2] + o2;  // at x = 0
+    const int i = o0;
     const T* __restrict__ g = a.in + b * a.in_grid;
     T v;
     if constexpr (!INTERP) {
@@ -615,13 +605,238 @@ static int launch_fused2(const XferPlan& p, const BC& bc, const void* in,
 
 long xfer_scratch_elems(const XferPlan& p, long nin)
 {
-    // pass z output + pass y output
-    const long t1 = (long)p.nin[0] * p.nin[1] * p.nout[2];
-    const long t2 = (long)p.nin[0] * p.nout[1] * p.nout[2];
-    return (t1 + t2) * nin;
+    // output of the z and y passes
+    return (long)p.nin[0] * p.nout[1] * p.nout[2] * nin;
 }
 
-template <typename T, int AX, int K, bool INTERP, int EPI>
+// z and y passes of a separable transfer in one launch: a block stages the
+// input rows under cy x zt outputs of one x plane in LDS, z-transforms them
+// there and writes the y transforms of the result.  As two launches the z
+// pass read each point K + 1 times through L1 and its result, as large as
+// half the input, went through memory.  The 1-D sums are those of the x pass.
+// Bound by the chain of a block (load, z, y; LDS reads of 7 values a point).
+// Two passes before -> this and x, K = 6: restriction of 4 real grids of 96^3
+// 25.4 -> 22.1 us, 32 of them 150 -> 122, one of 48^3 16.6 -> 8.4; staged
+// columns in order instead of even / odd: 24.2.  Interpolation of 4 complex
+// grids of 96^3 at K = 8 50.7 -> 38.6 (marching 112).
+template <typename T>
+struct ZyArgs {
+    const T* in;
+    T* out;
+    int n0, ni1, ni2, no1, no2;  // planes; rows and columns in and out
+    int cy, zt;                  // outputs of a block
+    int ry, rz;                  // staged rows and columns at most
+    int tiles_y, tiles_z, nblocks;
+    int off[2], skip0[2], periodic[2];  // y, z
+    double2 ph[2][2];
+};
+
+template <int K, bool INTERP>
+__device__ __host__ inline int zy_first(int i, int off, int skip0)
+{
+    return INTERP ? ((i + skip0) >> 1) + off - (K / 2 - 1)
+                  : 2 * i + off - (K - 1);
+}
+
+template <int K, bool INTERP>
+__device__ __host__ inline int zy_last(int i, int off, int skip0)
+{
+    return INTERP ? ((i + skip0) >> 1) + off + K / 2
+                  : 2 * i + off + (K - 1);
+}
+
+// output from the input at its centre p, neighbours s apart
+template <typename T, int K, bool INTERP>
+__device__ inline T zy_point(const T* p, int s, bool odd)
+{
+    typedef typename ScalarOf<T>::type S;
+    if constexpr (!INTERP) {
+        T acc = p[0];
+#pragma unroll
+        for (int m = 0; m < K / 2; m++) {
+            const int j = (2 * m + 1) * s;
+            acc = fmac(acc, (S)W<K>::w[m], p[j] + p[-j]);
+        }
+        return (S)0.5 * acc;
+    } else {
+        if (!odd) return p[0];
+        T acc = (S)W<K>::w[0] * (p[0] + p[s]);
+#pragma unroll
+        for (int m = 1; m < K / 2; m++)
+            acc = fmac(acc, (S)W<K>::w[m], p[-m * s] + p[(1 + m) * s]);
+        return acc;
+    }
+}
+
+template <typename T, int K, bool INTERP>
+__global__ void __launch_bounds__(256) k_xfer_zy(ZyArgs<T> a)
+{
+    typedef typename ScalarOf<T>::type S;
+    extern __shared__ __align__(16) char zy_lds[];
+    T* const E = reinterpret_cast<T*>(zy_lds);  // staged rows
+    T* const Z = E + a.ry * a.rz;               // their z transforms
+    int rem = xcd_remap(blockIdx.x, a.nblocks);
+    const int zt = rem % a.tiles_z;
+    rem /= a.tiles_z;
+    const int yt = rem % a.tiles_y;
+    const long pl = rem / a.tiles_y;
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int oy0 = yt * a.cy, oy1 = min(oy0 + a.cy, a.no1);
+    const int oz0 = zt * a.zt, oz1 = min(oz0 + a.zt, a.no2);
+    const int iy0 = zy_first<K, INTERP>(oy0, a.off[0], a.skip0[0]);
+    const int iz0 = zy_first<K, INTERP>(oz0, a.off[1], a.skip0[1]);
+    const int ny = zy_last<K, INTERP>(oy1 - 1, a.off[0], a.skip0[0]) - iy0 + 1;
+    const int nz = zy_last<K, INTERP>(oz1 - 1, a.off[1], a.skip0[1]) - iz0 + 1;
+    const T* __restrict__ g = a.in + pl * a.ni1 * a.ni2;
+    // staged column: for a restriction the even ones, then the odd ones, so
+    // that lanes next to each other read next to each other
+    const int half = (a.rz + 1) / 2;
+    auto col = [&](int z) {
+        return INTERP ? z : (z & 1) * half + (z >> 1);
+    };
+    // index inside the array (-1: zero) and its Bloch factor
+    auto wrap = [&](int i, int n, int c, double2& f, bool& ph) {
+        f = make_double2(1.0, 0.0);
+        ph = false;
+        if (i >= 0 && i < n) return i;
+        if (!a.periodic[c]) return -1;
+        while (i < 0) {
+            i += n;
+            f = ph ? cmul(a.ph[c][1], f) : a.ph[c][1];
+            ph = true;
+        }
+        while (i >= n) {
+            i -= n;
+            f = ph ? cmul(a.ph[c][0], f) : a.ph[c][0];
+            ph = true;
+        }
+        return i;
+    };
+    constexpr int JU = sizeof(T) == 16 ? 8 : 12;  // rows a wave has in flight
+    for (int z0 = 0; z0 < nz; z0 += 64) {
+        const int z = z0 + lane;
+        double2 f, fy;
+        bool ph, py;
+        const int iz = z < nz ? wrap(iz0 + z, a.ni2, 1, f, ph) : -1;
+        for (int j0 = w; j0 < ny; j0 += 4 * JU) {
+            T v[JU];
+#pragma unroll
+            for (int j = 0; j < JU; j++) {
+                v[j] = zero_of<T>();
+                const int r = j0 + 4 * j;
+                if (r >= ny) continue;
+                const int iy = wrap(iy0 + r, a.ni1, 0, fy, py);
+                if (iy >= 0 && iz >= 0) v[j] = g[(long)iy * a.ni2 + iz];
+            }
+#pragma unroll
+            for (int j = 0; j < JU; j++) {
+                const int r = j0 + 4 * j;
+                if constexpr (XIsCplx<T>::value)
+                    if (iz >= 0 && ph) v[j] = cmul(f, v[j]);
+                if (r < ny && z < nz) E[r * a.rz + col(z)] = v[j];
+            }
+        }
+    }
+    __syncthreads();
+    constexpr int BACK = INTERP ? K / 2 - 1 : K - 1;  // centre in its window
+    const int noz = oz1 - oz0;
+    const int dr = 256 / noz, dz = 256 % noz;
+    for (int r = t / noz, z = t % noz; r < ny;) {
+        T v;
+        if constexpr (INTERP) {
+            const int c = zy_first<K, INTERP>(oz0 + z, a.off[1],
+                                              a.skip0[1]) - iz0 + BACK;
+            v = zy_point<T, K, INTERP>(E + r * a.rz + c, 1,
+                                       (oz0 + z + a.skip0[1]) & 1);
+        } else {
+            // centre: staged column 2z + K - 1, neighbours: even columns
+            const T* p = E + r * a.rz + z + K / 2 - 1;
+            T acc = p[half];
+#pragma unroll
+            for (int m = 0; m < K / 2; m++)
+                acc = fmac(acc, (S)W<K>::w[m], p[m + 1] + p[-m]);
+            v = (S)0.5 * acc;
+        }
+        if constexpr (XIsCplx<T>::value) {
+            double2 f;
+            bool ph;
+            wrap(iy0 + r, a.ni1, 0, f, ph);
+            if (ph) v = cmul(f, v);
+        }
+        Z[r * a.zt + z] = v;
+        r += dr;
+        z += dz;
+        if (z >= noz) {
+            z -= noz;
+            r++;
+        }
+    }
+    __syncthreads();
+    T* __restrict__ o = a.out + pl * a.no1 * a.no2;
+    for (int oy = oy0 + w; oy < oy1; oy += 4) {
+        const int c =
+            zy_first<K, INTERP>(oy, a.off[0], a.skip0[0]) - iy0 + BACK;
+        const bool odd = (oy + a.skip0[0]) & 1;
+        for (int z = lane; z < noz; z += 64)
+            o[(long)oy * a.no2 + oz0 + z] =
+                zy_point<T, K, INTERP>(Z + c * a.zt + z, a.zt, odd);
+    }
+}
+
+// Outputs of a block: rows in equal parts of at most 64 columns (48 in
+// complex FP64, 128 when interpolating) by as many rows as leave 1024 blocks
+// and fit 64 KB of LDS; four rows always do (53 KB in complex FP64 at K = 8).
+template <typename T, int K, bool INTERP>
+static int launch_zy(const XferPlan& p, const BC& bc, const T* in, T* out,
+                     long nin, hipStream_t s)
+{
+    ZyArgs<T> a;
+    a.in = in;
+    a.out = out;
+    a.n0 = p.nin[0];
+    a.ni1 = p.nin[1];
+    a.ni2 = p.nin[2];
+    a.no1 = p.nout[1];
+    a.no2 = p.nout[2];
+    for (int c = 0; c < 2; c++) {
+        a.off[c] = p.ax[c + 1].off;
+        a.skip0[c] = p.ax[c + 1].skip0;
+        a.periodic[c] = bc.periodic[c + 1];
+        a.ph[c][0] = bc.phase[c + 1][0];
+        a.ph[c][1] = bc.phase[c + 1][1];
+    }
+    const long planes = (long)a.n0 * nin;
+    if (planes <= 0 || a.no1 <= 0 || a.no2 <= 0) return OK;
+    a.tiles_z = ceil_div(a.no2, INTERP ? 128 : sizeof(T) == 16 ? 48 : 64);
+    a.zt = ceil_div(a.no2, a.tiles_z);
+    // inputs under c outputs
+    auto span = [](int c) {
+        return INTERP ? c / 2 + K : 2 * (c - 1) + 2 * (K - 1) + 1;
+    };
+    a.rz = span(a.zt);
+    size_t lds = 0;
+    for (a.cy = INTERP ? 32 : 16;; a.cy /= 2) {
+        a.tiles_y = ceil_div(a.no1, a.cy);
+        a.ry = span(a.cy);
+        lds = (size_t)a.ry * (a.rz + a.zt) * sizeof(T);
+        if (a.cy == 4 || (lds <= 65536 &&
+                          planes * a.tiles_y * a.tiles_z >= 1024))
+            break;
+    }
+    const long nb = planes * a.tiles_y * a.tiles_z;
+    if (nb > 0x7fffffffL) {
+        set_error("transfer: too many blocks");
+        return ENOTSUP_;
+    }
+    a.nblocks = (int)nb;
+    hipLaunchKernelGGL((k_xfer_zy<T, K, INTERP>), dim3((unsigned)nb),
+                       dim3(256), lds, s, a);
+    GFD_LAUNCH_CHECK();
+    return OK;
+}
+
+template <typename T, int K, bool INTERP, int EPI>
 static int launch_pass(XArgs<T> a, hipStream_t s)
 {
     const long nb = (a.total + 255) / 256;
@@ -630,20 +845,20 @@ static int launch_pass(XArgs<T> a, hipStream_t s)
         set_error("transfer: too many blocks");
         return ENOTSUP_;
     }
-    hipLaunchKernelGGL((k_xfer1d<T, AX, K, INTERP, EPI>), dim3((unsigned)nb),
+    hipLaunchKernelGGL((k_xfer_x<T, K, INTERP, EPI>), dim3((unsigned)nb),
                        dim3(256), 0, s, a);
     GFD_LAUNCH_CHECK();
     return OK;
 }
 
-template <typename T, int AX, int K, bool INTERP>
+template <typename T, int K, bool INTERP>
 static int launch_pass_epi(XArgs<T> a, int epi, hipStream_t s)
 {
     switch (epi) {
-    case XEPI_PLAIN: return launch_pass<T, AX, K, INTERP, XEPI_PLAIN>(a, s);
-    case XEPI_NEG: return launch_pass<T, AX, K, INTERP, XEPI_NEG>(a, s);
-    case XEPI_SCALE2: return launch_pass<T, AX, K, INTERP, XEPI_SCALE2>(a, s);
-    case XEPI_SUBFROM: return launch_pass<T, AX, K, INTERP, XEPI_SUBFROM>(a, s);
+    case XEPI_PLAIN: return launch_pass<T, K, INTERP, XEPI_PLAIN>(a, s);
+    case XEPI_NEG: return launch_pass<T, K, INTERP, XEPI_NEG>(a, s);
+    case XEPI_SCALE2: return launch_pass<T, K, INTERP, XEPI_SCALE2>(a, s);
+    case XEPI_SUBFROM: return launch_pass<T, K, INTERP, XEPI_SUBFROM>(a, s);
     }
     set_error("transfer: bad epilogue %d", epi);
     return EINVAL_;
@@ -654,46 +869,29 @@ static int run_transfer(const XferPlan& p, const BC& bc, const void* in,
                         void* out, long nin, void* scratch,
                         const XEpiArgs& ea, hipStream_t s)
 {
-    T* t1 = (T*)scratch;
-    T* t2 = t1 + (long)p.nin[0] * p.nin[1] * p.nout[2] * nin;
-    const T* src = (const T*)in;
-    int cur[3] = {p.nin[0], p.nin[1], p.nin[2]};
-    // z, y, x
-    for (int step = 0; step < 3; step++) {
-        const int ax = 2 - step;
-        XArgs<T> a;
-        a.in = src;
-        a.ilen = cur[ax];
-        int d[3] = {cur[0], cur[1], cur[2]};
-        d[ax] = p.nout[ax];
-        a.d[0] = d[0];
-        a.d[1] = d[1];
-        a.d[2] = d[2];
-        a.istride = ax == 2 ? 1 : (ax == 1 ? (long)cur[2] : (long)cur[1] * cur[2]);
-        a.in_grid = (long)cur[0] * cur[1] * cur[2];
-        a.out_grid = (long)d[0] * d[1] * d[2];
-        a.total = a.out_grid * nin;
-        a.off = p.ax[ax].off;
-        a.skip0 = p.ax[ax].skip0;
-        a.periodic = bc.periodic[ax];
-        a.ph_hi = bc.phase[ax][0];
-        a.ph_lo = bc.phase[ax][1];
-        a.negate = ea.negate;
-        a.alpha = ea.alpha;
-        a.out2 = (T*)ea.out2;
-        a.base = (const T*)ea.base;
-        const bool last = (step == 2);
-        a.out = last ? (T*)out : (step == 0 ? t1 : t2);
-        const int epi = last ? ea.epi : XEPI_PLAIN;
-        int st;
-        if (ax == 2) st = launch_pass_epi<T, 2, K, INTERP>(a, epi, s);
-        else if (ax == 1) st = launch_pass_epi<T, 1, K, INTERP>(a, epi, s);
-        else st = launch_pass_epi<T, 0, K, INTERP>(a, epi, s);
-        if (st != OK) return st;
-        src = a.out;
-        cur[ax] = p.nout[ax];
-    }
-    return OK;
+    T* const t = (T*)scratch;
+    const int st =
+        launch_zy<T, K, INTERP>(p, bc, (const T*)in, t, nin, s);
+    if (st != OK) return st;
+    XArgs<T> a;
+    a.in = t;
+    a.out = (T*)out;
+    a.out2 = (T*)ea.out2;
+    a.base = (const T*)ea.base;
+    for (int c = 0; c < 3; c++) a.d[c] = p.nout[c];
+    a.ilen = p.nin[0];
+    a.istride = (long)p.nout[1] * p.nout[2];
+    a.in_grid = p.nin[0] * a.istride;
+    a.out_grid = p.nout[0] * a.istride;
+    a.total = a.out_grid * nin;
+    a.off = p.ax[0].off;
+    a.skip0 = p.ax[0].skip0;
+    a.periodic = bc.periodic[0];
+    a.ph_hi = bc.phase[0][0];
+    a.ph_lo = bc.phase[0][1];
+    a.negate = ea.negate;
+    a.alpha = ea.alpha;
+    return launch_pass_epi<T, K, INTERP>(a, ea.epi, s);
 }
 
 template <typename T>
@@ -867,7 +1065,7 @@ int launch_transfer(const XferPlan& p, int dtype, const BC& bc,
     return launch_other(p, dtype, bc, in, out, nin, scratch, ea, stream);
 }
 
-// the one-point-per-thread K = 2 kernels, or the three separable passes
+// the one-point-per-thread K = 2 kernels, or the separable passes
 static int launch_other(const XferPlan& p, int dtype, const BC& bc,
                         const void* in, void* out, long nin, void* scratch,
                         const XEpiArgs& ea, hipStream_t stream)

@@ -456,16 +456,15 @@ int gfd_woperator_get_diagonal_element(gfd_woperator* op, double* out,
  * "coarse_max_points" (default and 0: 4096, or 14000 with radius-1 stencils
  * and more than 4 sweeps) caps the points of its first level; "xfer_tile"
  * (0/1, default 0) runs every K = 2 restriction on the tiled kernel, which
- * is otherwise one of the timed choices; "tsmooth" (0/1, default 1) runs each half cycle of the levels between it and the
- * finest as one launch; "coarse_cheb" (0/1, default 1) makes the coarsest
- * level of
- * that solve in the mixed-precision schedules (single grid and batched)
+ * is otherwise one of the timed choices; "tsmooth" (0/1, default 1) runs
+ * each half cycle of the levels between it and the finest as one launch;
+ * "coarse_cheb" (0/1, default 1) makes the coarsest level of that solve in the mixed-precision schedules (single grid and batched)
  * run Chebyshev iteration on D^-1 A (eigenvalue bounds from the radius-1
  * stencil's Fourier / sine modes) instead of Jacobi sweeps; the reference
  * schedule keeps Jacobi;
- * "xfer_passes" (0/1) runs K = 2 transfers as three 1-D passes instead of
+ * "xfer_passes" (0/1) runs K = 2 transfers as separable passes instead of
  * the fused kernel; "xfer_march" (0/1, default 1) lets transfers use the
- * x-marching fused kernel (off: one point per thread for K = 2, three 1-D
+ * x-marching fused kernel (off: one point per thread for K = 2, separable
  * passes for K > 2); "xfer_march_scale" (>= 1, default 1) sets its tiles
  * per resident block to about 4 x value; "wx_march" (0/1, default 1) runs
  * weighted operators whose stencils are all axis-only (at most 4 of them)
