@@ -46,9 +46,15 @@ int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
 // estimated tile); nullptr clears.
 void dirmarch_set_tile(const XmTile* t);
 
+// Columns and rows of a tile, planes of an x chunk, threads of a block (one
+// per tile point, or more where the tile with its halo needs them to stage
+// it at four points each).
 struct DirTile {
-    int tz, ty, xchunk;
+    int tz, ty, xchunk, threads;
 };
+
+// The tile with the least estimated time; every grid of sides >= R has one.
+DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin);
 
 int dirmarch_f64(const DirStencil& d, const DirTile& t, const int n[3],
                  const BC& bc, const void* in, void* out, long nin, int epi,

@@ -81,7 +81,11 @@ void dirmarch_set_tile(const XmTile* t)
 {
     std::lock_guard<std::mutex> lk(g_dm_mu);
     g_dm_override = t != nullptr;
-    if (t) g_dm_tile = DirTile{t->tz, t->nseg * t->py, t->xchunk};
+    if (t) {
+        const int ty = t->nseg * t->py;
+        g_dm_tile = DirTile{t->tz, ty, t->xchunk,
+                            (t->tz * ty + 63) / 64 * 64};
+    }
 }
 
 // Tile (equal parts of a row by as many rows as 512 or 256 threads hold,
@@ -96,13 +100,13 @@ void dirmarch_set_tile(const XmTile* t)
 // 87x103x95: 48 x 10 in two chunks 174 us, whole x 184, 95 x 5 209; 24 c128
 // grids of 60x60x84, hexagonal: 28 x 9 in two chunks 55 us, whole x 58, in
 // four 64).
-static DirTile dm_tile(const DirStencil& d, int dtype, const int n[3],
-                       long nin)
+// pad: blocks of more threads than tile points, enough to stage the halo.
+static bool dm_search(const DirStencil& d, int dtype, const int n[3],
+                      long nin, bool pad, DirTile& best)
 {
     const int R = d.R;
     // waves a CU holds: complex FP64 takes about 128 registers at R = 3
     const int hold = dtype == 1 && R > 1 ? 16 : 32;
-    DirTile best{std::min(n[2], 64), std::min(n[1], 8), n[0]};
     double least = 1e300;
     for (int parts = 1; parts <= n[2]; parts++) {
         DirTile t;
@@ -114,11 +118,13 @@ static DirTile dm_tile(const DirStencil& d, int dtype, const int n[3],
             const int rows = std::min(nt / t.tz, n[1]);
             const int nr = (n[1] + rows - 1) / rows;
             t.ty = (n[1] + nr - 1) / nr;
-            const int threads = (t.tz * t.ty + 63) / 64 * 64;
+            t.threads = (t.tz * t.ty + 63) / 64 * 64;
             const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
-            if (lsz > 4L * threads) continue;
-            const int hm = lsz <= 2L * threads ? 2 : 4;
-            const int waves = threads / 64;
+            if (pad) t.threads = std::max(t.threads,
+                                          (int)((lsz + 255) / 256 * 64));
+            if (lsz > 4L * t.threads || t.threads > DM_THREADS) continue;
+            const int hm = lsz <= 2L * t.threads ? 2 : 4;
+            const int waves = t.threads / 64;
             const int es = dtype == 1 ? 16 : dtype == 2 ? 4 : 8;
             const double lines = (t.ty + 2 * R) *
                                  ((t.tz + 2 * R) * es / 128.0 + 1.0) /
@@ -143,7 +149,17 @@ static DirTile dm_tile(const DirStencil& d, int dtype, const int n[3],
             }
         }
     }
-    return best;
+    return least < 1e300;
+}
+
+DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin)
+{
+    DirTile t{};
+    // At R = 4 the halo of a few short rows (4 of 14 to 16 points, 5 of 12)
+    // is more than four points for each thread of their only tile.
+    if (!dm_search(d, dtype, n, nin, false, t))
+        dm_search(d, dtype, n, nin, true, t);
+    return t;
 }
 
 bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi)
@@ -166,8 +182,8 @@ bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi)
 long dirmarch_max_blocks(const DirStencil& d, int dtype, const int n[3],
                          long nin)
 {
-    if (d.R < 1) return 0;
-    const DirTile t = dm_tile(d, dtype, n, nin);
+    if (d.R < 1 || std::min({n[0], n[1], n[2]}) < d.R) return 0;
+    const DirTile t = dir_tile(d, dtype, n, nin);
     return (long)ceil_div(n[2], t.tz) * ceil_div(n[1], t.ty) *
            ceil_div(n[0], t.xchunk) * nin;
 }
@@ -177,13 +193,12 @@ int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
                     int epi, const EpiArgs& ea, hipStream_t s,
                     int* nblocks_out)
 {
-    DirTile t = dm_tile(d, dtype, n, nin);
+    DirTile t = dir_tile(d, dtype, n, nin);
     if (!ea.partial) {
         std::lock_guard<std::mutex> lk(g_dm_mu);
         const DirTile& o = g_dm_tile;
-        const int threads = (o.tz * o.ty + 63) / 64 * 64;
-        if (g_dm_override && threads <= DM_THREADS &&
-            (o.tz + 2 * d.R) * (o.ty + 2 * d.R) <= 4 * threads)
+        if (g_dm_override && o.threads <= DM_THREADS &&
+            (o.tz + 2 * d.R) * (o.ty + 2 * d.R) <= 4 * o.threads)
             t = o;
     }
     switch (dtype) {
@@ -197,3 +212,26 @@ int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
 }
 
 }  // namespace gfd
+
+extern "C" int gfd_march_tile(int npoints, const double* coefs,
+                              const int* offsets, const int n[3], int dtype,
+                              long nin, int tile[4])
+{
+    if (!coefs || !offsets || !n || !tile || npoints < 1 || nin < 1 ||
+        dtype < 0 || dtype > 3 || n[0] < 1 || n[1] < 1 || n[2] < 1) {
+        gfd::set_error("gfd_march_tile: bad arguments");
+        return gfd::EINVAL_;
+    }
+    gfd::DirStencil d;
+    if (!gfd::dir_stencil(npoints, coefs, offsets, d) ||
+        !gfd::dirmarch_fits(d, dtype, n, gfd::EPI_PLAIN)) {
+        gfd::set_error("gfd_march_tile: not for the direction march");
+        return gfd::ENOTSUP_;
+    }
+    const gfd::DirTile t = gfd::dir_tile(d, dtype, n, nin);
+    tile[0] = t.tz;
+    tile[1] = t.ty;
+    tile[2] = t.xchunk;
+    tile[3] = t.threads;
+    return gfd::OK;
+}

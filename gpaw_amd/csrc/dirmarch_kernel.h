@@ -333,10 +333,11 @@ static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
     a.xchunk = t.xchunk;
     a.chunks_x = ceil_div(n[0], t.xchunk);
     const long nb = (long)a.tiles_z * a.tiles_y * a.chunks_x * nin;
-    const int threads = (t.tz * t.ty + 63) / 64 * 64;
+    const int threads = t.threads;
     const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
     if (nb <= 0) return OK;
-    if (nb > 0x7fffffffL || threads > DM_NT || lsz > (long)HM * threads) {
+    if (nb > 0x7fffffffL || threads > DM_NT || threads < t.tz * t.ty ||
+        lsz > (long)HM * threads) {
         set_error("direction march: %ld blocks of %d x %d do not fit", nb,
                   t.ty, t.tz);
         return ENOTSUP_;
@@ -365,9 +366,8 @@ static int dm_launch_h(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
                        int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
 {
-    const int threads = (t.tz * t.ty + 63) / 64 * 64;
     const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
-    if (FULL && lsz <= 2L * threads)
+    if (FULL && lsz <= 2L * t.threads)
         return dm_launch_t<T, R, NI, NM, AUX, 2, FULL, NARROW>(
             d, t, n, bc, in, out, nin, epi, ea, s, nbo);
     return dm_launch_t<T, R, NI, NM, AUX, 4, FULL, NARROW>(

@@ -81,6 +81,15 @@ int gfd_operator_relax(gfd_operator* op, int method, double* f,
  * no such weights exist. */
 int gfd_gs_order(const int* offsets, int npoints, int* a0, int* a1);
 
+/* No counterpart in the reference (host only, no device calls): the tile
+ * with which the direction march runs a stencil of npoints points (offsets
+ * as o0, o1, o2 triples) over nin grids of n points of data type dtype (0
+ * FP64, 1 complex FP64, 2 FP32, 3 complex FP32): columns, rows, planes per
+ * block, threads.  GFD_ENOTSUP when the march does not take the stencil or
+ * the grid. */
+int gfd_march_tile(int npoints, const double* coefs, const int* offsets,
+                   const int n[3], int dtype, long nin, int tile[4]);
+
 /* Replaces Operator.get_diagonal_element() -- c/operators.cpp:319-332. */
 double gfd_operator_get_diagonal_element(const gfd_operator* op);
 

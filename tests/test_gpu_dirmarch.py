@@ -158,3 +158,25 @@ def test_preconditioner(cell, N, pbc, dtype, fp32):
         with path(p):
             outs.append(host(pc(res, kpt)))
     assert relerr(outs[0], outs[1]) < (2e-6 if fp32 else TOL)
+
+
+@pytest.mark.parametrize('N', [(8, 4, 14), (8, 4, 16), (5, 5, 12),
+                               (4, 4, 4), (9, 6, 70)])
+@pytest.mark.parametrize('dtype', [float, complex])
+def test_radius_4(N, dtype):
+    """Planes of a few short rows, whose halo at radius 4 is more than four
+    points per tile point; sides equal to the radius; a z remainder."""
+    rng = np.random.default_rng(4)
+    gd = grid(N, 'box', True)
+    count = 3 if dtype == complex else -(-620_000 // np.prod(N))
+    a = rand(rng, (count,) + N, dtype)
+    ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
+    for op in (Laplace(gd, -0.7, 4, dtype), Gradient(gd, 1, 1.0, 4, dtype)):
+        out = dev(np.zeros_like(a))
+        say('dirmarch radius 4', N, dtype, op.description)
+        for p in (0, 2):
+            with path(p):
+                op.apply(dev(a), out, ph)
+            ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c,
+                                  gd.neighbor_cd, a, ph)
+            assert relerr(host(out), ref) < TOL
