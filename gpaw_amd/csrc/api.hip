@@ -246,7 +246,8 @@ static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
     const bool dir = op->dir_ok && g_force_path != 3 &&
                      dirmarch_fits(op->dir, dtype, op->n, epi);
     if (dir && g_force_path == 2) return 2;
-    if (g_force_path == 0 && op->axis_ok &&
+    // (k_point reads every step of an axis; k_dirmarch only those there are)
+    if (g_force_path == 0 && op->axis_ok && !op->dir.some &&
         point_fits(op->ax, dtype, op->n, nin, epi))
         return 4;
     // Real FP64 just beyond those: 8 x 48^3, nn=3: 8.6 us, full rows 9.5;

@@ -13,9 +13,16 @@ constexpr int DM_NM = 4;  // directions (1, dy, dz) off the x axis
 // directions do not fit the registers)
 constexpr int DM_RSKEW = 3;
 
+// What a stencil has on a line: no points, points at every step 1..R on both
+// sides, or some of them (bits k - 1 of `has` for +k, MAXR_FAST + k - 1 for
+// -k).  A point that is not there is not read: multiplied by zero it would
+// turn an infinity into NaN.
+enum DirOn : int { DIR_NONE = 0, DIR_ALL = 1, DIR_SOME = 2 };
+
 // in(x + k d) has coefficient p[k - 1], in(x - k d) m[k - 1], k = 1..R
 struct DirLine {
-    int on;      // the stencil has points on it
+    int on;      // DirOn
+    unsigned has;
     int dy, dz;
     double p[MAXR_FAST], m[MAXR_FAST];
 };
@@ -23,7 +30,8 @@ struct DirLine {
 struct DirStencil {
     int R = 0;
     int ni = 2, nm = 0;  // in-plane / mixed directions
-    int full = 0;  // x and the ni, nm directions all there, p[k] = m[k]
+    int full = 0;  // x and the ni, nm directions all DIR_ALL, p[k] = m[k]
+    int some = 0;  // one of them is DIR_SOME
     DirLine x, in[DM_NI], mix[DM_NM];
 };
 

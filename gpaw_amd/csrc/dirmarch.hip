@@ -12,7 +12,6 @@ bool dir_stencil(int P, const double* coef, const int* off, DirStencil& d)
     d = DirStencil{};
     d.in[0].dz = 1;
     d.in[1].dy = 1;
-    bool seen[1 + DM_NI + DM_NM][2 * MAXR_FAST + 1] = {};
     int ncentre = 0;
     for (int q = 0; q < P; q++) {
         const int* o = off + 3 * q;
@@ -34,37 +33,38 @@ bool dir_stencil(int P, const double* coef, const int* off, DirStencil& d)
             if (v[c] != 0) sg = v[c];
         for (int c = 0; c < 3; c++) v[c] *= sg;
         DirLine* line = nullptr;
-        int id = -1;
         if (v[0] != 0 && v[1] == 0 && v[2] == 0) {
             line = &d.x;
-            id = 0;
         } else {
             DirLine* set = v[0] ? d.mix : d.in;
             int& n = v[0] ? d.nm : d.ni;
             const int most = v[0] ? DM_NM : DM_NI;
             for (int i = 0; i < n && !line; i++)
-                if (set[i].dy == v[1] && set[i].dz == v[2]) {
-                    line = set + i;
-                    id = 1 + i + (v[0] ? DM_NI : 0);
-                }
+                if (set[i].dy == v[1] && set[i].dz == v[2]) line = set + i;
             if (!line) {
                 if (n == most) return false;
                 line = set + n;
                 line->dy = v[1];
                 line->dz = v[2];
-                id = 1 + n + (v[0] ? DM_NI : 0);
                 n++;
             }
         }
-        line->on = 1;
-        bool& s = seen[id][MAXR_FAST + sg * k];
-        if (s) return false;
-        s = true;
+        const unsigned bit = 1u << (k - 1 + (sg > 0 ? 0 : MAXR_FAST));
+        if (line->has & bit) return false;
+        line->has |= bit;
         (sg > 0 ? line->p : line->m)[k - 1] = coef[q];
         d.R = std::max(d.R, k);
     }
+    const unsigned side = (1u << d.R) - 1, all = side | side << MAXR_FAST;
+    auto mark = [&](DirLine& l) {
+        l.on = !l.has ? DIR_NONE : l.has == all ? DIR_ALL : DIR_SOME;
+        d.some |= l.on == DIR_SOME;
+    };
+    mark(d.x);
+    for (DirLine& l : d.in) mark(l);
+    for (DirLine& l : d.mix) mark(l);
     auto full = [](const DirLine& l) {
-        return l.on && std::equal(l.p, l.p + MAXR_FAST, l.m);
+        return l.on == DIR_ALL && std::equal(l.p, l.p + MAXR_FAST, l.m);
     };
     d.full = full(d.x) && std::all_of(d.in, d.in + d.ni, full) &&
              std::all_of(d.mix, d.mix + d.nm, full);

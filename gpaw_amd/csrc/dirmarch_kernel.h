@@ -186,6 +186,10 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     auto cm = [](const DirLine& l, int k) {
         return (S)(FULL ? l.p[k - 1] : l.m[k - 1]);
     };
+    // the point k steps along l is there (k < 0: behind)
+    auto has = [](const DirLine& l, int k) {
+        return (l.has >> (k > 0 ? k - 1 : MAXR_FAST - k - 1) & 1u) != 0;
+    };
     S shift = (S)0;
     if constexpr (AUX == DM_POT)
         if (a.shift) shift = -(S)a.shift[b];
@@ -232,49 +236,50 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
             cfor<R>([&](auto j) { vq[j] = vq[j + 1]; });
             vq[R] = v;
             T mid = at(here);
-            // (a direction without points is skipped, not multiplied by
-            // zeros: its neighbours may hold infinities)
-            if (FULL || a.st.in[0].on) {
+            // in-plane direction l with its points o elements apart
+            auto inplane = [&](const DirLine& l, int o) {
+                if (FULL || l.on == DIR_ALL) {
 #pragma unroll
-                for (int k = 1; k <= R; k++) {
-                    mid = fmac(mid, (S)a.st.in[0].p[k - 1], p[k]);
-                    mid = fmac(mid, cm(a.st.in[0], k), p[-k]);
+                    for (int k = 1; k <= R; k++) {
+                        mid = fmac(mid, (S)l.p[k - 1], p[k * o]);
+                        mid = fmac(mid, cm(l, k), p[-k * o]);
+                    }
+                } else if (l.on != DIR_NONE) {
+#pragma unroll
+                    for (int k = 1; k <= R; k++) {
+                        if (has(l, k)) mid = fmac(mid, (S)l.p[k - 1], p[k * o]);
+                        if (has(l, -k)) mid = fmac(mid, cm(l, k), p[-k * o]);
+                    }
                 }
-            }
+            };
+            inplane(a.st.in[0], 1);
 #pragma unroll
-            for (int i = 1; i < NI; i++) {
-                if (!FULL && !a.st.in[i].on) continue;
-                const int o = i == 1 ? LW
-                                     : a.st.in[i].dy * LW + a.st.in[i].dz;
-#pragma unroll
-                for (int k = 1; k <= R; k++) {
-                    mid = fmac(mid, (S)a.st.in[i].p[k - 1], p[k * o]);
-                    mid = fmac(mid, cm(a.st.in[i], k), p[-k * o]);
-                }
-            }
+            for (int i = 1; i < NI; i++)
+                inplane(a.st.in[i],
+                        i == 1 ? LW : a.st.in[i].dy * LW + a.st.in[i].dz);
             at(here) = mid;
-            // the point k steps ahead of output x - k, behind output x + k
-            if (FULL || a.st.x.on)
-                cfor<R>([&](auto k0) {
+            // direction l off the x axis: the point k steps ahead of output
+            // x - k, behind output x + k
+            auto across = [&](const DirLine& l, auto&& point) {
+                auto step = [&](auto all, auto k0) {
                     constexpr int k = k0 + 1;
                     std::integral_constant<int, -k> ahead;
                     std::integral_constant<int, k> behind;
-                    at(ahead) = fmac(at(ahead), (S)a.st.x.p[k - 1], v);
-                    at(behind) = fmac(at(behind), cm(a.st.x, k), v);
-                });
+                    if (all || has(l, k))
+                        at(ahead) = fmac(at(ahead), (S)l.p[k - 1], point(k));
+                    if (all || has(l, -k))
+                        at(behind) = fmac(at(behind), cm(l, k), point(-k));
+                };
+                if (FULL || l.on == DIR_ALL)
+                    cfor<R>([&](auto k) { step(std::true_type{}, k); });
+                else if (l.on != DIR_NONE)
+                    cfor<R>([&](auto k) { step(std::false_type{}, k); });
+            };
+            across(a.st.x, [&](int) { return v; });
 #pragma unroll
             for (int i = 0; i < NM; i++) {
-                if (!FULL && !a.st.mix[i].on) continue;
                 const int o = a.st.mix[i].dy * LW + a.st.mix[i].dz;
-                cfor<R>([&](auto k0) {
-                    constexpr int k = k0 + 1;
-                    std::integral_constant<int, -k> ahead;
-                    std::integral_constant<int, k> behind;
-                    at(ahead) = fmac(at(ahead), (S)a.st.mix[i].p[k - 1],
-                                     p[k * o]);
-                    at(behind) = fmac(at(behind), cm(a.st.mix[i], k),
-                                      p[-k * o]);
-                });
+                across(a.st.mix[i], [&](int k) { return p[k * o]; });
             }
             // output plane x - R is complete (before the chunk: not stored)
             const int xo = x - R;

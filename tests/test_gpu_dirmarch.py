@@ -91,6 +91,39 @@ def test_infinities_stay_on_their_lines():
     assert bad[4, 4].all() and bad.sum() == 12
 
 
+def both(*steps):
+    """Each offset and its opposite."""
+    return [(0, 0, 0)] + [o for s in steps
+                          for o in (s, tuple(-i for i in s))]
+
+
+@pytest.mark.parametrize('offsets', [
+    # one side of a diagonal, the first step left out
+    [(0, 0, 0), (0, 2, 2)], [(0, 0, 0), (2, 2, 0), (-1, 0, 1)],
+    # equal coefficients, one line shorter than the others
+    both((1, 0, 0), (0, 1, 0), (0, 2, 0), (0, 0, 1), (0, 0, 2)),
+    both((1, 0, 0), (2, 0, 0), (0, 1, 0), (0, 2, 0), (0, 0, 1), (0, 0, 2),
+         (1, 1, 0))])
+@pytest.mark.parametrize('pbc', [True, False])
+def test_infinities_on_partly_filled_lines(offsets, pbc):
+    """Points that a line does not have are not read: an infinity there
+    leaves the sum finite."""
+    rng = np.random.default_rng(6)
+    gd = grid((9, 11, 15), 'box', pbc)
+    op = FDOperator([1.0] + [0.5] * (len(offsets) - 1), offsets, gd)
+    a = rand(rng, (2,) + tuple(gd.n_c))
+    a[rng.random(a.shape) < 0.02] = np.inf
+    out = dev(np.zeros_like(a))
+    with path(2):
+        op.apply(dev(a), out)
+    ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a)
+    got, fin = host(out), np.isfinite(ref)
+    assert 0 < (~fin).sum() < 0.5 * fin.size
+    assert (np.isfinite(got) == fin).all()
+    assert (np.isnan(got) == np.isnan(ref)).all()
+    assert relerr(got[fin], ref[fin]) < TOL
+
+
 @pytest.mark.parametrize('cell,N,pbc', [('box', (14, 23, 47), False),
                                         ('hex', (12, 12, 21), True)])
 def test_epilogues(cell, N, pbc):
