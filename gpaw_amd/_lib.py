@@ -41,7 +41,8 @@ SIGNATURES = {
     'gfd_operator_residual_noalloc': (_i, [_vp, _vp, _vp, _vp, _l, _dp, _dp,
                                            _vp]),
     'gfd_operator_residual_noalloc_max_blocks': (_l, []),
-    'gfd_march_tile': (_i, [_i, _dp, _ip, _ip, _i, _l, _ip]),
+    'gfd_march_tile': (_i, [_i, _dp, _ip, _ip, _i, _l, _i, _ip]),
+    'gfd_operator_family': (_i, [_vp, _i, _l, _i]),
     'gfd_gs_order': (_i, [_ip, _i, _ip, _ip]),
     'gfd_transformer_new': (_i, [_lp, _lp, _i, _lp, _lp, _lp, _lp, _i, _i,
                                  ctypes.POINTER(_vp)]),

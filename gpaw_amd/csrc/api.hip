@@ -237,6 +237,25 @@ static bool aligned16(const void* p)
     return ((uintptr_t)p & 15) == 0;
 }
 
+// Whether the direction march is the first choice of a complex FP64 pass.
+// k_xrow holds 2R + 2 planes of 16-byte points in registers (2 waves per
+// SIMD at R = 3).  Its time over the march's, 1, 4 and 32 grids of 48^3,
+// 96^3, 128^3 and 64x100x180: Laplacians' H psi 1.11-1.84 at R = 3, 1.26-4.1
+// at R = 4, 1.11-1.57 at R = 2, 0.99-1.72 at R = 1; plain passes 1.03-1.70 at
+// R = 3, 1.06-4.1 at R = 4, but 0.92-1.20 below.  Gradients, 1 to 217 grids
+// of 24^3 .. 128^3, 30x64x140, 47^3 and 63x81x95: along y and z 1.02-4.2 from
+// R = 3 on; along x k_xrow reads no halo either, 0.89-1.2 over even rows from
+// a million points up, 1.1-2.4 over odd ones.  Any other stencil runs in the
+// general form of the march, at 0.4-0.8 of k_xrow's rate.
+static bool march_first(const gfd_operator* op, int epi)
+{
+    const DirStencil& d = op->dir;
+    const int line = dir_line(d, epi);
+    if (d.full && epi == EPI_POT) return true;
+    return d.R >= 3 && (d.full || line > 0 ||
+                        (line == 0 && op->n[2] % 2 != 0));
+}
+
 // Kernel family for one pass: 4 one point per thread, 3 full-row, 2 direction
 // march, 1 general.
 static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
@@ -250,17 +269,14 @@ static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
     if (g_force_path == 0 && op->axis_ok && !op->dir.some &&
         point_fits(op->ax, dtype, op->n, nin, epi))
         return 4;
-    // Real FP64 just beyond those: 8 x 48^3, nn=3: 8.6 us, full rows 9.5;
-    // 96^3 8.8 / 9.5; but 4 x 64^3 9.1 / 8.8, 2 x 96^3 11.4 / 11.5.
-    if (dir && dtype == 0 && (double)op->ng() * nin <= 900e3) return 2;
-    // Complex FP64: the direction march from radius 3 on and for H psi at
-    // any radius.  k_xrow holds 2R + 2 planes of 16-byte points in registers
-    // (2 waves per SIMD at R = 3); measured over 1, 4 and 32 grids of 48^3,
-    // 96^3, 128^3 and 64x100x180, its time over the march's: H psi 1.11-1.84
-    // at R = 3, 1.26-4.1 at R = 4, 1.11-1.57 at R = 2, 0.99-1.72 at R = 1;
-    // plain passes 1.03-1.70 at R = 3, 1.06-4.1 at R = 4, but 0.92-1.20
-    // below.  Real data: 0.70-1.10 (plain), so the full rows stay first.
-    if (dir && dtype == 1 && (op->dir.R >= 3 || epi == EPI_POT)) return 2;
+    // Real FP64 Laplacians of radius 3 beyond those limits: 29 batches of 24^3
+    // to 100^3 points, 0.6 to 0.9 million in all, take 0.86-0.96 of the full
+    // rows' time with inputs in rotation, 0.90-1.05 repeated on one; radius 1,
+    // 2 and 4 0.90-1.10.  (8 x 48^3, whole calls: 9.3 us, rows 9.7.)
+    if (dir && dtype == 0 && op->dir.full && op->dir.R == 3 &&
+        (double)op->ng() * nin <= 900e3)
+        return 2;
+    if (dir && dtype == 1 && march_first(op, epi)) return 2;
     if (op->axis_ok && g_force_path != 2 && aligned16(in) &&
         aligned16(out) && (aux == nullptr || aligned16(aux)) &&
         row_stencil_fits(op->ax, dtype, op->n, nin))
@@ -286,6 +302,17 @@ static int op_pass(gfd_operator* op, int dtype, const void* in, void* out,
                                ea, s, nblocks);
     return launch_general_stencil(op->gen(ea.c0), dtype, op->n, bc, in, out,
                                   nin, epi, ea, s, nblocks);
+}
+
+extern "C" int gfd_operator_family(gfd_operator* op, int dtype, long nin,
+                                   int epilogue)
+{
+    if (!op || dtype < 0 || dtype > 3 || nin < 1 || epilogue < EPI_PLAIN ||
+        epilogue > EPI_RESN) {
+        set_error("gfd_operator_family: bad arguments");
+        return -1;
+    }
+    return op_path(op, dtype, nin, nullptr, nullptr, nullptr, epilogue);
 }
 
 // Upper bound of the blocks a residual pass may launch (partial sums).

@@ -32,6 +32,7 @@ struct DirStencil {
     int ni = 2, nm = 0;  // in-plane / mixed directions
     int full = 0;  // x and the ni, nm directions all DIR_ALL, p[k] = m[k]
     int some = 0;  // one of them is DIR_SOME
+    int line = -1; // the axis of a stencil of one DIR_ALL axis line
     DirLine x, in[DM_NI], mix[DM_NM];
 };
 
@@ -61,8 +62,27 @@ struct DirTile {
     int tz, ty, xchunk, threads;
 };
 
+// Widths of what a block stages beyond its points along y and z, and of the
+// planes it marches through beyond its chunk.
+struct DirHalo {
+    int x, y, z;
+};
+
+// A plain pass of a stencil on one axis reads along that axis only (the
+// other epilogues run it in the general form).
+constexpr DirHalo dir_halo(int R, int line)
+{
+    return {line < 1 ? R : 0, line < 0 || line == 1 ? R : 0,
+            line < 0 || line == 2 ? R : 0};
+}
+inline int dir_line(const DirStencil& d, int epi)
+{
+    return epi == EPI_PLAIN ? d.line : -1;
+}
+
 // The tile with the least estimated time; every grid of sides >= R has one.
-DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin);
+DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin,
+                 int epi);
 
 int dirmarch_f64(const DirStencil& d, const DirTile& t, const int n[3],
                  const BC& bc, const void* in, void* out, long nin, int epi,

@@ -63,6 +63,9 @@ bool dir_stencil(int P, const double* coef, const int* off, DirStencil& d)
     mark(d.x);
     for (DirLine& l : d.in) mark(l);
     for (DirLine& l : d.mix) mark(l);
+    if (!d.some && d.ni == 2 && d.nm == 0 &&
+        (d.x.on != 0) + (d.in[0].on != 0) + (d.in[1].on != 0) == 1)
+        d.line = d.x.on ? 0 : d.in[1].on ? 1 : 2;
     auto full = [](const DirLine& l) {
         return l.on == DIR_ALL && std::equal(l.p, l.p + MAXR_FAST, l.m);
     };
@@ -102,9 +105,10 @@ void dirmarch_set_tile(const XmTile* t)
 // four 64).
 // pad: blocks of more threads than tile points, enough to stage the halo.
 static bool dm_search(const DirStencil& d, int dtype, const int n[3],
-                      long nin, bool pad, DirTile& best)
+                      long nin, int epi, bool pad, DirTile& best)
 {
     const int R = d.R;
+    const DirHalo h = dir_halo(R, dir_line(d, epi));
     // waves a CU holds: complex FP64 takes about 128 registers at R = 3
     const int hold = dtype == 1 && R > 1 ? 16 : 32;
     double least = 1e300;
@@ -119,15 +123,16 @@ static bool dm_search(const DirStencil& d, int dtype, const int n[3],
             const int nr = (n[1] + rows - 1) / rows;
             t.ty = (n[1] + nr - 1) / nr;
             t.threads = (t.tz * t.ty + 63) / 64 * 64;
-            const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
+            const long lsz = (long)(t.tz + 2 * h.z) * (t.ty + 2 * h.y);
             if (pad) t.threads = std::max(t.threads,
                                           (int)((lsz + 255) / 256 * 64));
             if (lsz > 4L * t.threads || t.threads > DM_THREADS) continue;
-            const int hm = lsz <= 2L * t.threads ? 2 : 4;
+            const int hm = lsz <= t.threads ? 1 : lsz <= 2L * t.threads ? 2
+                                                                        : 4;
             const int waves = t.threads / 64;
             const int es = dtype == 1 ? 16 : dtype == 2 ? 4 : 8;
-            const double lines = (t.ty + 2 * R) *
-                                 ((t.tz + 2 * R) * es / 128.0 + 1.0) /
+            const double lines = (t.ty + 2 * h.y) *
+                                 ((t.tz + 2 * h.z) * es / 128.0 + 1.0) /
                                  (t.tz * t.ty * es / 128.0);
             const long tiles = (long)parts * nr * nin;
             for (int chunks = 1; chunks <= std::max(1, n[0] / 4);
@@ -137,7 +142,7 @@ static bool dm_search(const DirStencil& d, int dtype, const int n[3],
                     (tiles * ((n[0] + t.xchunk - 1) / t.xchunk) + 255) / 256;
                 const double resident =
                     std::min<long>(per, std::max(1, hold / waves)) * waves;
-                const double cost = (double)(t.xchunk + 2 * R) * per * waves *
+                const double cost = (double)(t.xchunk + 2 * h.x) * per * waves *
                                     (1.0 + 0.12 * hm) *
                                     (1.0 + 4.0 / resident) *
                                     (1.0 + 0.2 * lines);
@@ -152,13 +157,14 @@ static bool dm_search(const DirStencil& d, int dtype, const int n[3],
     return least < 1e300;
 }
 
-DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin)
+DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin,
+                 int epi)
 {
     DirTile t{};
     // At R = 4 the halo of a few short rows (4 of 14 to 16 points, 5 of 12)
     // is more than four points for each thread of their only tile.
-    if (!dm_search(d, dtype, n, nin, false, t))
-        dm_search(d, dtype, n, nin, true, t);
+    if (!dm_search(d, dtype, n, nin, epi, false, t))
+        dm_search(d, dtype, n, nin, epi, true, t);
     return t;
 }
 
@@ -183,7 +189,7 @@ long dirmarch_max_blocks(const DirStencil& d, int dtype, const int n[3],
                          long nin)
 {
     if (d.R < 1 || std::min({n[0], n[1], n[2]}) < d.R) return 0;
-    const DirTile t = dir_tile(d, dtype, n, nin);
+    const DirTile t = dir_tile(d, dtype, n, nin, EPI_RESID);
     return (long)ceil_div(n[2], t.tz) * ceil_div(n[1], t.ty) *
            ceil_div(n[0], t.xchunk) * nin;
 }
@@ -193,7 +199,7 @@ int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
                     int epi, const EpiArgs& ea, hipStream_t s,
                     int* nblocks_out)
 {
-    DirTile t = dir_tile(d, dtype, n, nin);
+    DirTile t = dir_tile(d, dtype, n, nin, epi);
     if (!ea.partial) {
         std::lock_guard<std::mutex> lk(g_dm_mu);
         const DirTile& o = g_dm_tile;
@@ -215,7 +221,7 @@ int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
 
 extern "C" int gfd_march_tile(int npoints, const double* coefs,
                               const int* offsets, const int n[3], int dtype,
-                              long nin, int tile[4])
+                              long nin, int plain, int tile[4])
 {
     if (!coefs || !offsets || !n || !tile || npoints < 1 || nin < 1 ||
         dtype < 0 || dtype > 3 || n[0] < 1 || n[1] < 1 || n[2] < 1) {
@@ -228,7 +234,9 @@ extern "C" int gfd_march_tile(int npoints, const double* coefs,
         gfd::set_error("gfd_march_tile: not for the direction march");
         return gfd::ENOTSUP_;
     }
-    const gfd::DirTile t = gfd::dir_tile(d, dtype, n, nin);
+    const gfd::DirTile t =
+        gfd::dir_tile(d, dtype, n, nin, plain ? gfd::EPI_PLAIN
+                                              : gfd::EPI_RESID);
     tile[0] = t.tz;
     tile[1] = t.ty;
     tile[2] = t.xchunk;

@@ -75,13 +75,20 @@ enum DmAux : int { DM_NONE = 0, DM_SAME = 1, DM_POT = 2, DM_WIDE = 3 };
 
 // AUX: DmAux.  HM: staged elements per thread.  NARROW: FP64 input, result
 // stored as FP32 (EPI_RESN).
-// FULL: every direction of the form is there with equal coefficients on
-// both sides of the centre (a Laplacian).  Then nothing is tested in the
-// plane loop, whose many scalar tests and branches were what bound the
-// first version (142 scalar instructions, 20 of them branches, beside 38
-// vector ones per plane), and one copy of the coefficients stays in scalar
-// registers.
-template <typename T, int R, int NI, int NM, int AUX, int HM, bool FULL,
+// FORM:
+//   DM_FULL: every direction of the form is there with equal coefficients on
+//     both sides of the centre (a Laplacian).  Then nothing is tested in the
+//     plane loop, whose many scalar tests and branches were what bound the
+//     first version (142 scalar instructions, 20 of them branches, beside 38
+//     vector ones per plane), and one copy of the coefficients stays in
+//     scalar registers.
+//   DM_LINE + axis: that axis line alone (a gradient).  Along x nothing is
+//     staged: a thread's own column is all it reads.  Along y or z a plane
+//     stands by itself, with a halo on that axis only.
+//   DM_GENERAL: any set of directions, each tested per plane.
+enum DmForm : int { DM_GENERAL = 0, DM_FULL = 1, DM_LINE = 2 };
+
+template <typename T, int R, int NI, int NM, int AUX, int HM, int FORM,
           bool NARROW>
 __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
 {
@@ -93,7 +100,10 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     typedef typename std::conditional<
         NARROW, float,
         typename std::conditional<AUX == DM_WIDE, WT, T>::type>::type TO;
-    constexpr int U = 2 * R + 1;
+    constexpr bool FULL = FORM == DM_FULL;
+    constexpr int LINE = FORM < DM_LINE ? -1 : FORM - DM_LINE;
+    constexpr DirHalo H = dir_halo(R, LINE);
+    constexpr int U = 2 * H.x + 1;
     constexpr bool CPLX = IsCplx<T>::value;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* lds = reinterpret_cast<T*>(smem_raw);
@@ -113,7 +123,7 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     const unsigned plane = (unsigned)n1 * (unsigned)n2;
     const int z0 = zt * a.tz, y0 = yt * a.ty;
     const int xs = cx * a.xchunk, xe = min(xs + a.xchunk, n0);
-    const int LW = a.tz + 2 * R, LSZ = (a.ty + 2 * R) * LW;
+    const int LW = a.tz + 2 * H.z, LSZ = (a.ty + 2 * H.y) * LW;
     const int buf1 = HM * NT;  // elements of one buffer (LSZ at most)
     const BC& bc = a.bc;
 
@@ -130,9 +140,9 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
         hf[m] = make_double2(1.0, 0.0);
         if (e < LSZ) {
             const int row = e / LW;
-            int y = y0 + row - R, z = z0 + (e - row * LW) - R;
+            int y = y0 + row - H.y, z = z0 + (e - row * LW) - H.z;
             // beyond the halo of the last row or column: never read
-            if (y < n1 + R && z < n2 + R &&
+            if (y < n1 + H.y && z < n2 + H.z &&
                 wrap_full(z, n2, bc.periodic[2], bc.phase[2][0],
                           bc.phase[2][1], hf[m], hph[m]) &&
                 wrap_full(y, n1, bc.periodic[1], bc.phase[1][0],
@@ -143,7 +153,7 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     // own point
     const int tr = tid / a.tz, tc = tid - tr * a.tz;
     const bool on = tr < a.ty && y0 + tr < n1 && z0 + tc < n2;
-    const int lown = (min(tr, a.ty - 1) + R) * LW + tc + R;
+    const int lown = (min(tr, a.ty - 1) + H.y) * LW + tc + H.z;
     const unsigned oidx = (unsigned)((y0 + tr) * n2 + z0 + tc);
     const unsigned ooff = on ? oidx * (unsigned)sizeof(TO) : BXM_OOB;
     const unsigned aoff = on ? oidx * (unsigned)sizeof(TA) : BXM_OOB;
@@ -197,48 +207,50 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
     T acc[U];
 #pragma unroll
     for (int j = 0; j < U; j++) acc[j] = zero_of<T>();
-    T vq[R + 1];  // centre values of planes x - R .. x
+    T vq[H.x + 1];  // centre values of planes x - H.x .. x
 #pragma unroll
-    for (int j = 0; j <= R; j++) vq[j] = zero_of<T>();
+    for (int j = 0; j <= H.x; j++) vq[j] = zero_of<T>();
     double nrm = 0.0;
 
-    ld_plane(xs - R);
+    ld_plane(xs - H.x);
     ld_aux(xs);
     int cur = 0;
-    for (int xb = xs - R; xb < xe + R; xb += U) {
+    for (int xb = xs - H.x; xb < xe + H.x; xb += U) {
         cfor<U>([&](auto uc) {
             constexpr int u = uc;
             const int x = xb + u;
-            if (x >= xe + R) return;
+            if (x >= xe + H.x) return;
             T* buf = lds + cur;
             cur = buf1 - cur;
+            T v;
 #pragma unroll
             for (int m = 0; m < HM; m++) {
-                T v = hv[m];
+                v = hv[m];
                 if constexpr (CPLX) {
                     if (hph[m]) v = scale_by<T>(v, hf[m], true);
                     if (phx) v = scale_by<T>(v, fx, true);
                 }
-                buf[tid + m * NT] = v;
+                if constexpr (LINE != 0) buf[tid + m * NT] = v;
             }
-            ld_plane(min(x + 1, xe + R - 1));
-            __syncthreads();
+            ld_plane(min(x + 1, xe + H.x - 1));
+            if constexpr (LINE != 0) __syncthreads();
 
-            // accumulator of output plane x + j: (u + R + j) mod U
+            // accumulator of output plane x + j: (u + H.x + j) mod U
             auto at = [&](auto j) -> T& {
-                constexpr int i = (u + R + decltype(j)::value + U) % U;
+                constexpr int i = (u + H.x + decltype(j)::value + U) % U;
                 return acc[i];
             };
             constexpr std::integral_constant<int, 0> here;
-            constexpr std::integral_constant<int, -R> oldest;
+            constexpr std::integral_constant<int, -H.x> oldest;
             const T* p = buf + lown;
-            const T v = p[0];
-            cfor<R>([&](auto j) { vq[j] = vq[j + 1]; });
-            vq[R] = v;
+            // (along x the one staged point is the thread's own)
+            if constexpr (LINE != 0) v = p[0];
+            cfor<H.x>([&](auto j) { vq[j] = vq[j + 1]; });
+            vq[H.x] = v;
             T mid = at(here);
             // in-plane direction l with its points o elements apart
             auto inplane = [&](const DirLine& l, int o) {
-                if (FULL || l.on == DIR_ALL) {
+                if (FORM != DM_GENERAL || l.on == DIR_ALL) {
 #pragma unroll
                     for (int k = 1; k <= R; k++) {
                         mid = fmac(mid, (S)l.p[k - 1], p[k * o]);
@@ -252,11 +264,11 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
                     }
                 }
             };
-            inplane(a.st.in[0], 1);
+            if constexpr (LINE < 0 || LINE == 2) inplane(a.st.in[0], 1);
+            if constexpr (LINE < 0 || LINE == 1) inplane(a.st.in[1], LW);
 #pragma unroll
-            for (int i = 1; i < NI; i++)
-                inplane(a.st.in[i],
-                        i == 1 ? LW : a.st.in[i].dy * LW + a.st.in[i].dz);
+            for (int i = 2; i < NI; i++)
+                inplane(a.st.in[i], a.st.in[i].dy * LW + a.st.in[i].dz);
             at(here) = mid;
             // direction l off the x axis: the point k steps ahead of output
             // x - k, behind output x + k
@@ -270,19 +282,19 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
                     if (all || has(l, -k))
                         at(behind) = fmac(at(behind), cm(l, k), point(-k));
                 };
-                if (FULL || l.on == DIR_ALL)
+                if (FORM != DM_GENERAL || l.on == DIR_ALL)
                     cfor<R>([&](auto k) { step(std::true_type{}, k); });
                 else if (l.on != DIR_NONE)
                     cfor<R>([&](auto k) { step(std::false_type{}, k); });
             };
-            across(a.st.x, [&](int) { return v; });
+            if constexpr (LINE < 1) across(a.st.x, [&](int) { return v; });
 #pragma unroll
             for (int i = 0; i < NM; i++) {
                 const int o = a.st.mix[i].dy * LW + a.st.mix[i].dz;
                 across(a.st.mix[i], [&](int k) { return p[k * o]; });
             }
-            // output plane x - R is complete (before the chunk: not stored)
-            const int xo = x - R;
+            // output plane x - H.x is complete (before the chunk: not stored)
+            const int xo = x - H.x;
             T r = at(oldest);
             const T vo = vq[0];
             if constexpr (AUX == DM_POT) {
@@ -318,7 +330,7 @@ __global__ void __launch_bounds__(DM_NT) k_dirmarch(DmArgs<T> a)
         if (a.partial) block_sum_store(nrm, a.partial, L);
 }
 
-template <typename T, int R, int NI, int NM, int AUX, int HM, bool FULL,
+template <typename T, int R, int NI, int NM, int AUX, int HM, int FORM,
           bool NARROW>
 static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
@@ -339,7 +351,8 @@ static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
     a.chunks_x = ceil_div(n[0], t.xchunk);
     const long nb = (long)a.tiles_z * a.tiles_y * a.chunks_x * nin;
     const int threads = t.threads;
-    const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
+    constexpr DirHalo H = dir_halo(R, FORM < DM_LINE ? -1 : FORM - DM_LINE);
+    const long lsz = (long)(t.tz + 2 * H.z) * (t.ty + 2 * H.y);
     if (nb <= 0) return OK;
     if (nb > 0x7fffffffL || threads > DM_NT || threads < t.tz * t.ty ||
         lsz > (long)HM * threads) {
@@ -358,35 +371,46 @@ static int dm_launch_t(const DirStencil& d, const DirTile& t, const int n[3],
     a.partial = epi == EPI_RESID || epi == EPI_RESN ? ea.partial : nullptr;
     a.shift = ea.shift;
     (void)hipGetLastError();
-    hipLaunchKernelGGL((k_dirmarch<T, R, NI, NM, AUX, HM, FULL, NARROW>),
+    hipLaunchKernelGGL((k_dirmarch<T, R, NI, NM, AUX, HM, FORM, NARROW>),
                        dim3((unsigned)nb), dim3(threads),
-                       2 * (size_t)HM * threads * sizeof(T), s, a);
+                       FORM == DM_LINE
+                           ? 0
+                           : 2 * (size_t)HM * threads * sizeof(T),
+                       s, a);
     GFD_LAUNCH_CHECK();
     if (nbo) *nbo = (int)nb;
     return OK;
 }
 
-template <typename T, int R, int NI, int NM, int AUX, bool FULL, bool NARROW>
+template <typename T, int R, int NI, int NM, int AUX, int FORM, bool NARROW>
 static int dm_launch_h(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
                        int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
 {
-    const long lsz = (long)(t.tz + 2 * R) * (t.ty + 2 * R);
-    if (FULL && lsz <= 2L * t.threads)
-        return dm_launch_t<T, R, NI, NM, AUX, 2, FULL, NARROW>(
-            d, t, n, bc, in, out, nin, epi, ea, s, nbo);
-    return dm_launch_t<T, R, NI, NM, AUX, 4, FULL, NARROW>(
-        d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+#define GFD_DM(HM)                                                          \
+    return dm_launch_t<T, R, NI, NM, AUX, HM, FORM, NARROW>(                \
+        d, t, n, bc, in, out, nin, epi, ea, s, nbo)
+    constexpr DirHalo H = dir_halo(R, FORM < DM_LINE ? -1 : FORM - DM_LINE);
+    const long lsz = (long)(t.tz + 2 * H.z) * (t.ty + 2 * H.y);
+    if constexpr (FORM == DM_LINE) GFD_DM(1);
+    else {
+        if constexpr (FORM != DM_GENERAL || (NM == 0 && R <= DM_RSKEW))
+            if (lsz <= 2L * t.threads) GFD_DM(2);
+        GFD_DM(4);
+    }
+#undef GFD_DM
 }
 
-template <typename T, int R, int NI, int NM, bool FULL>
+template <typename T, int R, int NI, int NM, int FORM>
 static int dm_launch_e(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
                        int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
 {
 #define GFD_DM(AUX, NARROW)                                                 \
-    return dm_launch_h<T, R, NI, NM, AUX, FULL, NARROW>(                    \
+    return dm_launch_h<T, R, NI, NM, AUX, FORM, NARROW>(                    \
         d, t, n, bc, in, out, nin, epi, ea, s, nbo)
+    if constexpr (FORM >= DM_LINE) GFD_DM(DM_NONE, false);  // EPI_PLAIN
+    else
     switch (epi) {
     case EPI_PLAIN: GFD_DM(DM_NONE, false);
     case EPI_RELAX:
@@ -414,20 +438,30 @@ static int dm_launch_r(const DirStencil& d, const DirTile& t, const int n[3],
                        const BC& bc, const void* in, void* out, long nin,
                        int epi, const EpiArgs& ea, hipStream_t s, int* nbo)
 {
-#define GFD_DM(NI, NM, FULL)                                                \
-    return dm_launch_e<T, R, NI, NM, FULL>(d, t, n, bc, in, out, nin, epi,  \
+#define GFD_DM(NI, NM, FORM)                                                \
+    return dm_launch_e<T, R, NI, NM, FORM>(d, t, n, bc, in, out, nin, epi,  \
                                            ea, s, nbo)
+    switch (dir_line(d, epi)) {
+    case 0: GFD_DM(2, 0, DM_LINE);
+    case 1: GFD_DM(2, 0, DM_LINE + 1);
+    case 2: GFD_DM(2, 0, DM_LINE + 2);
+    }
     if (d.full) {
-        if (d.ni == 2 && d.nm == 0) GFD_DM(2, 0, true);
+        if (d.ni == 2 && d.nm == 0) GFD_DM(2, 0, DM_FULL);
         if constexpr (R <= DM_RSKEW) {
-            if (d.ni == 2 && d.nm == 1) GFD_DM(2, 1, true);
-            if (d.ni == 3 && d.nm == 0) GFD_DM(3, 0, true);
-            if (d.ni == 3 && d.nm == 2) GFD_DM(3, 2, true);
+            if (d.ni == 2 && d.nm == 1) GFD_DM(2, 1, DM_FULL);
+            if (d.ni == 3 && d.nm == 0) GFD_DM(3, 0, DM_FULL);
+            if (d.ni == 3 && d.nm == 2) GFD_DM(3, 2, DM_FULL);
         }
     }
-    // anything else: the general form of the directions
-    if constexpr (R <= DM_RSKEW) GFD_DM(3, 4, false);
-    else GFD_DM(2, 0, false);
+    // anything else: the general form of the directions, of the axes for
+    // plain passes that need no more
+    if constexpr (R <= DM_RSKEW)
+        if (d.ni == 2 && d.nm == 0 && epi == EPI_PLAIN)
+            return dm_launch_h<T, R, 2, 0, DM_NONE, DM_GENERAL, false>(
+                d, t, n, bc, in, out, nin, epi, ea, s, nbo);
+    if constexpr (R <= DM_RSKEW) GFD_DM(3, 4, DM_GENERAL);
+    else GFD_DM(2, 0, DM_GENERAL);
 #undef GFD_DM
 }
 

@@ -4,10 +4,12 @@
 // The marching kernels read each value once, but a block walks through its
 // planes one latency after another; on arrays that the caches hold and that
 // fill the chip only a few times over, one load latency for everything is
-// faster (PT_MAX64 in point.h).  k_point issues its 6R + 1 loads at once, with the
+// faster (limits in point.h).  k_point issues its 6R + 1 loads at once, with the
 // wrapped offsets from compares and selects, and has the accumulation order
 // (z, y, x) and the epilogues of the full-row kernel.
 #include "point.h"
+
+#include <algorithm>
 
 #include "stencil_dev.h"
 
@@ -158,10 +160,17 @@ bool point_fits(const AxisStencil& st, int dtype, const int n[3], long nin,
 {
     const bool has = (dtype == 0 && epi != EPI_UPDW) ||
                      (dtype == 2 && epi != EPI_POT && epi != EPI_RESN);
-    return has && st.R >= 1 && st.R <= MAXR_FAST && n[0] >= st.R &&
-           n[1] >= st.R && n[2] >= st.R &&
-           (double)n[0] * n[1] * n[2] * (double)nin <=
-               (dtype == 0 ? PT_MAX64 : PT_MAX32);
+    if (!has || st.R < 1 || st.R > MAXR_FAST || n[0] < st.R ||
+        n[1] < st.R || n[2] < st.R)
+        return false;
+    const bool line = (st.has[0] != 0) + (st.has[1] != 0) +
+                          (st.has[2] != 0) == 1;
+    double most = dtype == 2 ? PT_MAX32
+                  : line     ? PT_MAX64_LINE
+                             : PT_MAX64[st.R - 1];
+    if (!row_stencil_fits(st, dtype, n, nin))
+        most = std::max(most, PT_MAX64_ODD);
+    return (double)n[0] * n[1] * n[2] * (double)nin <= most;
 }
 
 int launch_point(const AxisStencil& st, int dtype, const int n[3],

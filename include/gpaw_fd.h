@@ -71,6 +71,14 @@ int gfd_operator_apply(gfd_operator* op, const void* in, void* out, long nin,
 int gfd_operator_relax(gfd_operator* op, int method, double* f,
                        const double* src, int nrelax, double w, void* stream);
 
+/* No counterpart in the reference (no device calls): the kernel family of
+ * an operator's pass over nin grids at 16-byte aligned addresses, as the
+ * values of the tuning key "force_path", and 4: one point per thread; -1 for
+ * bad arguments.  dtype: 0 FP64, 1 complex FP64, 2 FP32, 3 complex FP32;
+ * epilogue: 0 apply, 1 Jacobi sweep, 2 residual, 3 residual update, 4 H psi,
+ * 5 and 6 update and residual of mixed precision. */
+int gfd_operator_family(gfd_operator* op, int dtype, long nin, int epilogue);
+
 /* No counterpart in the reference (host only, no device calls): the step
  * weights of the Gauss-Seidel sweep of gfd_operator_relax(method 1).  The
  * sweep updates point (i0, i1, i2) at step a0 i0 + a1 i1 + i2; the
@@ -85,10 +93,12 @@ int gfd_gs_order(const int* offsets, int npoints, int* a0, int* a1);
  * with which the direction march runs a stencil of npoints points (offsets
  * as o0, o1, o2 triples) over nin grids of n points of data type dtype (0
  * FP64, 1 complex FP64, 2 FP32, 3 complex FP32): columns, rows, planes per
- * block, threads.  GFD_ENOTSUP when the march does not take the stencil or
+ * block, threads.  plain: of an apply, else of the passes with a residual
+ * or an update.  GFD_ENOTSUP when the march does not take the stencil or
  * the grid. */
 int gfd_march_tile(int npoints, const double* coefs, const int* offsets,
-                   const int n[3], int dtype, long nin, int tile[4]);
+                   const int n[3], int dtype, long nin, int plain,
+                   int tile[4]);
 
 /* Replaces Operator.get_diagonal_element() -- c/operators.cpp:319-332. */
 double gfd_operator_get_diagonal_element(const gfd_operator* op);

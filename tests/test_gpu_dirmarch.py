@@ -59,12 +59,33 @@ def test_laplace(cell, nn, N, pbc, dtype):
     assert relerr(host(out), ref) < TOL
 
 
-@pytest.mark.parametrize('make', [
-    lambda gd: Gradient(gd, 1, 1.0, 3), lambda gd: LaplaceA(gd, 0.3),
-    lambda gd: LaplaceB(gd),
-    lambda gd: FDOperator([1.0, 0.5], [(0, 0, 0), (0, 2, 2)], gd)])
-def test_other_stencils(make):
-    """One axis only, the Mehrstellen pair (edges of the cube), points on
+def both(*steps):
+    """Each offset and its opposite."""
+    return [(0, 0, 0)] + [o for s in steps
+                          for o in (s, tuple(-i for i in s))]
+
+
+def family(op, dtype=0, nin=1, epilogue=0):
+    """Kernel family of a pass (1 general, 2 march, 3 full rows, 4 point)."""
+    return _lib.load().gfd_operator_family(op._handle(), dtype, nin, epilogue)
+
+
+def edges(gd):
+    """Every in-plane and off-axis direction the march holds."""
+    steps = [(0, 0, 1), (0, 1, 0), (0, 1, 1), (1, 0, 0), (1, 1, 0),
+             (1, -1, 0), (1, 0, 1), (1, 0, -1)]
+    off = both(*steps)
+    return FDOperator([-3.0] + [0.1 + 0.2 * i for i in range(1, len(off))],
+                      off, gd)
+
+
+@pytest.mark.parametrize('make,takes', [
+    (lambda gd: Gradient(gd, 1, 1.0, 3), 2), (edges, 2),
+    (lambda gd: LaplaceA(gd, 0.3), 1), (lambda gd: LaplaceB(gd), 2),
+    (lambda gd: FDOperator([1.0, 0.5], [(0, 0, 0), (0, 2, 2)], gd), 2)])
+def test_other_stencils(make, takes):
+    """One axis only; edges of the cube, and one in-plane direction more than
+    the march holds (the Mehrstellen operator: the general kernel); points on
     one side of the centre."""
     rng = np.random.default_rng(3)
     gd = grid((9, 20, 33), 'box', (True, False, True))
@@ -73,9 +94,62 @@ def test_other_stencils(make):
     out = dev(np.zeros_like(a))
     say('dirmarch stencil', op.description)
     with path(2):
+        assert family(op, nin=2) == takes
         op.apply(dev(a), out)
     ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a)
     assert relerr(host(out), ref) < TOL
+
+
+@pytest.mark.parametrize('axis', [0, 1, 2])
+@pytest.mark.parametrize('nn', [1, 2, 3, 4])
+@pytest.mark.parametrize('N,pbc', [((4, 5, 6), True), ((9, 12, 70), False),
+                                   ((21, 37, 16), (False, True, True)),
+                                   ((16, 4, 131), (True, False, False))])
+@pytest.mark.parametrize('dtype', [float, complex])
+def test_gradient(axis, nn, N, pbc, dtype):
+    """One axis: its line alone, over tile remainders and sides down to the
+    radius."""
+    rng = np.random.default_rng(nn)
+    gd = grid(tuple(n + 1 - p for n, p in
+                    zip(N, np.broadcast_to(pbc, 3))), 'box', pbc)
+    op = Gradient(gd, axis, 1.0, nn, dtype)
+    a = rand(rng, (3,) + N, dtype)
+    ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
+    ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a,
+                          ph)
+    say('dirmarch gradient', axis, nn, N, pbc, dtype)
+    for p in (2, 0):
+        out = dev(np.zeros_like(a))
+        with path(p):
+            assert p == 0 or family(op, int(dtype == complex), 3) == 2
+            op.apply(dev(a), out, ph)
+        assert relerr(host(out), ref) < TOL
+
+
+def test_which_kernel():
+    """The rule's lines: few real points, complex Laplacians and gradients,
+    the passes with other epilogues."""
+    even, odd = (grid(N, 'box', True) for N in ((48,) * 3, (47, 48, 49)))
+    for R, most in ((1, 5), (2, 4), (3, 5), (4, 4)):
+        op = Laplace(even, 1.0, R)
+        next = 2 if R == 3 else 3
+        assert [family(op, nin=most + i) for i in (0, 1)] == [4, next]
+        assert [family(op, nin=i) for i in (8, 9)] == [next, 3]
+        op = Gradient(even, 0, 1.0, R)
+        assert [family(op, nin=i) for i in (6, 7)] == [4, 3]
+        op = Laplace(odd, 1.0, R)
+        assert [family(op, nin=i) for i in (5, 8)] == [4, 2]
+        lap = [Laplace(gd, 1.0, R, complex) for gd in (even, odd)]
+        grad = [[Gradient(gd, c, 1.0, R, complex) for c in range(3)]
+                for gd in (even, odd)]
+        want = 2 if R >= 3 else 3
+        assert [family(op, 1) for op in lap] == [want] * 2
+        assert [family(op, 1) for op in grad[0]] == [3, want, want]
+        assert [family(op, 1) for op in grad[1]] == [want] * 3
+        for epilogue in (2, 3, 4):
+            assert family(grad[0][1], 1, 1, epilogue) == 3
+            assert family(lap[0], 1, 1, epilogue) == (
+                2 if epilogue == 4 else want)
 
 
 def test_infinities_stay_on_their_lines():
@@ -89,12 +163,6 @@ def test_infinities_stay_on_their_lines():
         op.apply(dev(a), out)
     bad = ~np.isfinite(host(out)[0])
     assert bad[4, 4].all() and bad.sum() == 12
-
-
-def both(*steps):
-    """Each offset and its opposite."""
-    return [(0, 0, 0)] + [o for s in steps
-                          for o in (s, tuple(-i for i in s))]
 
 
 @pytest.mark.parametrize('offsets', [
