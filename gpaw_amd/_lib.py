@@ -42,6 +42,7 @@ SIGNATURES = {
                                            _vp]),
     'gfd_operator_residual_noalloc_max_blocks': (_l, []),
     'gfd_march_tile': (_i, [_i, _dp, _ip, _ip, _i, _l, _i, _ip]),
+    'gfd_march_tile_searches': (_l, []),
     'gfd_operator_family': (_i, [_vp, _i, _l, _i]),
     'gfd_gs_order': (_i, [_ip, _i, _ip, _ip]),
     'gfd_transformer_new': (_i, [_lp, _lp, _i, _lp, _lp, _lp, _lp, _i, _i,

@@ -298,8 +298,8 @@ static int op_pass(gfd_operator* op, int dtype, const void* in, void* out,
         return launch_point(op->ax, dtype, op->n, bc, in, out, nin, epi, ea,
                             s, nblocks);
     if (path == 2)
-        return launch_dirmarch(op->dir, dtype, op->n, bc, in, out, nin, epi,
-                               ea, s, nblocks);
+        return launch_dirmarch(op->dir, op->dir_tiles, dtype, op->n, bc, in,
+                               out, nin, epi, ea, s, nblocks);
     return launch_general_stencil(op->gen(ea.c0), dtype, op->n, bc, in, out,
                                   nin, epi, ea, s, nblocks);
 }
@@ -320,7 +320,8 @@ static long op_max_blocks(gfd_operator* op, int dtype, long nin)
 {
     long m = general_stencil_max_blocks(op->n, nin);
     if (op->dir_ok)
-        m = std::max(m, dirmarch_max_blocks(op->dir, dtype, op->n, nin));
+        m = std::max(m, dirmarch_max_blocks(op->dir, op->dir_tiles, dtype,
+                                            op->n, nin));
     if (op->use_fast()) {
         m = std::max(m, row_stencil_max_blocks(op->ax, dtype, op->n, nin));
     }

@@ -3,6 +3,8 @@
 // pair), marching along x.
 #pragma once
 
+#include <mutex>
+
 #include "stencil.h"
 
 namespace gfd {
@@ -41,15 +43,6 @@ struct DirStencil {
 // lies beyond MAXR_FAST steps, or more directions are needed.
 bool dir_stencil(int P, const double* coef, const int* off, DirStencil& d);
 
-// Whether k_dirmarch takes this pass.
-bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi);
-long dirmarch_max_blocks(const DirStencil& d, int dtype, const int n[3],
-                         long nin);
-int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
-                    const BC& bc, const void* in, void* out, long nin,
-                    int epi, const EpiArgs& ea, hipStream_t s,
-                    int* nblocks_out);
-
 // Tile in place of the estimated one (tuning key "xm_tile"; rows nseg x py),
 // where it fits and the pass sums no norm (its buffer is sized for the
 // estimated tile); nullptr clears.
@@ -81,8 +74,38 @@ inline int dir_line(const DirStencil& d, int epi)
 }
 
 // The tile with the least estimated time; every grid of sides >= R has one.
+// A search of 1 to 11 us on the host (8 f64 grids of 48^3, one c128 grid of
+// 160^3), as long as the kernels of small grids run.
 DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin,
                  int epi);
+
+// The tiles one operator has used, by data type, batch and halo: looked up on
+// each launch, from any thread.  The oldest of them makes room for a new one.
+class DirTiles {
+public:
+    DirTile get(const DirStencil& d, int dtype, const int n[3], long nin,
+                int epi);
+
+private:
+    struct Entry {
+        int dtype, line;
+        long nin;
+        DirTile t;
+    };
+    static constexpr int MOST = 16;
+    std::mutex mu;
+    Entry e[MOST];
+    int used = 0, next = 0;
+};
+
+// Whether k_dirmarch takes this pass.
+bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi);
+long dirmarch_max_blocks(const DirStencil& d, DirTiles& tiles, int dtype,
+                         const int n[3], long nin);
+int launch_dirmarch(const DirStencil& d, DirTiles& tiles, int dtype,
+                    const int n[3], const BC& bc, const void* in, void* out,
+                    long nin, int epi, const EpiArgs& ea, hipStream_t s,
+                    int* nblocks_out);
 
 int dirmarch_f64(const DirStencil& d, const DirTile& t, const int n[3],
                  const BC& bc, const void* in, void* out, long nin, int epi,

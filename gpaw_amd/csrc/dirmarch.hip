@@ -2,8 +2,8 @@
 #include "dirmarch.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
-#include <mutex>
 
 namespace gfd {
 
@@ -157,15 +157,33 @@ static bool dm_search(const DirStencil& d, int dtype, const int n[3],
     return least < 1e300;
 }
 
+static std::atomic<long> g_dm_searches{0};
+
 DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin,
                  int epi)
 {
+    g_dm_searches++;
     DirTile t{};
     // At R = 4 the halo of a few short rows (4 of 14 to 16 points, 5 of 12)
     // is more than four points for each thread of their only tile.
     if (!dm_search(d, dtype, n, nin, epi, false, t))
         dm_search(d, dtype, n, nin, epi, true, t);
     return t;
+}
+
+DirTile DirTiles::get(const DirStencil& d, int dtype, const int n[3],
+                      long nin, int epi)
+{
+    const int line = dir_line(d, epi);
+    std::lock_guard<std::mutex> lk(mu);
+    for (int i = 0; i < used; i++)
+        if (e[i].nin == nin && e[i].dtype == dtype && e[i].line == line)
+            return e[i].t;
+    Entry& x = e[next];
+    x = Entry{dtype, line, nin, dir_tile(d, dtype, n, nin, epi)};
+    next = (next + 1) % MOST;
+    used = std::max(used, next ? next : MOST);
+    return x.t;
 }
 
 bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi)
@@ -185,21 +203,21 @@ bool dirmarch_fits(const DirStencil& d, int dtype, const int n[3], int epi)
     return true;
 }
 
-long dirmarch_max_blocks(const DirStencil& d, int dtype, const int n[3],
-                         long nin)
+long dirmarch_max_blocks(const DirStencil& d, DirTiles& tiles, int dtype,
+                         const int n[3], long nin)
 {
     if (d.R < 1 || std::min({n[0], n[1], n[2]}) < d.R) return 0;
-    const DirTile t = dir_tile(d, dtype, n, nin, EPI_RESID);
+    const DirTile t = tiles.get(d, dtype, n, nin, EPI_RESID);
     return (long)ceil_div(n[2], t.tz) * ceil_div(n[1], t.ty) *
            ceil_div(n[0], t.xchunk) * nin;
 }
 
-int launch_dirmarch(const DirStencil& d, int dtype, const int n[3],
-                    const BC& bc, const void* in, void* out, long nin,
-                    int epi, const EpiArgs& ea, hipStream_t s,
+int launch_dirmarch(const DirStencil& d, DirTiles& tiles, int dtype,
+                    const int n[3], const BC& bc, const void* in, void* out,
+                    long nin, int epi, const EpiArgs& ea, hipStream_t s,
                     int* nblocks_out)
 {
-    DirTile t = dir_tile(d, dtype, n, nin, epi);
+    DirTile t = tiles.get(d, dtype, n, nin, epi);
     if (!ea.partial) {
         std::lock_guard<std::mutex> lk(g_dm_mu);
         const DirTile& o = g_dm_tile;
@@ -242,4 +260,9 @@ extern "C" int gfd_march_tile(int npoints, const double* coefs,
     tile[2] = t.xchunk;
     tile[3] = t.threads;
     return gfd::OK;
+}
+
+extern "C" long gfd_march_tile_searches(void)
+{
+    return gfd::g_dm_searches;
 }

@@ -12,7 +12,7 @@
 
 namespace gfd {
 
-// 0 auto, 1 general kernel, 2 tiled x-march kernel, 3 full-row kernel
+// 0 auto, 1 general kernel, 2 direction march, 3 full-row kernel
 extern int g_force_path;
 
 // Grow-only device buffer.  Growing waits for the stream first, so a buffer
@@ -85,6 +85,7 @@ struct gfd_operator {
         return g;
     }
     gfd::DirStencil dir;   // direction form (dir_ok)
+    gfd::DirTiles dir_tiles;
     bool dir_ok = false;
     bool use_fast() const { return axis_ok && g_force_path != 1; }
 };

@@ -100,6 +100,11 @@ int gfd_march_tile(int npoints, const double* coefs, const int* offsets,
                    const int n[3], int dtype, long nin, int plain,
                    int tile[4]);
 
+/* No counterpart in the reference (host only): how often this process has
+ * searched for such a tile.  An operator searches once per data type and
+ * batch, of which it keeps the last 16. */
+long gfd_march_tile_searches(void);
+
 /* Replaces Operator.get_diagonal_element() -- c/operators.cpp:319-332. */
 double gfd_operator_get_diagonal_element(const gfd_operator* op);
 

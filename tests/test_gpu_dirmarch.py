@@ -281,3 +281,31 @@ def test_radius_4(N, dtype):
             ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c,
                                   gd.neighbor_cd, a, ph)
             assert relerr(host(out), ref) < TOL
+
+
+def test_tiles_are_looked_up():
+    """A batch searches for its tile once, with the residual's block bound;
+    batches beyond the number kept still run right."""
+    rng = np.random.default_rng(8)
+    gd = grid((9, 13, 17), 'hex', True)
+    op = Laplace(gd, -0.7, 2, complex)
+    searches = _lib.load().gfd_march_tile_searches
+    a = rand(rng, (40,) + tuple(gd.n_c), complex)
+    da, out = dev(a), dev(np.zeros_like(a))
+    ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a)
+    op.apply(da[:3], out[:3])
+    n = searches()
+    for _ in range(3):
+        op.apply(da[:3], out[:3])
+    assert searches() == n
+    norm, lib = _lib.ctypes.c_double(), _lib.load()
+    for new in (1, 0, 0):      # one halo more, with and without a norm
+        n = searches()
+        _lib.check(lib.gfd_operator_residual(
+            op._handle(), da.data_ptr(), da.data_ptr(), out.data_ptr(), 2,
+            None, _lib.ctypes.byref(norm), None), 'residual')
+        assert searches() == n + new
+    for nb in (*range(1, 41), 1, 40):
+        out.zero_()
+        op.apply(da[:nb], out[:nb])
+        assert relerr(host(out)[:nb], ref[:nb]) < TOL
