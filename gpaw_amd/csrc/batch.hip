@@ -438,7 +438,7 @@ struct gfd_batch_poisson {
     hipStream_t gs = nullptr;
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
     hipGraphExec_t graph = nullptr;
-    int gkey[4] = {-1, -1, -1, -1};
+    int gkey[5] = {-1, -1, -1, -1, -1};
     int num_cu = 256;
     // per-grid levels L-1 .. nlev-1 in LDS-resident workgroups (one per
     // grid) in place of the coarsest batched level
@@ -1592,8 +1592,9 @@ extern "C" int gfd_batch_poisson_solve_mixed(
     bool cchanged = false;
     GFD_TRY(b_plan_coarse(b, pre, post, coarse_sweeps, s, &cchanged));
     GFD_TRY(b_plan_blocked(b, pre, post, s));
-    const int key[4] = {pre, post, coarse_sweeps, b->coarse ? 1 : 0};
-    if (b->graph && (cchanged || !std::equal(key, key + 4, b->gkey))) {
+    const int key[5] = {pre, post, coarse_sweeps, b->coarse ? 1 : 0,
+                        ts_enabled() ? 1 : 0};
+    if (b->graph && (cchanged || !std::equal(key, key + 5, b->gkey))) {
         (void)hipGraphExecDestroy(b->graph);
         b->graph = nullptr;
     }
@@ -1624,7 +1625,7 @@ extern "C" int gfd_batch_poisson_solve_mixed(
                               hipGetErrorString(e2));
                     return EHIP;
                 }
-                std::copy(key, key + 4, b->gkey);
+                std::copy(key, key + 5, b->gkey);
             }
             GFD_CHECK_HIP(hipGraphLaunch(b->graph, s));
         } else {

@@ -81,3 +81,16 @@ def batch_xfer(code):
         yield
     finally:
         lib.gfd_set_tuning(b'batch_xfer', 0)
+
+
+def kernels_of(f):
+    """(f(), the names of the kernels it launched, graph replays among them),
+    names None where the profiler records none."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        out = f()
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages() if 'gfd::k_' in e.key]
+    return out, names or None

@@ -5,9 +5,10 @@ import numpy as np
 import pytest
 
 from gpaw_amd import _lib
+from gpaw_amd.batch_poisson import BatchedPoissonSolver
 from gpaw_amd.grid_descriptor import GridDescriptor
-from gpaw_amd.poisson import FDPoissonSolver
-from gpu_util import dev, host, say
+from gpaw_amd.poisson import FDPoissonSolver, PoissonConvergenceError
+from gpu_util import dev, host, kernels_of, say
 from helpers import relerr
 
 pytestmark = pytest.mark.gpu
@@ -79,3 +80,46 @@ def test_sweep_counts(pre, post, fp64):
     # the solutions differ by their residuals: 1e-10 times the condition
     # number of this operator (some 1e3) at most
     assert relerr(out[0][1], out[1][1]) < 1e-7
+
+
+def test_batched():
+    """Uneven grids of both boundaries in one launch, and the switch taking
+    effect on a solver that has already captured its step: two refinement
+    steps by graph replays run the kernels of the setting and equal the eager
+    ones bit for bit, and the two settings agree to the FP32 rounding of some
+    60 sweeps of 10 operations in each cycle (60 * 10 * 6e-8 = 4e-5, times
+    3)."""
+    grids = [((24, 32, 40), True), ((40, 24, 16), False), ((16, 16, 16), True),
+             ((32, 56, 24), (True, False, True)), ((48, 40, 72), False)]
+    gds = [GridDescriptor(n, np.array(n) * 0.35, p) for n, p in grids]
+    solver = BatchedPoissonSolver(nn=3)
+    solver.set_grid_descriptors(gds)
+    rng = np.random.default_rng(4)
+    rhos = []
+    for gd in gds:
+        rho = rng.uniform(-1, 1, tuple(gd.n_c))
+        rhos.append(dev(rho - rho.mean() if gd.pbc_c.all() else rho))
+
+    def steps(on, graph):
+        lib = _lib.load()
+        _lib.check(lib.gfd_set_tuning(b'tsmooth', on), 'tsmooth')
+        try:
+            phis = [dev(np.zeros(tuple(gd.n_c))) for gd in gds]
+            with pytest.raises(PoissonConvergenceError):
+                solver.solve_mixed(phis, rhos, 1e-30, max_outer=2,
+                                   graph=graph)
+            return [host(p) for p in phis]
+        finally:
+            lib.gfd_set_tuning(b'tsmooth', 1)
+
+    want = {}
+    for on in (1, 0, 1):
+        say('blocked smoothing, batched', on)
+        got, names = kernels_of(lambda: steps(on, True))
+        if names:
+            assert any('k_tsmooth' in k for k in names) == bool(on)
+        want[on] = steps(on, False)
+        for a, b in zip(got, want[on]):
+            assert (a == b).all()
+    for a, b in zip(want[0], want[1]):
+        assert relerr(a, b) < 1.2e-4
