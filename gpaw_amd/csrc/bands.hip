@@ -669,6 +669,32 @@ int band_update(int dtype, int mode, const double* alpha, double scale,
     return OK;
 }
 
+// Chunks of the points: the count with the least estimated time on 256 CUs
+// that run one block at a time each, rounds x (points of a chunk + 61): a
+// block's 262 KB of partial sums cost as much to write and read back as some
+// 61 points of its tile take to multiply.  (500 bands, 10 lower tiles: 231
+// chunks started a tenth round for 6 blocks, 18.6 ms.)  At most 9 rounds (the
+// partial sums of 2304 tiles take 604 MB), at least 4 stages per chunk; a few
+// per cent in favour of more rounds, which even out blocks of unequal speed.
+// Within a round more chunks are always better, so each has one candidate.
+static long gram_chunks(long nt, long K)
+{
+    const long top = std::max(1L, std::min(2304L / nt, K / (4 * GK)));
+    long chunks = 1;
+    double least = 1e300;
+    for (long r = 1; r <= 9; r++) {
+        const long c = std::min(top, std::max(1L, 256 * r / nt));
+        const double rounds = (double)((nt * c + 255) / 256);
+        const double cost =
+            rounds * ((double)K / c + 61.0) * (1.0 + 0.06 / rounds);
+        if (cost < least) {
+            least = cost;
+            chunks = c;
+        }
+    }
+    return chunks;
+}
+
 int gram(BandWork& w, const double2* A, long lda, const double2* B, long ldb,
          int M, int N, long K, double alpha, int conj, int lower_only,
          double2* out, long ldo, hipStream_t s)
@@ -684,25 +710,7 @@ int gram(BandWork& w, const double2* A, long lda, const double2* B, long ldb,
         set_error("gram: no points");
         return EINVAL_;
     }
-    // chunks: the count with the least estimated time on 256 CUs that run
-    // one block at a time each, rounds x (points of a chunk + 61): a block's
-    // 262 KB of partial sums cost as much to write and read back as some 61
-    // points of its tile take to multiply.  (500 bands, 10 lower tiles: 231
-    // chunks started a tenth round for 6 blocks, 18.6 ms.)  At most 10
-    // rounds, at least 4 stages per chunk; a few per cent in favour of more
-    // rounds, which even out blocks of unequal speed.
-    long chunks = 1;
-    double least = 1e300;
-    const long top = std::max(1L, std::min(2560L / nt, K / (4 * GK)));
-    for (long c = 1; c <= top; c++) {
-        const double rounds = (double)((nt * c + 255) / 256);
-        const double cost =
-            rounds * ((double)K / c + 61.0) * (1.0 + 0.06 / rounds);
-        if (cost < least) {
-            least = cost;
-            chunks = c;
-        }
-    }
+    long chunks = gram_chunks(nt, K);
     long kchunk = (K + chunks - 1) / chunks;
     kchunk = (kchunk + GK - 1) / GK * GK;
     chunks = (K + kchunk - 1) / kchunk;
@@ -876,3 +884,12 @@ int cholesky_orth(BandWork& w, double2* S, int n, const double2* psi,
 }
 
 }  // namespace gfd
+
+extern "C" long gfd_gram_chunks(long ntiles, long npts)
+{
+    if (ntiles < 1 || npts < 1) {
+        gfd::set_error("gfd_gram_chunks: bad arguments");
+        return -1;
+    }
+    return gfd::gram_chunks(ntiles, npts);
+}

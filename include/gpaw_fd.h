@@ -358,6 +358,12 @@ int gfd_band_dots(int is_complex, const void* a, const void* b, int nbands,
 int gfd_rmm_lambda(int is_complex, const void* dR, const void* R, int nbands,
                    long npts, long ld, double* lam, void* stream);
 
+/* No counterpart in the reference (host only): the parts into which a
+ * contraction of ntiles 128 x 128 tiles (gfd_band_overlap, gfd_band_matrix)
+ * splits its npts points.  Its work space holds ntiles x parts tiles of 256
+ * KiB; -1 for bad arguments. */
+long gfd_gram_chunks(long ntiles, long npts);
+
 /* gfd_band_dots and gfd_rmm_lambda with nwork doubles of device memory as
  * work space (not shared by calls that overlap in time): from
  * 2 (2048 + nbands) on, a band's sum is split over several blocks when
