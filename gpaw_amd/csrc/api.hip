@@ -259,10 +259,11 @@ static bool march_first(const gfd_operator* op, int epi)
 // Kernel family for one pass: 4 one point per thread, 3 full-row, 2 direction
 // march, 1 general.
 static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
-                   const void* out, const void* aux, int epi)
+                   const void* out, const void* aux, int epi,
+                   bool march = true)
 {
     if (g_force_path == 1) return 1;
-    const bool dir = op->dir_ok && g_force_path != 3 &&
+    const bool dir = march && op->dir_ok && g_force_path != 3 &&
                      dirmarch_fits(op->dir, dtype, op->n, epi);
     if (dir && g_force_path == 2) return 2;
     // (k_point reads every step of an axis; k_dirmarch only those there are)
@@ -287,10 +288,10 @@ static int op_path(gfd_operator* op, int dtype, long nin, const void* in,
 // One stencil pass with an epilogue (the building block of every driver).
 static int op_pass(gfd_operator* op, int dtype, const void* in, void* out,
                    long nin, const double* phases, int epi, EpiArgs ea,
-                   hipStream_t s, int* nblocks)
+                   hipStream_t s, int* nblocks, bool march = true)
 {
     const BC bc = make_bc(op->periodic, phases);
-    const int path = op_path(op, dtype, nin, in, out, ea.aux, epi);
+    const int path = op_path(op, dtype, nin, in, out, ea.aux, epi, march);
     if (path == 3)
         return launch_row_stencil(op->ax, dtype, op->n, bc, in, out, nin, epi,
                                   ea, s, nblocks);
@@ -316,10 +317,11 @@ extern "C" int gfd_operator_family(gfd_operator* op, int dtype, long nin,
 }
 
 // Upper bound of the blocks a residual pass may launch (partial sums).
-static long op_max_blocks(gfd_operator* op, int dtype, long nin)
+static long op_max_blocks(gfd_operator* op, int dtype, long nin,
+                          bool march = true)
 {
     long m = general_stencil_max_blocks(op->n, nin);
-    if (op->dir_ok)
+    if (op->dir_ok && march)
         m = std::max(m, dirmarch_max_blocks(op->dir, op->dir_tiles, dtype,
                                             op->n, nin));
     if (op->use_fast()) {
@@ -458,7 +460,7 @@ static int residual_norm(gfd_operator* op, int dtype, const void* in,
                          const void* b, void* r, long nin,
                          const double* phases, double* dev_norm,
                          hipStream_t s, bool narrow = false,
-                         double* partial = nullptr)
+                         double* partial = nullptr, bool march = true)
 {
     EpiArgs ea{};
     ea.aux = b;
@@ -473,7 +475,7 @@ static int residual_norm(gfd_operator* op, int dtype, const void* in,
     }
     int nb = 0;
     GFD_TRY(op_pass(op, dtype, in, r, nin, phases,
-                    narrow ? EPI_RESN : EPI_RESID, ea, s, &nb));
+                    narrow ? EPI_RESN : EPI_RESID, ea, s, &nb, march));
     if (dev_norm) GFD_TRY(launch_sum_partials(ea.partial, nb, dev_norm, s));
     return OK;
 }
@@ -564,7 +566,12 @@ extern "C" int gfd_operator_residual_noalloc(gfd_operator* op,
         return OK;
     }
     const int dtype = op->dtype();
-    const long nbmax = op_max_blocks(op, dtype, nin);
+    long nbmax = op_max_blocks(op, dtype, nin);
+    // a batch of very many tiny skew cells: the march has a block for each
+    // grid, the general kernel one for every 256 points of all
+    const bool march = !norm2 || nbmax <= NA_DOUBLES - NA_PARTIAL ||
+                       op->axis_ok;
+    if (!march) nbmax = op_max_blocks(op, dtype, nin, false);
     if (norm2 && nbmax > NA_DOUBLES - NA_PARTIAL) {
         set_error("gfd_operator_residual_noalloc: %ld grids of %d x %d x %d "
                   "need %ld partial sums, above the fixed %ld; split the "
@@ -578,7 +585,7 @@ extern "C" int gfd_operator_residual_noalloc(gfd_operator* op,
     xr_no_tune_here(true);
     const int st =
         residual_norm(op, dtype, in, b, r, nin, op->real ? nullptr : phases,
-                      sp, s, false, sp ? sp + NA_PARTIAL : nullptr);
+                      sp, s, false, sp ? sp + NA_PARTIAL : nullptr, march);
     xr_no_tune_here(false);
     GFD_TRY(st);
     if (norm2) {

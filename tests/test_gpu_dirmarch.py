@@ -309,3 +309,24 @@ def test_tiles_are_looked_up():
         out.zero_()
         op.apply(da[:nb], out[:nb])
         assert relerr(host(out)[:nb], ref[:nb]) < TOL
+
+
+def test_many_tiny_skew_cells():
+    """A residual on fixed scratch of more cells than it has partial sums
+    for one block each: the general kernel, with one per 256 points."""
+    import torch
+    gd = grid((4, 4, 4), 'hex', True)
+    op = Laplace(gd, -0.7, 1)
+    lib = _lib.load()
+    nb = lib.gfd_operator_residual_noalloc_max_blocks() + 60
+    g = torch.Generator(device='cuda').manual_seed(2)
+    a, b = (torch.randn((nb, 4, 4, 4), generator=g, dtype=torch.float64,
+                        device='cuda') for _ in range(2))
+    r, norm = torch.empty_like(a), _lib.ctypes.c_double()
+    _lib.check(lib.gfd_operator_residual_noalloc(
+        op._handle(), a.data_ptr(), b.data_ptr(), r.data_ptr(), nb, None,
+        _lib.ctypes.byref(norm), None), 'residual')
+    ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd,
+                          host(a)) - host(b)
+    assert relerr(host(r), ref) < TOL
+    assert abs(norm.value / (ref**2).sum() - 1) < 1e-12
