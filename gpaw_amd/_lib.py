@@ -58,6 +58,7 @@ SIGNATURES = {
     'gfd_poisson_iterate': (_i, [_vp, _vp, _vp, _dp, _vp]),
     'gfd_poisson_solve': (_i, [_vp, _vp, _vp, _d, _i, _i, _ip, _dp, _vp]),
     'gfd_poisson_set_graph': (_i, [_vp, _i]),
+    'gfd_poisson_coarse_plan': (_i, [_vp, _i, _ip, _i]),
     'gfd_poisson_solve_mixed': (_i, [_vp, _vp, _vp, _d, _i, _i, _i, _i, _d,
                                      _d, _i, _i, _i, _ip, _dp, _vp]),
     'gfd_batch_poisson_new': (_i, [_i, _i, ctypes.POINTER(_vp),

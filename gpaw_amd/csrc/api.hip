@@ -1737,6 +1737,23 @@ extern "C" int gfd_poisson_solve_mixed(gfd_poisson* p, double* phi,
     return OK;
 }
 
+extern "C" int gfd_poisson_coarse_plan(const gfd_poisson* p, int which,
+                                       int* plan, int nplan)
+{
+    if (!p || !plan || nplan < 2 || which < 0 || which > 2) {
+        set_error("gfd_poisson_coarse_plan: bad arguments");
+        return -1;
+    }
+    const CoarseSolve& c = which == 0 ? p->cs64
+                           : which == 1 ? p->cs32 : p->cs64r;
+    plan[0] = c.valid ? c.lc : -1;
+    plan[1] = c.valid && c.one;
+    int n = 2;
+    for (int i = 0; plan[0] >= 0 && i < c.host.nlev && n < nplan; i++)
+        plan[n++] = plan[1] ? c.host.lev[i].xl : 0;
+    return n;
+}
+
 // =================================================================== bands
 
 // Work spaces of the band calls and of gfd_dot, one per stream, so that

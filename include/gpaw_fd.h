@@ -203,6 +203,15 @@ int gfd_poisson_solve(gfd_poisson* p, double* phi, const double* rho,
  * (no reference counterpart).  Results are identical either way. */
 int gfd_poisson_set_graph(gfd_poisson* p, int on);
 
+/* No counterpart in the reference (no device calls): what the last solve
+ * planned for its coarse levels, which 0 the FP64 schedule, 1 the FP32 and 2
+ * the FP64 refinement.  plan[0]: first level of the one-workgroup solve, -1
+ * without one; plan[1]: 1 when it keeps x segments in registers; then for
+ * each of its levels the longest segment (0 in the other form).  Returns the
+ * entries written, nplan at most, -1 for bad arguments. */
+int gfd_poisson_coarse_plan(const gfd_poisson* p, int which, int* plan,
+                            int nplan);
+
 /* Mixed-precision solve (no reference counterpart; the FP64 equations are
  * those of FDPoissonSolver): FP64 iterative refinement on the level-0
  * residual r = L phi - rho, each step solving L e = r with `inner` FP32
