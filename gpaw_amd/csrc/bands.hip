@@ -529,10 +529,27 @@ k_band_join(const double* __restrict__ work, int chunks, double dv,
         out[blockIdx.x] = LAMBDA ? (s1 > 0.0 ? -s0 / s1 : 0.0) : dv * s0;
 }
 
-// Blocks per band: about 2048 in all, at least 4096 points each (1: not
-// split, and no work space needed).
-static int band_chunks(int nbands, long npts, long nwork)
+// Blocks per band (1: not split, and no work space needed): about 2048 in
+// all, at least 4096 points each, where bands of that many points, too few to
+// fill the GPU, gain by it.  Time split over one block of 1024 threads each:
+//   f64   17k points 0.97 (1 band) .. 1.00 (64), 20k 0.93 .. 0.95 (40) but 1.2
+//         (64), 44k 0.51 .. 0.81 (100), 96k 1.18 (150), 130k 0.20 .. 0.80
+//         (150); from 220 bands on 1.05 to 1.27 at any length
+//   c128  twice the bytes: 17k 0.96 .. 0.98 (20), 20k 1.18 (40), 44k 0.51 ..
+//         0.94 (64), 72k 1.12 (100), 96k 0.26 .. 0.76 (100) and 0.92 (116); 150
+//         to 220 bands 1.00 to 1.19, 300 (two blocks on some CUs) 0.76 to
+//         0.95, beyond 0.92 to 1.09
+static int band_chunks(int nbands, long npts, bool cplx, long nwork)
 {
+    const int w = cplx ? 2 * nbands : nbands;
+    const long least = w <= 40    ? 18000
+                       : w <= 128 ? 40000
+                       : cplx     ? 96000
+                                  : 130000;
+    const bool gains = cplx && nbands > 256
+                           ? npts >= 40000
+                           : nbands <= (cplx ? 120 : 150) && npts >= least;
+    if (!gains) return 1;
     long c = std::min((2048L + nbands - 1) / nbands, npts / 4096);
     c = std::min(c, nwork / (2L * nbands));
     return nbands > 65535 || c < 2 ? 1 : (int)c;
@@ -560,7 +577,7 @@ int rmm_lambda(int dtype, const void* dR, const void* R, int nbands,
                hipStream_t s)
 {
     if (nbands <= 0) return OK;
-    const int chunks = band_chunks(nbands, npts, work ? nwork : 0);
+    const int chunks = band_chunks(nbands, npts, dtype == 1, work ? nwork : 0);
     if (chunks > 1)
         return dtype == 1
                    ? band_split<double2, true>(dR, R, nbands, npts, ld, 0.0,
@@ -584,7 +601,7 @@ int band_dots(int dtype, const void* A, const void* B, int nbands, long npts,
               hipStream_t s)
 {
     if (nbands <= 0) return OK;
-    const int chunks = band_chunks(nbands, npts, work ? nwork : 0);
+    const int chunks = band_chunks(nbands, npts, dtype == 1, work ? nwork : 0);
     if (chunks > 1)
         return dtype == 1
                    ? band_split<double2, false>(A, B, nbands, npts, ld, dv,
