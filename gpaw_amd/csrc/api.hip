@@ -2058,7 +2058,7 @@ extern "C" int gfd_set_tuning(const char* key, long value)
         return OK;
     }
     if (std::strcmp(key, "xfer_passes") == 0) {
-        xfer_force_passes(value != 0);
+        xfer_force_passes(value != 0, value == 2);
         return OK;
     }
     if (std::strcmp(key, "wx_march") == 0) {

@@ -40,11 +40,11 @@ struct XferPlan {
     XferAxis ax[3];
 };
 
-// K = 2 transfers run as one fused kernel unless forced to the 3 passes.
-void xfer_force_passes(bool on);
+// Every transfer on the separable passes (x after z and y in one launch;
+// three: after z and y in one each).
+void xfer_force_passes(bool on, bool three);
 // Use the x-marching fused kernels (every K; default on).  Off: K = 2 by
-// the one-point-per-thread fused kernels, K > 2 by separable passes (z and y in one
-// launch, then x).
+// the one-point-per-thread fused kernels, K > 2 by separable passes.
 void xfer_set_march(bool on);
 // Whether K = 2 transfers are forced onto the separable passes (they then
 // need the passes' work space).

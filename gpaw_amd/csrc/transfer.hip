@@ -104,9 +104,9 @@ __device__ inline T xload(const XArgs<T>& a, const T* __restrict__ g,
     return v;
 }
 
-// x pass
-template <typename T, int K, bool INTERP, int EPI>
-__global__ void __launch_bounds__(256) k_xfer_x(XArgs<T> a)
+// One axis, one point per thread.
+template <typename T, int AX, int K, bool INTERP, int EPI>
+__global__ void __launch_bounds__(256) k_xfer1d(XArgs<T> a)
 {
     typedef typename ScalarOf<T>::type S;
     const long gid = (long)blockIdx.x * 256 + threadIdx.x;
@@ -114,8 +114,11 @@ __global__ void __launch_bounds__(256) k_xfer_x(XArgs<T> a)
     long b;
     int o0, o1, o2;
     flat_split(gid, a.total, a.out_grid, a.d[1], a.d[2], b, o0, o1, o2);
-    const long pos = (long)o1 * a.d[2] + o2;  // at x = 0
-    const int i = o0;
+    // input position with the pass axis at 0
+    const long pos = AX == 2   ? ((long)o0 * a.d[1] + o1) * a.ilen
+                     : AX == 1 ? (long)o0 * a.ilen * a.d[2] + o2
+                               : (long)o1 * a.d[2] + o2;
+    const int i = AX == 2 ? o2 : AX == 1 ? o1 : o0;
     const T* __restrict__ g = a.in + b * a.in_grid;
     T v;
     if constexpr (!INTERP) {
@@ -605,8 +608,8 @@ static int launch_fused2(const XferPlan& p, const BC& bc, const void* in,
 
 long xfer_scratch_elems(const XferPlan& p, long nin)
 {
-    // output of the z and y passes
-    return (long)p.nin[0] * p.nout[1] * p.nout[2] * nin;
+    // outputs of the z pass and of the y pass
+    return (long)p.nin[0] * (p.nin[1] + p.nout[1]) * p.nout[2] * nin;
 }
 
 // z and y passes of a separable transfer in one launch: a block stages the
@@ -618,7 +621,11 @@ long xfer_scratch_elems(const XferPlan& p, long nin)
 // Two passes before -> this and x, K = 6: restriction of 4 real grids of 96^3
 // 25.4 -> 22.1 us, 32 of them 150 -> 122, one of 48^3 16.6 -> 8.4; staged
 // columns in order instead of even / odd: 24.2.  Interpolation of 4 complex
-// grids of 96^3 at K = 8 50.7 -> 38.6 (marching 112).
+// grids of 96^3 at K = 8 50.7 -> 38.6 (marching 112).  Threads take columns
+// side by side: with a wave per row 35 grids of 200x60x24 took 64 us at K = 4
+// (now 41, two passes 42).  Where a tile's halo is large against it, at K = 8
+// above all, two passes stay the faster ones (56 boxes of 30x40x150 53 us, 69
+// here), so both are timed per shape.
 template <typename T>
 struct ZyArgs {
     const T* in;
@@ -680,8 +687,7 @@ __global__ void __launch_bounds__(256) k_xfer_zy(ZyArgs<T> a)
     rem /= a.tiles_z;
     const int yt = rem % a.tiles_y;
     const long pl = rem / a.tiles_y;
-    const int t = threadIdx.x, lane = t & 63;
-    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int t = threadIdx.x;
     const int oy0 = yt * a.cy, oy1 = min(oy0 + a.cy, a.no1);
     const int oz0 = zt * a.zt, oz1 = min(oz0 + a.zt, a.no2);
     const int iy0 = zy_first<K, INTERP>(oy0, a.off[0], a.skip0[0]);
@@ -713,28 +719,31 @@ __global__ void __launch_bounds__(256) k_xfer_zy(ZyArgs<T> a)
         }
         return i;
     };
-    constexpr int JU = sizeof(T) == 16 ? 8 : 12;  // rows a wave has in flight
-    for (int z0 = 0; z0 < nz; z0 += 64) {
-        const int z = z0 + lane;
+    // A thread keeps one column of the staged rows, as many rows side by side
+    // as the block holds.
+    constexpr int JU = sizeof(T) == 16 ? 8 : 12;  // loads in flight
+    {
+        const int side = 256 / nz;
+        const int r0 = t / nz, z = t - r0 * nz;
         double2 f, fy;
         bool ph, py;
-        const int iz = z < nz ? wrap(iz0 + z, a.ni2, 1, f, ph) : -1;
-        for (int j0 = w; j0 < ny; j0 += 4 * JU) {
+        const int iz = wrap(iz0 + z, a.ni2, 1, f, ph);
+        for (int j0 = r0 < side ? r0 : ny; j0 < ny; j0 += side * JU) {
             T v[JU];
 #pragma unroll
             for (int j = 0; j < JU; j++) {
                 v[j] = zero_of<T>();
-                const int r = j0 + 4 * j;
+                const int r = j0 + side * j;
                 if (r >= ny) continue;
                 const int iy = wrap(iy0 + r, a.ni1, 0, fy, py);
                 if (iy >= 0 && iz >= 0) v[j] = g[(long)iy * a.ni2 + iz];
             }
 #pragma unroll
             for (int j = 0; j < JU; j++) {
-                const int r = j0 + 4 * j;
+                const int r = j0 + side * j;
                 if constexpr (XIsCplx<T>::value)
                     if (iz >= 0 && ph) v[j] = cmul(f, v[j]);
-                if (r < ny && z < nz) E[r * a.rz + col(z)] = v[j];
+                if (r < ny) E[r * a.rz + col(z)] = v[j];
             }
         }
     }
@@ -774,13 +783,14 @@ __global__ void __launch_bounds__(256) k_xfer_zy(ZyArgs<T> a)
     }
     __syncthreads();
     T* __restrict__ o = a.out + pl * a.no1 * a.no2;
-    for (int oy = oy0 + w; oy < oy1; oy += 4) {
+    const int side = 256 / noz;
+    const int z = t % noz;
+    for (int oy = oy0 + (t < side * noz ? t / noz : a.cy); oy < oy1;
+         oy += side) {
         const int c =
             zy_first<K, INTERP>(oy, a.off[0], a.skip0[0]) - iy0 + BACK;
-        const bool odd = (oy + a.skip0[0]) & 1;
-        for (int z = lane; z < noz; z += 64)
-            o[(long)oy * a.no2 + oz0 + z] =
-                zy_point<T, K, INTERP>(Z + c * a.zt + z, a.zt, odd);
+        o[(long)oy * a.no2 + oz0 + z] = zy_point<T, K, INTERP>(
+            Z + c * a.zt + z, a.zt, (oy + a.skip0[0]) & 1);
     }
 }
 
@@ -836,7 +846,7 @@ static int launch_zy(const XferPlan& p, const BC& bc, const T* in, T* out,
     return OK;
 }
 
-template <typename T, int K, bool INTERP, int EPI>
+template <typename T, int AX, int K, bool INTERP, int EPI>
 static int launch_pass(XArgs<T> a, hipStream_t s)
 {
     const long nb = (a.total + 255) / 256;
@@ -845,7 +855,7 @@ static int launch_pass(XArgs<T> a, hipStream_t s)
         set_error("transfer: too many blocks");
         return ENOTSUP_;
     }
-    hipLaunchKernelGGL((k_xfer_x<T, K, INTERP, EPI>), dim3((unsigned)nb),
+    hipLaunchKernelGGL((k_xfer1d<T, AX, K, INTERP, EPI>), dim3((unsigned)nb),
                        dim3(256), 0, s, a);
     GFD_LAUNCH_CHECK();
     return OK;
@@ -855,71 +865,89 @@ template <typename T, int K, bool INTERP>
 static int launch_pass_epi(XArgs<T> a, int epi, hipStream_t s)
 {
     switch (epi) {
-    case XEPI_PLAIN: return launch_pass<T, K, INTERP, XEPI_PLAIN>(a, s);
-    case XEPI_NEG: return launch_pass<T, K, INTERP, XEPI_NEG>(a, s);
-    case XEPI_SCALE2: return launch_pass<T, K, INTERP, XEPI_SCALE2>(a, s);
-    case XEPI_SUBFROM: return launch_pass<T, K, INTERP, XEPI_SUBFROM>(a, s);
+    case XEPI_PLAIN: return launch_pass<T, 0, K, INTERP, XEPI_PLAIN>(a, s);
+    case XEPI_NEG: return launch_pass<T, 0, K, INTERP, XEPI_NEG>(a, s);
+    case XEPI_SCALE2: return launch_pass<T, 0, K, INTERP, XEPI_SCALE2>(a, s);
+    case XEPI_SUBFROM: return launch_pass<T, 0, K, INTERP, XEPI_SUBFROM>(a, s);
     }
     set_error("transfer: bad epilogue %d", epi);
     return EINVAL_;
 }
 
+// three: z and y in a launch each, z's result in front of y's in the work
+// space; else both in one (k_xfer_zy).
 template <typename T, int K, bool INTERP>
 static int run_transfer(const XferPlan& p, const BC& bc, const void* in,
-                        void* out, long nin, void* scratch,
+                        void* out, long nin, void* scratch, bool three,
                         const XEpiArgs& ea, hipStream_t s)
 {
-    T* const t = (T*)scratch;
-    const int st =
-        launch_zy<T, K, INTERP>(p, bc, (const T*)in, t, nin, s);
-    if (st != OK) return st;
-    XArgs<T> a;
-    a.in = t;
-    a.out = (T*)out;
-    a.out2 = (T*)ea.out2;
-    a.base = (const T*)ea.base;
-    for (int c = 0; c < 3; c++) a.d[c] = p.nout[c];
-    a.ilen = p.nin[0];
-    a.istride = (long)p.nout[1] * p.nout[2];
-    a.in_grid = p.nin[0] * a.istride;
-    a.out_grid = p.nout[0] * a.istride;
-    a.total = a.out_grid * nin;
-    a.off = p.ax[0].off;
-    a.skip0 = p.ax[0].skip0;
-    a.periodic = bc.periodic[0];
-    a.ph_hi = bc.phase[0][0];
-    a.ph_lo = bc.phase[0][1];
-    a.negate = ea.negate;
-    a.alpha = ea.alpha;
-    return launch_pass_epi<T, K, INTERP>(a, ea.epi, s);
+    auto pass = [&](int ax, const T* from, T* to) {
+        XArgs<T> a;
+        a.in = from;
+        a.out = to;
+        a.out2 = (T*)ea.out2;
+        a.base = (const T*)ea.base;
+        // the axes after this one are done, those before it are not
+        for (int c = 0; c < 3; c++) a.d[c] = c < ax ? p.nin[c] : p.nout[c];
+        a.ilen = p.nin[ax];
+        a.istride = ax == 2   ? 1
+                    : ax == 1 ? (long)p.nout[2]
+                              : (long)p.nout[1] * p.nout[2];
+        a.out_grid = (long)a.d[0] * a.d[1] * a.d[2];
+        a.in_grid = a.out_grid / a.d[ax] * a.ilen;
+        a.total = a.out_grid * nin;
+        a.off = p.ax[ax].off;
+        a.skip0 = p.ax[ax].skip0;
+        a.periodic = bc.periodic[ax];
+        a.ph_hi = bc.phase[ax][0];
+        a.ph_lo = bc.phase[ax][1];
+        a.negate = ea.negate;
+        a.alpha = ea.alpha;
+        return a;
+    };
+    T* const z = (T*)scratch;
+    T* const zy = z + (long)p.nin[0] * p.nin[1] * p.nout[2] * nin;
+    if (three) {
+        GFD_TRY((launch_pass<T, 2, K, INTERP, XEPI_PLAIN>(
+            pass(2, (const T*)in, z), s)));
+        GFD_TRY((launch_pass<T, 1, K, INTERP, XEPI_PLAIN>(pass(1, z, zy), s)));
+    } else {
+        GFD_TRY((launch_zy<T, K, INTERP>(p, bc, (const T*)in, zy, nin, s)));
+    }
+    return launch_pass_epi<T, K, INTERP>(pass(0, zy, (T*)out), ea.epi, s);
 }
 
 template <typename T>
 static int run_transfer_k(const XferPlan& p, const BC& bc, const void* in,
-                          void* out, long nin, void* scratch,
+                          void* out, long nin, void* scratch, bool three,
                           const XEpiArgs& ea, hipStream_t s)
 {
     const bool I = p.interpolate != 0;
     switch (p.K) {
-    case 2: return I ? run_transfer<T, 2, true>(p, bc, in, out, nin, scratch, ea, s)
-                     : run_transfer<T, 2, false>(p, bc, in, out, nin, scratch, ea, s);
-    case 4: return I ? run_transfer<T, 4, true>(p, bc, in, out, nin, scratch, ea, s)
-                     : run_transfer<T, 4, false>(p, bc, in, out, nin, scratch, ea, s);
-    case 6: return I ? run_transfer<T, 6, true>(p, bc, in, out, nin, scratch, ea, s)
-                     : run_transfer<T, 6, false>(p, bc, in, out, nin, scratch, ea, s);
-    case 8: return I ? run_transfer<T, 8, true>(p, bc, in, out, nin, scratch, ea, s)
-                     : run_transfer<T, 8, false>(p, bc, in, out, nin, scratch, ea, s);
+    case 2: return I ? run_transfer<T, 2, true>(p, bc, in, out, nin, scratch, three, ea, s)
+                     : run_transfer<T, 2, false>(p, bc, in, out, nin, scratch, three, ea, s);
+    case 4: return I ? run_transfer<T, 4, true>(p, bc, in, out, nin, scratch, three, ea, s)
+                     : run_transfer<T, 4, false>(p, bc, in, out, nin, scratch, three, ea, s);
+    case 6: return I ? run_transfer<T, 6, true>(p, bc, in, out, nin, scratch, three, ea, s)
+                     : run_transfer<T, 6, false>(p, bc, in, out, nin, scratch, three, ea, s);
+    case 8: return I ? run_transfer<T, 8, true>(p, bc, in, out, nin, scratch, three, ea, s)
+                     : run_transfer<T, 8, false>(p, bc, in, out, nin, scratch, three, ea, s);
     }
     set_error("transfer: unsupported K=%d", p.K);
     return EINVAL_;
 }
 
 static bool g_xfer_force_passes = false;
+static bool g_xfer_three = false;  // forced passes in a launch each
 static bool g_xfer_march = true;
 
 bool xfer_passes_forced() { return g_xfer_force_passes; }
 
-void xfer_force_passes(bool on) { g_xfer_force_passes = on; }
+void xfer_force_passes(bool on, bool three)
+{
+    g_xfer_force_passes = on;
+    g_xfer_three = on && three;
+}
 void xfer_set_march(bool on) { g_xfer_march = on; }
 
 // ------------------------------------------------- kernel choice (timed)
@@ -938,7 +966,8 @@ struct XKey {
 };
 
 static std::mutex g_xc_mu;
-// 0 marching, 1 other kernels, 2 tiled K = 2 restriction
+// 0 marching, 1 other kernels, 2 tiled K = 2 restriction, 3 (K > 2) z and y
+// passes in a launch each
 static std::map<XKey, int> g_xchoice;
 static std::atomic<bool> g_xfer_tile{false};  // tiled wherever it fits
 
@@ -971,7 +1000,7 @@ static XKey xkey(const XferPlan& p, int dtype, long nin, int in_wide)
 
 static int launch_other(const XferPlan& p, int dtype, const BC& bc,
                         const void* in, void* out, long nin, void* scratch,
-                        const XEpiArgs& ea, hipStream_t stream);
+                        bool three, const XEpiArgs& ea, hipStream_t stream);
 
 bool xfer_needs_tuning(const XferPlan& p, int dtype, long nin, int in_wide)
 {
@@ -995,14 +1024,16 @@ int xfer_tune(const XferPlan& p, int dtype, const BC& bc, const void* in,
     }
     float best = 1e30f;
     int choice = 0;
-    for (int c = 0; c < (p.K == 2 && !p.interpolate ? 3 : 2); c++) {
+    for (int c = 0; c < 4; c++) {
+        if (c == 2 && (p.K != 2 || p.interpolate)) continue;
+        if (c == 3 && p.K == 2) continue;
         auto run = [&]() {
             return c == 0 ? launch_transfer_march(p, dtype, bc, in, tune_out,
                                                   nin, ea, s)
-                 : c == 1 ? launch_other(p, dtype, bc, in, tune_out, nin,
-                                         scratch, ea, s)
-                          : launch_restrict_tile(p, dtype, bc, in, tune_out,
-                                                 nin, ea, s);
+                 : c == 2 ? launch_restrict_tile(p, dtype, bc, in, tune_out,
+                                                 nin, ea, s)
+                          : launch_other(p, dtype, bc, in, tune_out, nin,
+                                         scratch, c == 3, ea, s);
         };
         if (run() != OK) {  // this kernel cannot take the shape
             set_error("");
@@ -1041,12 +1072,14 @@ int launch_transfer(const XferPlan& p, int dtype, const BC& bc,
     }
     bool march = g_xfer_march && !g_xfer_force_passes;
     bool tile = g_xfer_tile && p.K == 2 && !p.interpolate;
+    bool three = g_xfer_three;
     if (march && !tile) {
         std::lock_guard<std::mutex> lk(g_xc_mu);
         auto it = g_xchoice.find(xkey(p, dtype, nin, ea.in_wide));
         if (it != g_xchoice.end()) {
             march = it->second == 0;
             tile = it->second == 2;
+            three = it->second == 3;
         }
     }
     if (tile) {
@@ -1062,13 +1095,14 @@ int launch_transfer(const XferPlan& p, int dtype, const BC& bc,
         if (st != ENOTSUP_) return st;
         set_error("");
     }
-    return launch_other(p, dtype, bc, in, out, nin, scratch, ea, stream);
+    return launch_other(p, dtype, bc, in, out, nin, scratch, three, ea,
+                        stream);
 }
 
 // the one-point-per-thread K = 2 kernels, or the separable passes
 static int launch_other(const XferPlan& p, int dtype, const BC& bc,
                         const void* in, void* out, long nin, void* scratch,
-                        const XEpiArgs& ea, hipStream_t stream)
+                        bool three, const XEpiArgs& ea, hipStream_t stream)
 {
     if (dtype == 3 && p.K != 2) {
         set_error("transfer: complex64 data only for K = 2");
@@ -1095,11 +1129,14 @@ static int launch_other(const XferPlan& p, int dtype, const BC& bc,
                                                stream);
     }
     if (dtype == 0)
-        return run_transfer_k<double>(p, bc, in, out, nin, scratch, ea, stream);
+        return run_transfer_k<double>(p, bc, in, out, nin, scratch, three, ea,
+                                      stream);
     if (dtype == 1)
-        return run_transfer_k<double2>(p, bc, in, out, nin, scratch, ea, stream);
+        return run_transfer_k<double2>(p, bc, in, out, nin, scratch, three, ea,
+                                      stream);
     if (dtype == 2)
-        return run_transfer_k<float>(p, bc, in, out, nin, scratch, ea, stream);
+        return run_transfer_k<float>(p, bc, in, out, nin, scratch, three, ea,
+                                      stream);
     set_error("transfer: bad dtype %d", dtype);
     return EINVAL_;
 }

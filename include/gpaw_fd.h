@@ -501,10 +501,11 @@ int gfd_woperator_get_diagonal_element(gfd_woperator* op, double* out,
  * run Chebyshev iteration on D^-1 A (eigenvalue bounds from the radius-1
  * stencil's Fourier / sine modes) instead of Jacobi sweeps; the reference
  * schedule keeps Jacobi;
- * "xfer_passes" (0/1) runs K = 2 transfers as separable passes instead of
- * the fused kernel; "xfer_march" (0/1, default 1) lets transfers use the
- * x-marching fused kernel (off: one point per thread for K = 2, separable
- * passes for K > 2); "xfer_march_scale" (>= 1, default 1) sets its tiles
+ * "xfer_passes" (0/1/2) runs every transfer as separable passes instead of
+ * the fused kernels (1: z and y in one launch, 2: in one each, which are
+ * otherwise timed choices for K > 2); "xfer_march" (0/1, default 1) lets
+ * transfers use the x-marching fused kernel (off: one point per thread for
+ * K = 2, separable passes for K > 2); "xfer_march_scale" (>= 1, default 1) sets its tiles
  * per resident block to about 4 x value; "wx_march" (0/1, default 1) runs
  * weighted operators whose stencils are all axis-only (at most 4 of them)
  * through the weighted x-march kernel (off: one point per thread);
