@@ -135,11 +135,16 @@ static bool dm_search(const DirStencil& d, int dtype, const int n[3],
                                  ((t.tz + 2 * h.z) * es / 128.0 + 1.0) /
                                  (t.tz * t.ty * es / 128.0);
             const long tiles = (long)parts * nr * nin;
-            for (int chunks = 1; chunks <= std::max(1, n[0] / 4);
-                 chunks++) {
+            for (int chunks = 1; chunks <= n[0]; chunks++) {
                 t.xchunk = (n[0] + chunks - 1) / chunks;
-                const long per =
-                    (tiles * ((n[0] + t.xchunk - 1) / t.xchunk) + 255) / 256;
+                const long blocks =
+                    tiles * ((n[0] + t.xchunk - 1) / t.xchunk);
+                const long per = (blocks + 255) / 256;
+                // fewer than four planes: only where half the CUs are idle
+                // (one c128 grid of 23^3, R = 4: 11.6 -> 10.2 us)
+                if (4 * chunks > n[0] && chunks > 1 &&
+                    (blocks > 128 || h.x == 0))
+                    break;
                 const double resident =
                     std::min<long>(per, std::max(1, hold / waves)) * waves;
                 const double cost = (double)(t.xchunk + 2 * h.x) * per * waves *
