@@ -416,7 +416,8 @@ k_coarse(const CGrid* __restrict__ grids, const T* __restrict__ rhs,
 // (up to 10 x 20 x 20) 94 -> 30 us; FP32 24^3 .. 3^3 74 us against some 190
 // us as launches with k_coarse from 12^3 down.
 // Threads of a block, and the longest segment (FP32 first levels up to 24
-// planes; in FP64 24 would spill).  Segments beyond C1_X only on the first
+// planes; in FP64 the 128 registers of a 1024-thread block leave 76 bytes of
+// scratch per thread at 12 already, which the 26 us above include).  Segments beyond C1_X only on the first
 // level (a deeper one has at most a quarter of its columns) and not with
 // the Chebyshev iteration.
 constexpr int C1_NT = 1024, C1_X = 12, C1_XFIRST = 24;

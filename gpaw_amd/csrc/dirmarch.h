@@ -1,6 +1,5 @@
 // Stencils made of straight lines of points through the centre (axis
-// stencils, the Laplacians and gradients of skew cells, the Mehrstellen
-// pair), marching along x.
+// stencils, the Laplacians and gradients of skew cells), marching along x.
 #pragma once
 
 #include <mutex>
@@ -11,8 +10,9 @@ namespace gfd {
 
 constexpr int DM_NI = 3;  // in-plane directions: (0, 1), (1, 0) and one more
 constexpr int DM_NM = 4;  // directions (1, dy, dz) off the x axis
-// largest radius of the skew forms (the 9 accumulators of radius 4 and the
-// directions do not fit the registers)
+// largest radius the skew forms are built for.  (Radius 4 would fit: the
+// hexagonal Laplacian compiles to 103 registers in complex FP64 and no
+// scratch.  It is not built; those cells run on k_general.)
 constexpr int DM_RSKEW = 3;
 
 // What a stencil has on a line: no points, points at every step 1..R on both

@@ -101,15 +101,16 @@ void dirmarch_set_tile(const XmTile* t)
 // The weights fit measured sweeps (48 c128 grids of 128^3: 64 x 8 threads
 // 703 us, 128 x 4 with 4 staged elements 795, 32 x 8 802; 40 f64 grids of
 // 87x103x95: 48 x 10 in two chunks 174 us, whole x 184, 95 x 5 209; 24 c128
-// grids of 60x60x84, hexagonal: 28 x 9 in two chunks 55 us, whole x 58, in
-// four 64).
+// grids of 60x60x84, hexagonal, repeated on one input: 28 x 9 in two chunks
+// 55 us, whole x 58, in four 64).
 // pad: blocks of more threads than tile points, enough to stage the halo.
 static bool dm_search(const DirStencil& d, int dtype, const int n[3],
                       long nin, int epi, bool pad, DirTile& best)
 {
     const int R = d.R;
     const DirHalo h = dir_halo(R, dir_line(d, epi));
-    // waves a CU holds: complex FP64 takes about 128 registers at R = 3
+    // waves a CU holds: two blocks of 8 at the 86 registers of complex FP64
+    // at R = 3
     const int hold = dtype == 1 && R > 1 ? 16 : 32;
     double least = 1e300;
     for (int parts = 1; parts <= n[2]; parts++) {

@@ -18,13 +18,15 @@
 // All global traffic goes through per-plane buffer resources: zero
 // boundaries and idle lanes are out-of-range offsets, not branches.
 //
-// What bounds it: loads and stores for complex data (48 c128 grids of 128^3,
-// H psi - eps psi: 702 us, 4.6 TB/s; k_xrow 1006 us at 2 waves per SIMD);
-// for real data the instruction stream of one point per thread and plane
-// (40 f64 grids of 87x103x95: H psi 175 us, 3.1 TB/s; one point per thread
-// with every index wrapped took 790 us); for the skew stencils the LDS
-// reads (18 of 16 bytes per complex point of the 25-point hexagonal
-// Laplacian: 24 grids of 60x60x84 65 us; wrapped point by point 247 us).
+// What bounds it, by counters: HBM traffic, of which halo rows read again are
+// a third or more (48 c128 grids of 128^3, H psi - eps psi: 703 us, 2.4 GiB
+// fetched for 1.5, 5.9 TB/s in all; k_xrow 1006 us at 2 waves per SIMD; 40 f64
+// grids of 87x103x95, H psi: 174 us, 573 MiB fetched for 268, 5.1 TB/s; one
+// point per thread with every index wrapped took 790 us); for the skew
+// stencils the LDS reads (18 of 16 bytes beside the own point per complex
+// point of the 25-point hexagonal Laplacian, the LDS unit active 70 % of the
+// time and a third of that on bank conflicts: 24 grids of 60x60x84 64 us, 60
+// repeated on one input; wrapped point by point 247 us).
 #pragma once
 
 #include "dirmarch.h"

@@ -11,10 +11,12 @@
 // block order runs over the grids of the batch first: their blocks of one
 // tile read its four weights from the same XCD's L2.
 //
-// What bounds it: L2 and LDS traffic (32 bytes of weights beside 16 of data
-// per point; 12 LDS reads).  k_wxmarch, which takes the other operators,
-// tests every stencil's axes at every neighbour: 16 densities of 96^3 take
-// 202 us there, 112 us here (read and written once with the weights: 42).
+// What bounds it: latency and traffic together (32 bytes of weights beside 16
+// of data per point; by counters 279 MiB fetched for 135, 4.5 TB/s in all,
+// the LDS unit active 35 % of the time, waves waiting a third of it).
+// k_wxmarch, which takes the other operators, tests every stencil's axes at
+// every neighbour: 16 densities of 96^3 take 202 us there, 113 us here, 89
+// repeated on one input (read and written once with the weights: 42).
 #include "wstencil.h"
 
 #include "batch.h"

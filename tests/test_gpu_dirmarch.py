@@ -38,8 +38,19 @@ def grid(N, cell, pbc):
     return GridDescriptor(N, CELLS[cell] * 0.3 * np.array(N)[:, None], pbc)
 
 
+def both(*steps):
+    """Each offset and its opposite."""
+    return [(0, 0, 0)] + [o for s in steps
+                          for o in (s, tuple(-i for i in s))]
+
+
+def family(op, dtype=0, nin=1, epilogue=0):
+    """Kernel family of a pass (1 general, 2 march, 3 full rows, 4 point)."""
+    return _lib.load().gfd_operator_family(op._handle(), dtype, nin, epilogue)
+
+
 @pytest.mark.parametrize('cell', list(CELLS))
-@pytest.mark.parametrize('nn', [1, 2, 3])
+@pytest.mark.parametrize('nn', [1, 2, 3, 4])
 @pytest.mark.parametrize('N,pbc', [((8, 7, 9), True),
                                    ((13, 22, 71), (True, True, False)),
                                    ((24, 19, 130), False)])
@@ -52,22 +63,14 @@ def test_laplace(cell, nn, N, pbc, dtype):
     ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
     out = dev(np.zeros_like(a))
     say('dirmarch laplace', cell, nn, N, pbc, dtype)
+    # the march holds the directions of every cell, at radius 4 the axes only
+    takes = 2 if cell == 'box' or nn < 4 else 1
     with path(2):
+        assert family(op, int(dtype == complex), 3) == takes
         op.apply(dev(a), out, ph)
     ref = oracle.fd_apply(op.coef_p, op.offset_pc, gd.n_c, gd.neighbor_cd, a,
                           ph)
     assert relerr(host(out), ref) < TOL
-
-
-def both(*steps):
-    """Each offset and its opposite."""
-    return [(0, 0, 0)] + [o for s in steps
-                          for o in (s, tuple(-i for i in s))]
-
-
-def family(op, dtype=0, nin=1, epilogue=0):
-    """Kernel family of a pass (1 general, 2 march, 3 full rows, 4 point)."""
-    return _lib.load().gfd_operator_family(op._handle(), dtype, nin, epilogue)
 
 
 def edges(gd):
@@ -222,8 +225,10 @@ def test_epilogues(cell, N, pbc):
                                gd.neighbor_cd, f) - src
         assert relerr(host(r), want) < TOL
         assert abs(norm.value / (want**2).sum() - 1) < 1e-12
-        for dtype in (float, complex):
-            kin = Laplace(gd, -0.5, 3, dtype)
+        for dtype, nn in ((float, 3), (complex, 3),
+                          (complex, 4 if cell == 'box' else 2)):
+            kin = Laplace(gd, -0.5, nn, dtype)
+            assert family(kin, int(dtype == complex), 3, 4) == 2
             psi = rand(rng, (3,) + n, dtype)
             vt, eps = rng.uniform(-2, 0, n), rng.uniform(-1, 1, 3)
             ph = bloch_phases(rng, gd.pbc_c) if dtype == complex else None
