@@ -475,7 +475,7 @@ k_rmm_lambda(const T* __restrict__ dR, const T* __restrict__ R, long npts,
 // Band sums with a few bands: a band split over `chunks` blocks, whose
 // partial sums (two per block, in `work`) a second launch adds in a fixed
 // order.  One block per band leaves most CUs idle below a few hundred bands
-// (40 f64 bands of 87x103x95: lambda 440 us with one block each, now 149 us
+// (40 f64 bands of 87x103x95: lambda 440 us with one block each, now 145 us
 // split).  LAMBDA: both sums of the step length, else Re <a|b> only.
 constexpr int SPLIT_NT = 256;
 

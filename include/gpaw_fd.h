@@ -376,8 +376,9 @@ long gfd_gram_chunks(long ntiles, long npts);
 /* gfd_band_dots and gfd_rmm_lambda with nwork doubles of device memory as
  * work space (not shared by calls that overlap in time): from
  * 2 (2048 + nbands) on, a band's sum is split over several blocks when
- * there are too few bands to fill the GPU.  The order of the sum is fixed
- * by nbands, npts and nwork. */
+ * there are too few bands to fill the GPU and each has enough points.  The
+ * order of the sum is fixed by the data type,
+ * nbands, npts and nwork. */
 int gfd_band_dots_work(int is_complex, const void* a, const void* b,
                        int nbands, long npts, long ld, double dv, double* out,
                        double* work, long nwork, void* stream);
