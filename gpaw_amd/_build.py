@@ -17,13 +17,14 @@ HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 ARCH = 'gfx950'
 
 # longest compiles first (the pool runs them in this order)
-SOURCES = ['dirmarch_c128.hip', 'dirmarch_f64.hip', 'dirmarch_c64.hip',
-           'dirmarch_f32.hip', 'dirmarch.hip', 'rows_dma.hip', 'rows_dma32.hip', 'rows_f64.hip', 'rows_c128.hip', 'rows_f32.hip', 'rows_c64.hip',
-           'stencil.hip', 'batch.hip', 'transfer.hip', 'api.hip',
-           'stencil_rows.hip', 'point.hip', 'vector.hip', 'bands.hip', 'coarse.hip', 'tsmooth.hip',
-           'fftpoisson.hip', 'wstencil.hip', 'gs.hip',
-           'xfer_march.hip', 'wxmarch.hip', 'wdielectric.hip', 'bxmarch.hip', 'bxfer_march.hip',
-           'precond_fine.hip']
+SOURCES = ['rows_c128.hip', 'dirmarch_c128.hip', 'dirmarch_c64.hip',
+           'dirmarch_f64.hip', 'rows_c64.hip', 'dirmarch_f32.hip',
+           'rows_f32.hip', 'transfer.hip', 'rows_f64.hip', 'wxmarch.hip',
+           'xfer_march.hip', 'precond_fine.hip', 'bxmarch.hip', 'batch.hip',
+           'rows_dma.hip', 'rows_dma32.hip', 'coarse.hip', 'bxfer_march.hip',
+           'tsmooth.hip', 'wdielectric.hip', 'stencil.hip', 'point.hip',
+           'api.hip', 'bands.hip', 'dirmarch.hip', 'stencil_rows.hip',
+           'vector.hip', 'fftpoisson.hip', 'wstencil.hip', 'gs.hip']
 
 FLAGS = [
     '-std=c++20', '-O3', '-fPIC', f'--offload-arch={ARCH}',

@@ -250,7 +250,7 @@ static bool aligned16(const void* p)
 static bool march_first(const gfd_operator* op, int epi)
 {
     const DirStencil& d = op->dir;
-    const int line = dir_line(d, epi);
+    const int line = dir_line(d, 1, epi);
     if (d.full && epi == EPI_POT) return true;
     return d.R >= 3 && (d.full || line > 0 ||
                         (line == 0 && op->n[2] % 2 != 0));

@@ -61,16 +61,17 @@ struct DirHalo {
     int x, y, z;
 };
 
-// A plain pass of a stencil on one axis reads along that axis only (the
-// other epilogues run it in the general form).
+// A plain FP64 pass of a stencil on one axis reads along that axis only (the
+// other epilogues, and FP32 data, which has no gradients, run the general
+// form).
 constexpr DirHalo dir_halo(int R, int line)
 {
     return {line < 1 ? R : 0, line < 0 || line == 1 ? R : 0,
             line < 0 || line == 2 ? R : 0};
 }
-inline int dir_line(const DirStencil& d, int epi)
+inline int dir_line(const DirStencil& d, int dtype, int epi)
 {
-    return epi == EPI_PLAIN ? d.line : -1;
+    return epi == EPI_PLAIN && dtype < 2 ? d.line : -1;
 }
 
 // The tile with the least estimated time; every grid of sides >= R has one.

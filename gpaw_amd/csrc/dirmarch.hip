@@ -108,7 +108,7 @@ static bool dm_search(const DirStencil& d, int dtype, const int n[3],
                       long nin, int epi, bool pad, DirTile& best)
 {
     const int R = d.R;
-    const DirHalo h = dir_halo(R, dir_line(d, epi));
+    const DirHalo h = dir_halo(R, dir_line(d, dtype, epi));
     // waves a CU holds: two blocks of 8 at the 86 registers of complex FP64
     // at R = 3
     const int hold = dtype == 1 && R > 1 ? 16 : 32;
@@ -180,7 +180,7 @@ DirTile dir_tile(const DirStencil& d, int dtype, const int n[3], long nin,
 DirTile DirTiles::get(const DirStencil& d, int dtype, const int n[3],
                       long nin, int epi)
 {
-    const int line = dir_line(d, epi);
+    const int line = dir_line(d, dtype, epi);
     std::lock_guard<std::mutex> lk(mu);
     for (int i = 0; i < used; i++)
         if (e[i].nin == nin && e[i].dtype == dtype && e[i].line == line)

@@ -443,10 +443,13 @@ static int dm_launch_r(const DirStencil& d, const DirTile& t, const int n[3],
 #define GFD_DM(NI, NM, FORM)                                                \
     return dm_launch_e<T, R, NI, NM, FORM>(d, t, n, bc, in, out, nin, epi,  \
                                            ea, s, nbo)
-    switch (dir_line(d, epi)) {
-    case 0: GFD_DM(2, 0, DM_LINE);
-    case 1: GFD_DM(2, 0, DM_LINE + 1);
-    case 2: GFD_DM(2, 0, DM_LINE + 2);
+    constexpr bool WIDE = sizeof(typename ScalarOf<T>::type) == 8;
+    if constexpr (WIDE) {
+        switch (dir_line(d, IsCplx<T>::value, epi)) {
+        case 0: GFD_DM(2, 0, DM_LINE);
+        case 1: GFD_DM(2, 0, DM_LINE + 1);
+        case 2: GFD_DM(2, 0, DM_LINE + 2);
+        }
     }
     if (d.full) {
         if (d.ni == 2 && d.nm == 0) GFD_DM(2, 0, DM_FULL);
@@ -457,8 +460,8 @@ static int dm_launch_r(const DirStencil& d, const DirTile& t, const int n[3],
         }
     }
     // anything else: the general form of the directions, of the axes for
-    // plain passes that need no more
-    if constexpr (R <= DM_RSKEW)
+    // plain FP64 passes that need no more
+    if constexpr (WIDE && R <= DM_RSKEW)
         if (d.ni == 2 && d.nm == 0 && epi == EPI_PLAIN)
             return dm_launch_h<T, R, 2, 0, DM_NONE, DM_GENERAL, false>(
                 d, t, n, bc, in, out, nin, epi, ea, s, nbo);
