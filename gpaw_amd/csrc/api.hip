@@ -681,19 +681,19 @@ extern "C" void gfd_transformer_free(gfd_transformer* t)
 }
 
 static size_t xfer_scratch_bytes(const gfd_transformer* t, int dtype,
-                                 long nin)
+                                 long nin, bool three = true)
 {
     const size_t es = dtype == 1 ? 16 : (dtype == 2 ? 4 : 8);  // 3: c64
     return t->plan.K == 2 && !xfer_passes_forced()
                ? 0
-               : es * xfer_scratch_elems(t->plan, nin) + 16;
+               : es * xfer_scratch_elems(t->plan, nin, three) + 16;
 }
 
 // Time the transfer kernel families for this shape once (not under graph
 // capture), into the transformer's output-sized tuning buffer.
 static int xfer_maybe_tune(gfd_transformer* t, int dtype, const BC& bc,
-                           const void* in, long nin, void* work, int in_wide,
-                           hipStream_t s)
+                           const void* in, long nin, void* work, bool room,
+                           int in_wide, hipStream_t s)
 {
     if (!xfer_needs_tuning(t->plan, dtype, nin, in_wide)) return OK;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -704,7 +704,7 @@ static int xfer_maybe_tune(gfd_transformer* t, int dtype, const BC& bc,
     if (cs != hipStreamCaptureStatusNone) return OK;
     const size_t es = dtype == 1 ? 16 : (dtype == 2 ? 4 : 8);
     GFD_TRY(t->tune_out.ensure(es * t->ngout() * nin, s));
-    return xfer_tune(t->plan, dtype, bc, in, t->tune_out.p, nin, work,
+    return xfer_tune(t->plan, dtype, bc, in, t->tune_out.p, nin, work, room,
                      in_wide, s);
 }
 
@@ -714,13 +714,19 @@ static int xfer_dt(gfd_transformer* t, int dtype, const void* in, void* out,
                    long nin, const double* phases, const XEpiArgs& ea,
                    hipStream_t s, void* work = nullptr)
 {
+    // own work space: no larger than the kernel chosen for the shape needs
+    bool room = true;
     if (!work && (t->plan.K != 2 || xfer_passes_forced())) {
-        GFD_TRY(t->scratch.ensure(xfer_scratch_bytes(t, dtype, nin), s));
+        room = xfer_wants_three(t->plan, dtype, nin, ea.in_wide);
+        GFD_TRY(t->scratch.ensure(xfer_scratch_bytes(t, dtype, nin, room),
+                                  s));
         work = t->scratch.p;
     }
     const BC bc = make_bc(t->periodic, t->real ? nullptr : phases);
-    GFD_TRY(xfer_maybe_tune(t, dtype, bc, in, nin, work, ea.in_wide, s));
-    return launch_transfer(t->plan, dtype, bc, in, out, nin, work, ea, s);
+    GFD_TRY(xfer_maybe_tune(t, dtype, bc, in, nin, work, room, ea.in_wide,
+                            s));
+    return launch_transfer(t->plan, dtype, bc, in, out, nin, work, room, ea,
+                           s);
 }
 
 static int xfer(gfd_transformer* t, const void* in, void* out, long nin,
@@ -1453,10 +1459,10 @@ static int pretune_levels(gfd_poisson* p, Levels& lv, hipStream_t s)
             // the transfer kernel choices of this level pair
             const BC br = make_bc(p->rst[l]->periodic, nullptr);
             GFD_TRY(xfer_maybe_tune(p->rst[l], lv.dtype, br, lv.res[l], 1,
-                                    p->xscratch.p, 0, s));
+                                    p->xscratch.p, true, 0, s));
             const BC bi = make_bc(p->itp[l]->periodic, nullptr);
             GFD_TRY(xfer_maybe_tune(p->itp[l], lv.dtype, bi, lv.phi[l + 1],
-                                    1, p->xscratch.p, 0, s));
+                                    1, p->xscratch.p, true, 0, s));
         }
     }
     return OK;

@@ -65,8 +65,8 @@ bool xfer_needs_tuning(const XferPlan& p, int dtype, long nin, int in_wide);
 // Time the kernel families with PLAIN passes of `in` into tune_out
 // (output-sized scratch) and record the faster.  Not under graph capture.
 int xfer_tune(const XferPlan& p, int dtype, const BC& bc, const void* in,
-              void* tune_out, long nin, void* scratch, int in_wide,
-              hipStream_t s);
+              void* tune_out, long nin, void* scratch, bool room,
+              int in_wide, hipStream_t s);
 
 // The x-marching fused transfer (xfer_march.hip); ENOTSUP_ for a shape
 // its tiles cannot take.
@@ -74,12 +74,16 @@ int launch_transfer_march(const XferPlan& p, int dtype, const BC& bc,
                           const void* in, void* out, long nin,
                           const XEpiArgs& ea, hipStream_t stream);
 
-// Scratch (in elements of the data type) needed for `nin` grids.
-long xfer_scratch_elems(const XferPlan& p, long nin);
+// Scratch (in elements of the data type) needed for `nin` grids; three: also
+// by the z and y passes in a launch each.
+long xfer_scratch_elems(const XferPlan& p, long nin, bool three);
+// Whether those passes may run for this shape (chosen, or not yet timed).
+bool xfer_wants_three(const XferPlan& p, int dtype, long nin, int in_wide);
 
-// dtype: 0 f64, 1 c128, 2 f32, 3 c64 (c64: K = 2 only)
+// dtype: 0 f64, 1 c128, 2 f32, 3 c64 (c64: K = 2 only).  room: the scratch has
+// room for the z and y passes in a launch each.
 int launch_transfer(const XferPlan& p, int dtype, const BC& bc,
                     const void* in, void* out, long nin, void* scratch,
-                    const XEpiArgs& ea, hipStream_t stream);
+                    bool room, const XEpiArgs& ea, hipStream_t stream);
 
 }  // namespace gfd

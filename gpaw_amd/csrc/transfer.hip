@@ -606,10 +606,11 @@ static int launch_fused2(const XferPlan& p, const BC& bc, const void* in,
     return EINVAL_;
 }
 
-long xfer_scratch_elems(const XferPlan& p, long nin)
+long xfer_scratch_elems(const XferPlan& p, long nin, bool three)
 {
-    // outputs of the z pass and of the y pass
-    return (long)p.nin[0] * (p.nin[1] + p.nout[1]) * p.nout[2] * nin;
+    // output of the y pass, and of a z pass of its own
+    return (long)p.nin[0] * (p.nout[1] + (three ? p.nin[1] : 0)) *
+           p.nout[2] * nin;
 }
 
 // z and y passes of a separable transfer in one launch: a block stages the
@@ -874,8 +875,8 @@ static int launch_pass_epi(XArgs<T> a, int epi, hipStream_t s)
     return EINVAL_;
 }
 
-// three: z and y in a launch each, z's result in front of y's in the work
-// space; else both in one (k_xfer_zy).
+// three: z and y in a launch each, z's result behind y's in the work space;
+// else both in one (k_xfer_zy).
 template <typename T, int K, bool INTERP>
 static int run_transfer(const XferPlan& p, const BC& bc, const void* in,
                         void* out, long nin, void* scratch, bool three,
@@ -905,8 +906,8 @@ static int run_transfer(const XferPlan& p, const BC& bc, const void* in,
         a.alpha = ea.alpha;
         return a;
     };
-    T* const z = (T*)scratch;
-    T* const zy = z + (long)p.nin[0] * p.nin[1] * p.nout[2] * nin;
+    T* const zy = (T*)scratch;
+    T* const z = zy + (long)p.nin[0] * p.nout[1] * p.nout[2] * nin;
     if (three) {
         GFD_TRY((launch_pass<T, 2, K, INTERP, XEPI_PLAIN>(
             pass(2, (const T*)in, z), s)));
@@ -1009,9 +1010,18 @@ bool xfer_needs_tuning(const XferPlan& p, int dtype, long nin, int in_wide)
            g_xchoice.find(xkey(p, dtype, nin, in_wide)) == g_xchoice.end();
 }
 
+bool xfer_wants_three(const XferPlan& p, int dtype, long nin, int in_wide)
+{
+    if (g_xfer_three) return true;
+    if (p.K == 2) return false;
+    std::lock_guard<std::mutex> lk(g_xc_mu);
+    auto it = g_xchoice.find(xkey(p, dtype, nin, in_wide));
+    return it == g_xchoice.end() ? g_xtune : it->second == 3;
+}
+
 int xfer_tune(const XferPlan& p, int dtype, const BC& bc, const void* in,
-              void* tune_out, long nin, void* scratch, int in_wide,
-              hipStream_t s)
+              void* tune_out, long nin, void* scratch, bool room,
+              int in_wide, hipStream_t s)
 {
     XEpiArgs ea;
     ea.in_wide = in_wide;
@@ -1026,7 +1036,7 @@ int xfer_tune(const XferPlan& p, int dtype, const BC& bc, const void* in,
     int choice = 0;
     for (int c = 0; c < 4; c++) {
         if (c == 2 && (p.K != 2 || p.interpolate)) continue;
-        if (c == 3 && p.K == 2) continue;
+        if (c == 3 && (p.K == 2 || !room)) continue;
         auto run = [&]() {
             return c == 0 ? launch_transfer_march(p, dtype, bc, in, tune_out,
                                                   nin, ea, s)
@@ -1064,7 +1074,7 @@ int xfer_tune(const XferPlan& p, int dtype, const BC& bc, const void* in,
 
 int launch_transfer(const XferPlan& p, int dtype, const BC& bc,
                     const void* in, void* out, long nin, void* scratch,
-                    const XEpiArgs& ea, hipStream_t stream)
+                    bool room, const XEpiArgs& ea, hipStream_t stream)
 {
     if (ea.in_wide && (p.K != 2 || (dtype != 2 && dtype != 3))) {
         set_error("transfer: FP64 input only for FP32 data and K = 2");
@@ -1095,8 +1105,8 @@ int launch_transfer(const XferPlan& p, int dtype, const BC& bc,
         if (st != ENOTSUP_) return st;
         set_error("");
     }
-    return launch_other(p, dtype, bc, in, out, nin, scratch, three, ea,
-                        stream);
+    return launch_other(p, dtype, bc, in, out, nin, scratch, three && room,
+                        ea, stream);
 }
 
 // the one-point-per-thread K = 2 kernels, or the separable passes
