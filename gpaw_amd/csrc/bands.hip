@@ -537,8 +537,8 @@ k_band_join(const double* __restrict__ work, int chunks, double dv,
 //         (150); from 220 bands on 1.05 to 1.27 at any length
 //   c128  twice the bytes: 17k 0.96 .. 0.98 (20), 20k 1.18 (40), 44k 0.51 ..
 //         0.94 (64), 72k 1.12 (100), 96k 0.26 .. 0.76 (100) and 0.92 (116); 150
-//         to 220 bands 1.00 to 1.19, 300 (two blocks on some CUs) 0.76 to
-//         0.95, beyond 0.92 to 1.09
+//         to 220 bands 1.00 to 1.19; two blocks on some CUs only: 260 0.68, 300
+//         0.76, 400 0.89, 512 1.00 to 1.02, 1024 1.05
 static int band_chunks(int nbands, long npts, bool cplx, long nwork)
 {
     const int w = cplx ? 2 * nbands : nbands;
@@ -547,12 +547,12 @@ static int band_chunks(int nbands, long npts, bool cplx, long nwork)
                        : cplx     ? 96000
                                   : 130000;
     const bool gains = cplx && nbands > 256
-                           ? npts >= 40000
+                           ? nbands < 512 && npts >= 40000
                            : nbands <= (cplx ? 120 : 150) && npts >= least;
     if (!gains) return 1;
     long c = std::min((2048L + nbands - 1) / nbands, npts / 4096);
     c = std::min(c, nwork / (2L * nbands));
-    return nbands > 65535 || c < 2 ? 1 : (int)c;
+    return c < 2 ? 1 : (int)c;
 }
 
 template <typename T, bool LAMBDA>
